@@ -20,6 +20,7 @@
 //      unresolved node, so the loop ends);
 //   5. compact the level, remap the parent level's child pointers.
 // Finally the whole DAG is re-deduplicated exactly (:1176).
+#include <algorithm>
 #include "svd_internal.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -111,44 +112,137 @@ __device__ __forceinline__ uint32_t hamming512(const uint4* a, const uint32_t s[
   return h;
 }
 
-// Exhaustive pre-filter lists: block = 256 consecutive j; the earlier nodes are
-// streamed through LDS in tiles of 256 signatures (16 KB) that every lane
-// reads in the same order (LDS broadcast).  Stops once every lane holds cap.
-__global__ void __launch_bounds__(256) k_exhaustive_lists(const uint32_t* __restrict__ sig, uint64_t n,
-                                                          const uint64_t* __restrict__ refs, uint64_t maxRefs,
-                                                          uint32_t bound, uint32_t cap, uint32_t* __restrict__ lists,
-                                                          uint32_t* __restrict__ counts) {
-  __shared__ uint4 tile[256 * 4];
-  const uint64_t j0 = (uint64_t)blockIdx.x * 256;
-  const uint64_t j = j0 + threadIdx.x;
-  const bool active = j < n && refs[j] <= maxRefs;
-  uint32_t s[16];
-  if (j < n) {
-    const uint4* p = reinterpret_cast<const uint4*>(sig + j * 16);
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// One signature word as 32 fp4 (e2m1) values of a matrix operand: bit 4p + d
+// becomes nibble p of dword d, 0 -> +1.0 (0x2), 1 -> -1.0 (0xA).  The order of
+// the 512 positions along K is free as long as both operands share it.
+__device__ __forceinline__ i32x4_t bits_to_fp4(uint32_t w) {
+  constexpr uint32_t kOne = 0x22222222u, kSign = 0x88888888u;
+  i32x4_t r;
+  r[0] = (int)(((w << 3) & kSign) | kOne);
+  r[1] = (int)(((w << 2) & kSign) | kOne);
+  r[2] = (int)(((w << 1) & kSign) | kOne);
+  r[3] = (int)((w & kSign) | kOne);
+  return r;
+}
+
+// Exhaustive pre-filter lists on the matrix cores.  With bits as +-1 the dot
+// product of two signatures is 512 - 2 Hamming, so popcount(a ^ b) <= bound is
+// one comparison of an fp32 sum of +-1 (exact) with 512 - 2 bound, and the
+// all-pairs scan is a GEMM of fp4 operands (v_mfma_f32_32x32x64_f8f6f4: 8 of
+// them per 32 x 32 pairs) that never leaves the registers.  A workgroup holds
+// 128 JT consecutive j, a wavefront 32 JT of them expanded as its B operand;
+// the earlier nodes i stream through LDS in stages of 256 signatures, still as
+// bits (rows padded to 80 bytes: the 16-byte reads of eight lanes fall in
+// distinct banks), and are expanded as they are read (8 VALU operations per 32
+// positions).  Accumulator element v of lane l is pair
+// (i = 8 (v/4) + 4 (l/32) + v%4, j = l%32) of a tile; the matches of a tile
+// are appended in index order, and a wavefront stops once all its j hold cap.
+// Later j have more to scan, so the last workgroups start first.
+template <int JT>
+__global__ void __launch_bounds__(256, 2) k_exhaustive_lists(const uint32_t* __restrict__ sig, uint64_t n,
+                                                             const uint64_t* __restrict__ refs, uint64_t maxRefs,
+                                                             uint32_t bound, uint32_t cap,
+                                                             uint32_t* __restrict__ lists,
+                                                             uint32_t* __restrict__ counts) {
+  constexpr int kStage = 256, kRow = 20;         // signatures per stage, dwords per LDS row
+  __shared__ __attribute__((aligned(16))) uint32_t tile[2][kStage * kRow];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+  const uint32_t j0 = (gridDim.x - 1 - blockIdx.x) * (128 * JT);     // node ids are 32-bit
+  const uint32_t jw = j0 + wave * (32 * JT);               // the wavefront's first j
+  const float limit = bound >= 512u ? -513.f : 512.f - 2.f * (float)bound;
+  i32x4_t b[JT][8];
+  float thr[JT];                                 // +inf: inactive or full
+  uint32_t cnt[JT];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) { const uint4 t = p[q]; s[4 * q] = t.x; s[4 * q + 1] = t.y; s[4 * q + 2] = t.z; s[4 * q + 3] = t.w; }
-  }
-  uint32_t cnt = 0;
-  const uint64_t jend = j0 + 256 < n ? j0 + 256 : n;
-  for (uint64_t i0 = 0; i0 < jend; i0 += 256) {
-    if (!__syncthreads_or(active && cnt < cap)) break;
-    for (int q = threadIdx.x; q < 256 * 4; q += 256) {
-      const uint64_t i = i0 + (q >> 2);
-      tile[q] = i < n ? reinterpret_cast<const uint4*>(sig + i * 16)[q & 3] : make_uint4(0, 0, 0, 0);
+  for (int t = 0; t < JT; ++t) {
+    const uint32_t j = jw + 32 * t + col;
+    uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+    if (j < n) {
+      const uint4* p = reinterpret_cast<const uint4*>(sig + (uint64_t)j * 16 + 8 * half);
+      lo = p[0];
+      hi = p[1];
     }
-    __syncthreads();
-    if (active && cnt < cap) {
-      const uint64_t iend = i0 + 256 < j ? i0 + 256 : j;
-      for (uint64_t i = i0; i < iend; ++i) {
-        if (hamming512(&tile[(i - i0) * 4], s) <= bound) {
-          lists[j * cap + cnt] = (uint32_t)i;
-          if (++cnt == cap) break;
-        }
+    const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) b[t][k] = bits_to_fp4(w[k]);
+    thr[t] = j < n && refs[j] <= maxRefs ? limit : __builtin_inff();
+    cnt[t] = 0;
+  }
+  auto open = [&]() {
+    bool o = false;
+#pragma unroll
+    for (int t = 0; t < JT; ++t) o |= thr[t] < __builtin_inff();
+    return __any(o) != 0;
+  };
+  bool live = open();
+  const uint32_t iEnd = (uint32_t)(j0 + 128 * JT < n ? j0 + 128 * JT : n);
+  uint4 r[4];
+  auto load = [&](uint32_t i0) {
+    const uint32_t i = i0 + tid;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      r[q] = i < n ? reinterpret_cast<const uint4*>(sig + (uint64_t)i * 16)[q] : make_uint4(0, 0, 0, 0);
+  };
+  load(0);
+  int buf = 0;
+  for (uint32_t i0 = 0; i0 < iEnd; i0 += kStage, buf ^= 1) {
+    uint4* d = reinterpret_cast<uint4*>(&tile[buf][tid * kRow]);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[q] = r[q];
+    if (!__syncthreads_or(live)) break;          // two buffers: one barrier per stage
+    if (i0 + kStage < iEnd) load(i0 + kStage);
+    for (int it = 0; it < kStage / 32; ++it) {
+      const uint32_t base = i0 + 32 * it;
+      if (!live || base >= jw + 32 * JT) break;  // every i of the tile is past the wavefront's j
+      const uint4* a4 = reinterpret_cast<const uint4*>(&tile[buf][(32 * it + col) * kRow + 8 * half]);
+      const uint4 lo = a4[0], hi = a4[1];
+      const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+      f32x16_t acc[JT];
+#pragma unroll
+      for (int t = 0; t < JT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const i32x4_t a = bits_to_fp4(w[k]);
+#pragma unroll
+        for (int t = 0; t < JT; ++t)
+          acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+              __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1),
+              __builtin_shufflevector(b[t][k], b[t][k], 0, 1, 2, 3, -1, -1, -1, -1), acc[t], 4, 4, 0, 0, 0, 0);
       }
+#pragma unroll
+      for (int t = 0; t < JT; ++t) {
+        float m = acc[t][0];
+#pragma unroll
+        for (int v = 1; v < 16; ++v) m = fmaxf(m, acc[t][v]);
+        if (!__any(m >= thr[t])) continue;
+        uint32_t hits = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          hits |= (acc[t][v] >= thr[t] ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+        hits <<= 4 * half;
+        hits |= __shfl_xor(hits, 32, 64);
+        const uint32_t j = jw + 32 * t + col;
+        if (j < base + 32) hits = j > base ? hits & ((1u << (j - base)) - 1u) : 0u;
+        while (hits && cnt[t] < cap) {
+          if (half == 0) lists[(uint64_t)j * cap + cnt[t]] = base + (uint32_t)(__ffs(hits) - 1);
+          hits &= hits - 1;
+          ++cnt[t];
+        }
+        if (cnt[t] == cap) thr[t] = __builtin_inff();
+      }
+      live = open();
     }
-    __syncthreads();
   }
-  if (j < n) counts[j] = active ? cnt : 0u;
+#pragma unroll
+  for (int t = 0; t < JT; ++t) {
+    const uint32_t j = jw + 32 * t + col;
+    if (half == 0 && j < n) counts[j] = cnt[t];
+  }
 }
 
 // Ranked pre-filter lists: every earlier node i < j within the bound, the K
@@ -411,6 +505,18 @@ __global__ void k_remap_inplace(uint32_t* __restrict__ rec, uint64_t n, const ui
     if ((m >> c) & 1u) r[1 + c] = corr[r[1 + c]];
 }
 
+void exhaustive_lists(svd_ctx* c, const uint32_t* sig, uint64_t n, const uint64_t* refs, uint64_t maxRefs,
+                      uint32_t bound, uint32_t cap, uint32_t* lists, uint32_t* counts) {
+  // the widest tile that still gives every CU a workgroup
+  const uint64_t cus = (uint64_t)std::max(c->numCU, 1);
+  if (n >= 512 * cus)
+    k_exhaustive_lists<4><<<div_up(n, 512), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
+  else if (n >= 256 * cus)
+    k_exhaustive_lists<2><<<div_up(n, 256), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
+  else
+    k_exhaustive_lists<1><<<div_up(n, 128), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
+}
+
 LevelView make_view(const svd_octree* o, const std::vector<uint64_t*>& vox) {
   LevelView v = {};
   v.L = o->levels;
@@ -534,9 +640,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
     clk.mark(1);
     if (!learned) {
       clk.mark(2);
-      if (n && !ranked)
-        k_exhaustive_lists<<<div_up(n, 256), 256, 0, c->stream>>>(sig, n, refs[lev], maxRefs, bound, cap, lists,
-                                                                  counts);
+      if (n && !ranked) exhaustive_lists(c, sig, n, refs[lev], maxRefs, bound, cap, lists, counts);
       else if (n && cap <= 16)
         k_ranked_lists<16><<<div_up(n, 256), 256, 0, c->stream>>>(sig, n, refs[lev], maxRefs, bound, cap, lists,
                                                                    counts);
