@@ -128,121 +128,261 @@ __device__ __forceinline__ i32x4_t bits_to_fp4(uint32_t w) {
   return r;
 }
 
+// Order of the exhaustive scan: chunks of C consecutive nodes, by popcount
+// within a chunk (stable).  Key = chunk * 513 + popcount.
+constexpr uint32_t kPopBins = 513;
+__global__ void k_list_keys(const uint32_t* __restrict__ sig, uint64_t n, uint32_t C, uint32_t* __restrict__ keys,
+                            uint32_t* __restrict__ ids) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const uint4* p = reinterpret_cast<const uint4*>(sig + i * 16);
+  uint32_t pc = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) { const uint4 t = p[q]; pc += __popc(t.x) + __popc(t.y) + __popc(t.z) + __popc(t.w); }
+  keys[i] = (uint32_t)i / C * kPopBins + pc;
+  ids[i] = (uint32_t)i;
+}
+
+// Signatures in scan order (four lanes each), and off[key] = the first
+// position whose key is at least key (nKeys + 1 entries).
+__global__ void k_list_gather(const uint32_t* __restrict__ sig, const uint32_t* __restrict__ ids,
+                              const uint32_t* __restrict__ keys, uint64_t n, uint32_t nKeys,
+                              uint4* __restrict__ ssig, uint32_t* __restrict__ off) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const uint64_t p = e >> 2;
+  if (p >= n) return;
+  ssig[e] = reinterpret_cast<const uint4*>(sig + (uint64_t)ids[p] * 16)[e & 3];
+  if (e & 3) return;
+  const uint32_t key = keys[p];
+  for (uint32_t k = p ? keys[p - 1] + 1 : 0; k <= key; ++k) off[k] = (uint32_t)p;
+  if (p == n - 1)
+    for (uint32_t k = key + 1; k <= nKeys; ++k) off[k] = (uint32_t)n;
+}
+
+// The entries of one j's list, cap in lists and cap more in spill, in no
+// order, two per lane of a wavefront (at most 2 cap <= 128 of them).
+__device__ __forceinline__ void load_list(const uint32_t* lists, const uint32_t* spill, uint64_t at, uint32_t cnt,
+                                          uint32_t cap, int lane, uint32_t v[2]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t e = (uint32_t)lane + 64 * h;
+    const uint32_t* p = e < cap ? lists + at + e : spill + at + (e - cap);
+    v[h] = e < cnt ? __atomic_load_n(p, __ATOMIC_RELAXED) : kNone;
+  }
+}
+// Their smallest cap go to lists, ascending.  Returns the largest one kept.
+__device__ __forceinline__ uint32_t order_list(uint32_t* lists, uint64_t at, uint32_t cnt, uint32_t cap,
+                                               const uint32_t v[2]) {
+  uint32_t rank[2] = {0, 0};
+  const int m = (int)(cnt < 64u ? cnt : 64u);
+  for (int r = 0; r < m; ++r) {
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v[0], r);
+    rank[0] += a < v[0] ? 1u : 0u;
+    rank[1] += a < v[1] ? 1u : 0u;
+  }
+  for (int r = 64; r < (int)cnt; ++r) {
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v[1], r - 64);
+    rank[0] += a < v[0] ? 1u : 0u;
+    rank[1] += a < v[1] ? 1u : 0u;
+  }
+  const uint32_t keep = cnt < cap ? cnt : cap;
+  uint32_t last = 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    if (v[h] != kNone && rank[h] < keep) {
+      lists[at + rank[h]] = v[h];
+      if (rank[h] == keep - 1) last = v[h];
+    }
+  const unsigned long long w = __ballot(last != 0);   // one lane at most: node 0 alone gives 0
+  return w ? (uint32_t)__builtin_amdgcn_readlane((int)last, __ffsll(w) - 1) : 0u;
+}
+
 // Exhaustive pre-filter lists on the matrix cores.  With bits as +-1 the dot
 // product of two signatures is 512 - 2 Hamming, so popcount(a ^ b) <= bound is
 // one comparison of an fp32 sum of +-1 (exact) with 512 - 2 bound, and the
-// all-pairs scan is a GEMM of fp4 operands (v_mfma_f32_32x32x64_f8f6f4: 8 of
-// them per 32 x 32 pairs) that never leaves the registers.  A workgroup holds
-// 128 JT consecutive j, a wavefront 32 JT of them expanded as its B operand;
-// the earlier nodes i stream through LDS in stages of 256 signatures, still as
-// bits (rows padded to 80 bytes: the 16-byte reads of eight lanes fall in
-// distinct banks), and are expanded as they are read (8 VALU operations per 32
-// positions).  Accumulator element v of lane l is pair
-// (i = 8 (v/4) + 4 (l/32) + v%4, j = l%32) of a tile; the matches of a tile
-// are appended in index order, and a wavefront stops once all its j hold cap.
-// Later j have more to scan, so the last workgroups start first.
+// scan is a GEMM of fp4 operands (v_mfma_f32_32x32x64_f8f6f4: 8 of them per
+// 32 x 32 pairs) that never leaves the registers.
+//  - |popcount(a) - popcount(b)| <= Hamming: chunk by chunk in node order, a
+//    workgroup's j (32 JT per wavefront, expanded as its B operand) meet only
+//    the nodes whose popcount is within the bound of theirs.  Chunks keep the
+//    scan to earlier nodes and let a j stop once the chunks behind it hold
+//    cap matches (16 of them, or fewer of at least 512 nodes: on 10K nodes
+//    0.30 ms against 0.46 ms for one chunk, on 466K nodes 4 to 64 chunks
+//    measure the same).
+//  - i streams through LDS in stages of 256 signatures, still as bits (rows
+//    padded to 80 bytes: the 16-byte reads of eight lanes fall in distinct
+//    banks), expanded as they are read (8 VALU operations per 32 positions).
+//  - Accumulator element v of lane l is pair (i = 8 (v/4) + 4 (l/32) + v%4,
+//    j = l%32) of a tile.  Matches are appended unordered, 2 cap of them at
+//    most before the smallest cap are kept; k_list_order sorts at the end.
+//  - Later j have more to scan, so the last workgroups start first.
+// Bound by the matrix cores: on 466K nodes of the 2048^3 caves (bound 10, 36%
+// of the pairs inside the popcount window) 9.0 ms at 66% of the MFMA cycles,
+// against 19.3 ms without the window and 172 ms for an XOR/popcount scan.
 template <int JT>
-__global__ void __launch_bounds__(256, 2) k_exhaustive_lists(const uint32_t* __restrict__ sig, uint64_t n,
-                                                             const uint64_t* __restrict__ refs, uint64_t maxRefs,
-                                                             uint32_t bound, uint32_t cap,
-                                                             uint32_t* __restrict__ lists,
-                                                             uint32_t* __restrict__ counts) {
+__global__ void __launch_bounds__(256, 3)
+k_exhaustive_lists(const uint4* __restrict__ ssig, const uint32_t* __restrict__ ids, const uint32_t* __restrict__ keys,
+                   const uint32_t* __restrict__ off, uint32_t n, uint32_t C, const uint64_t* __restrict__ refs,
+                   uint64_t maxRefs, uint32_t bound, uint32_t cap, uint32_t* lists, uint32_t* spill,
+                   uint32_t* __restrict__ counts) {
   constexpr int kStage = 256, kRow = 20;         // signatures per stage, dwords per LDS row
   __shared__ __attribute__((aligned(16))) uint32_t tile[2][kStage * kRow];
+  __shared__ uint32_t tileId[2][kStage], tileMin[2][kStage / 32];   // node ids, the smallest of each 32
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
-  const uint32_t j0 = (gridDim.x - 1 - blockIdx.x) * (128 * JT);     // node ids are 32-bit
-  const uint32_t jw = j0 + wave * (32 * JT);               // the wavefront's first j
+  const uint32_t j0 = (gridDim.x - 1 - blockIdx.x) * (128 * JT);
+  const uint32_t jw = j0 + wave * (32 * JT);     // the wavefront's first position
   const float limit = bound >= 512u ? -513.f : 512.f - 2.f * (float)bound;
   i32x4_t b[JT][8];
   float thr[JT];                                 // +inf: inactive or full
-  uint32_t cnt[JT];
+  uint32_t cnt[JT], jid[JT], top[JT];            // matches held, node id, ids from top on are not needed
 #pragma unroll
   for (int t = 0; t < JT; ++t) {
     const uint32_t j = jw + 32 * t + col;
     uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+    jid[t] = 0;
     if (j < n) {
-      const uint4* p = reinterpret_cast<const uint4*>(sig + (uint64_t)j * 16 + 8 * half);
-      lo = p[0];
-      hi = p[1];
+      lo = ssig[(uint64_t)j * 4 + 2 * half];
+      hi = ssig[(uint64_t)j * 4 + 2 * half + 1];
+      jid[t] = ids[j];
     }
     const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
     for (int k = 0; k < 8; ++k) b[t][k] = bits_to_fp4(w[k]);
-    thr[t] = j < n && refs[j] <= maxRefs ? limit : __builtin_inff();
+    thr[t] = j < n && refs[jid[t]] <= maxRefs ? limit : __builtin_inff();
     cnt[t] = 0;
+    top[t] = jid[t];
   }
-  auto open = [&]() {
-    bool o = false;
-#pragma unroll
-    for (int t = 0; t < JT; ++t) o |= thr[t] < __builtin_inff();
-    return __any(o) != 0;
-  };
-  bool live = open();
-  const uint32_t iEnd = (uint32_t)(j0 + 128 * JT < n ? j0 + 128 * JT : n);
-  uint4 r[4];
-  auto load = [&](uint32_t i0) {
-    const uint32_t i = i0 + tid;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      r[q] = i < n ? reinterpret_cast<const uint4*>(sig + (uint64_t)i * 16)[q] : make_uint4(0, 0, 0, 0);
-  };
-  load(0);
+  // 128 JT divides C: a workgroup's positions are of one chunk
+  const uint32_t ch = j0 / C;
+  const uint32_t jl = min(j0 + 128 * JT, n) - 1;
+  const uint32_t pcLo = keys[j0] - ch * kPopBins, pcHi = keys[jl] - ch * kPopBins;
+  const uint32_t binLo = pcLo > bound ? pcLo - bound : 0;
+  const uint32_t binHi = bound >= 512u - pcHi ? 512u : pcHi + bound;
   int buf = 0;
-  for (uint32_t i0 = 0; i0 < iEnd; i0 += kStage, buf ^= 1) {
-    uint4* d = reinterpret_cast<uint4*>(&tile[buf][tid * kRow]);
+  for (uint32_t q = 0; q <= ch; ++q) {
+    bool live = false;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) d[q] = r[q];
-    if (!__syncthreads_or(live)) break;          // two buffers: one barrier per stage
-    if (i0 + kStage < iEnd) load(i0 + kStage);
-    for (int it = 0; it < kStage / 32; ++it) {
-      const uint32_t base = i0 + 32 * it;
-      if (!live || base >= jw + 32 * JT) break;  // every i of the tile is past the wavefront's j
-      const uint4* a4 = reinterpret_cast<const uint4*>(&tile[buf][(32 * it + col) * kRow + 8 * half]);
-      const uint4 lo = a4[0], hi = a4[1];
-      const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-      f32x16_t acc[JT];
+    for (int t = 0; t < JT; ++t) {
+      if (cnt[t] >= cap) thr[t] = __builtin_inff();   // every later match has a larger id
+      live |= thr[t] < __builtin_inff();
+    }
+    live = __any(live) != 0;
+    const uint32_t iBeg = off[q * kPopBins + binLo], iEnd = off[q * kPopBins + binHi + 1];
+    uint4 r[4];
+    uint32_t rid = 0;
+    auto load = [&](uint32_t i0) {
+      const uint32_t i = i0 + tid;
 #pragma unroll
-      for (int t = 0; t < JT; ++t)
+      for (int x = 0; x < 4; ++x) r[x] = i < iEnd ? ssig[(uint64_t)i * 4 + x] : make_uint4(0, 0, 0, 0);
+      rid = i < iEnd ? ids[i] : kNone;
+    };
+    load(iBeg);
+    for (uint32_t i0 = iBeg; i0 < iEnd; i0 += kStage, buf ^= 1) {
+      uint4* d = reinterpret_cast<uint4*>(&tile[buf][tid * kRow]);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+      for (int x = 0; x < 4; ++x) d[x] = r[x];
+      tileId[buf][tid] = rid;
+      uint32_t mn = rid;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const i32x4_t a = bits_to_fp4(w[k]);
+      for (int o = 16; o >= 1; o >>= 1) mn = min(mn, (uint32_t)__shfl_xor(mn, o, 64));
+      if (col == 0) tileMin[buf][tid >> 5] = mn;
+      if (!__syncthreads_or(live)) break;
+      if (i0 + kStage < iEnd) load(i0 + kStage);
+      if (!live) continue;
+      for (uint32_t base = i0; base < i0 + kStage && base < iEnd; base += 32) {
+        const uint4* a4 = reinterpret_cast<const uint4*>(&tile[buf][(base - i0 + col) * kRow + 8 * half]);
+        const uint4 lo = a4[0], hi = a4[1];
+        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        f32x16_t acc[JT];
 #pragma unroll
         for (int t = 0; t < JT; ++t)
-          acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
-              __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1),
-              __builtin_shufflevector(b[t][k], b[t][k], 0, 1, 2, 3, -1, -1, -1, -1), acc[t], 4, 4, 0, 0, 0, 0);
-      }
 #pragma unroll
-      for (int t = 0; t < JT; ++t) {
-        float m = acc[t][0];
+          for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
 #pragma unroll
-        for (int v = 1; v < 16; ++v) m = fmaxf(m, acc[t][v]);
-        if (!__any(m >= thr[t])) continue;
-        uint32_t hits = 0;
+        for (int k = 0; k < 8; ++k) {
+          const i32x4_t a = bits_to_fp4(w[k]);
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          hits |= (acc[t][v] >= thr[t] ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
-        hits <<= 4 * half;
-        hits |= __shfl_xor(hits, 32, 64);
-        const uint32_t j = jw + 32 * t + col;
-        if (j < base + 32) hits = j > base ? hits & ((1u << (j - base)) - 1u) : 0u;
-        while (hits && cnt[t] < cap) {
-          if (half == 0) lists[(uint64_t)j * cap + cnt[t]] = base + (uint32_t)(__ffs(hits) - 1);
-          hits &= hits - 1;
-          ++cnt[t];
+          for (int t = 0; t < JT; ++t)
+            acc[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+                __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1),
+                __builtin_shufflevector(b[t][k], b[t][k], 0, 1, 2, 3, -1, -1, -1, -1), acc[t], 4, 4, 0, 0, 0, 0);
         }
-        if (cnt[t] == cap) thr[t] = __builtin_inff();
+        const uint32_t least = tileMin[buf][(base - i0) >> 5];
+        const uint32_t rows = iEnd - base < 32 ? (1u << (iEnd - base)) - 1u : 0xFFFFFFFFu;
+#pragma unroll
+        for (int t = 0; t < JT; ++t) {
+          float m = acc[t][0];
+#pragma unroll
+          for (int v = 1; v < 16; ++v) m = fmaxf(m, acc[t][v]);
+          const float th = least < top[t] ? thr[t] : __builtin_inff();
+          if (!__any(m >= th)) continue;
+          uint32_t hits = 0;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) hits |= (acc[t][v] >= th ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+          hits <<= 4 * half;
+          hits |= __shfl_xor(hits, 32, 64);
+          hits &= rows;
+          const uint64_t at = (uint64_t)jid[t] * cap;
+          while (true) {
+            while (hits && cnt[t] < 2 * cap) {
+              const uint32_t id = tileId[buf][base - i0 + (uint32_t)(__ffs(hits) - 1)];
+              hits &= hits - 1;
+              if (id < top[t]) {
+                if (half == 0)
+                  __atomic_store_n(cnt[t] < cap ? lists + at + cnt[t] : spill + at + (cnt[t] - cap), id,
+                                   __ATOMIC_RELAXED);
+                ++cnt[t];
+              }
+            }
+            unsigned long long f = __ballot(half == 0 && cnt[t] == 2 * cap);
+            if (!f) break;
+            // full lists keep their smallest cap entries; four are loaded at a time
+            __threadfence_block();
+            while (f) {
+              int l[4];
+              uint32_t v[4][2];
+#pragma unroll
+              for (int x = 0; x < 4; ++x) {
+                l[x] = f ? __ffsll(f) - 1 : -1;
+                f &= f - 1;                                 // 0 stays 0
+                if (l[x] >= 0)
+                  load_list(lists, spill, (uint64_t)__builtin_amdgcn_readlane((int)jid[t], l[x]) * cap, 2 * cap, cap,
+                            lane, v[x]);
+              }
+#pragma unroll
+              for (int x = 0; x < 4; ++x) {
+                if (l[x] < 0) break;
+                const uint32_t last = order_list(
+                    lists, (uint64_t)__builtin_amdgcn_readlane((int)jid[t], l[x]) * cap, 2 * cap, cap, v[x]);
+                if (col == l[x]) { cnt[t] = cap; top[t] = last; }
+              }
+            }
+            __threadfence_block();
+          }
+        }
       }
-      live = open();
     }
   }
 #pragma unroll
   for (int t = 0; t < JT; ++t) {
     const uint32_t j = jw + 32 * t + col;
-    if (half == 0 && j < n) counts[j] = cnt[t];
+    if (half == 0 && j < n) counts[jid[t]] = cnt[t];
   }
+}
+
+// Every list in ascending order, cut to cap: one wavefront per node.
+__global__ void __launch_bounds__(256) k_list_order(uint64_t n, uint32_t cap, uint32_t* lists, uint32_t* spill,
+                                                    uint32_t* counts) {
+  const uint64_t j = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (j >= n) return;
+  const int lane = threadIdx.x & 63;
+  const uint32_t cnt = counts[j];
+  if (cnt > 1) {
+    uint32_t v[2];
+    load_list(lists, spill, j * cap, cnt, cap, lane, v);
+    order_list(lists, j * cap, cnt, cap, v);
+  }
+  if (cnt > cap && lane == 0) counts[j] = cap;
 }
 
 // Ranked pre-filter lists: every earlier node i < j within the bound, the K
@@ -505,16 +645,36 @@ __global__ void k_remap_inplace(uint32_t* __restrict__ rec, uint64_t n, const ui
     if ((m >> c) & 1u) r[1 + c] = corr[r[1 + c]];
 }
 
+// lists and spill hold cap entries per node each (spill is scratch).
 void exhaustive_lists(svd_ctx* c, const uint32_t* sig, uint64_t n, const uint64_t* refs, uint64_t maxRefs,
-                      uint32_t bound, uint32_t cap, uint32_t* lists, uint32_t* counts) {
-  // the widest tile that still gives every CU a workgroup
-  const uint64_t cus = (uint64_t)std::max(c->numCU, 1);
-  if (n >= 512 * cus)
-    k_exhaustive_lists<4><<<div_up(n, 512), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
-  else if (n >= 256 * cus)
-    k_exhaustive_lists<2><<<div_up(n, 256), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
+                      uint32_t bound, uint32_t cap, uint32_t* lists, uint32_t* spill, uint32_t* counts) {
+  const uint32_t chunks = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, n / 512));
+  const uint32_t C = div_up(div_up(n, chunks), 512) * 512;
+  const uint32_t nKeys = div_up(n, C) * kPopBins;
+  uint32_t bits = 1;
+  while (nKeys >> bits) ++bits;
+  uint32_t* keys = dalloc<uint32_t>(c, n);
+  uint32_t* keys2 = dalloc<uint32_t>(c, n);
+  uint32_t* ids = dalloc<uint32_t>(c, n);
+  uint32_t* ids2 = dalloc<uint32_t>(c, n);
+  uint32_t* off = dalloc<uint32_t>(c, (uint64_t)nKeys + 1);
+  uint4* ssig = dalloc<uint4>(c, n * 4);
+  k_list_keys<<<div_up(n, kB), kB, 0, c->stream>>>(sig, n, C, keys, ids);
+  size_t bytes = 0;
+  SVD_HIP(rocprim::radix_sort_pairs(nullptr, bytes, keys, keys2, ids, ids2, (size_t)n, 0, bits, c->stream));
+  void* tmp = c->arena->get(bytes + 16);
+  SVD_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, ids, ids2, (size_t)n, 0, bits, c->stream));
+  c->arena->put(tmp);
+  k_list_gather<<<div_up(n * 4, kB), kB, 0, c->stream>>>(sig, ids2, keys2, n, nKeys, ssig, off);
+  // two j tiles per wavefront where that still gives every CU a workgroup
+  if (n >= 256 * (uint64_t)std::max(c->numCU, 1))
+    k_exhaustive_lists<2><<<div_up(n, 256), 256, 0, c->stream>>>(ssig, ids2, keys2, off, (uint32_t)n, C, refs, maxRefs,
+                                                                 bound, cap, lists, spill, counts);
   else
-    k_exhaustive_lists<1><<<div_up(n, 128), 256, 0, c->stream>>>(sig, n, refs, maxRefs, bound, cap, lists, counts);
+    k_exhaustive_lists<1><<<div_up(n, 128), 256, 0, c->stream>>>(ssig, ids2, keys2, off, (uint32_t)n, C, refs, maxRefs,
+                                                                 bound, cap, lists, spill, counts);
+  k_list_order<<<div_up(n, 4), 256, 0, c->stream>>>(n, cap, lists, spill, counts);
+  dfree(c, keys); dfree(c, keys2); dfree(c, ids); dfree(c, ids2); dfree(c, off); dfree(c, ssig);
 }
 
 LevelView make_view(const svd_octree* o, const std::vector<uint64_t*>& vox) {
@@ -640,7 +800,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
     clk.mark(1);
     if (!learned) {
       clk.mark(2);
-      if (n && !ranked) exhaustive_lists(c, sig, n, refs[lev], maxRefs, bound, cap, lists, counts);
+      if (n && !ranked) exhaustive_lists(c, sig, n, refs[lev], maxRefs, bound, cap, lists, dv, counts);
       else if (n && cap <= 16)
         k_ranked_lists<16><<<div_up(n, 256), 256, 0, c->stream>>>(sig, n, refs[lev], maxRefs, bound, cap, lists,
                                                                    counts);

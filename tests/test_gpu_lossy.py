@@ -104,6 +104,38 @@ def test_lossy_ranked_bit_exact(ctx, name, mode):
     assert g.encoded_bytes(S.FMT_SVDAG) == o.encode(0)
 
 
+@pytest.mark.parametrize("cap", [1, 2, 64])
+@pytest.mark.parametrize("bound", [1, 24, 600])
+def test_lossy_exhaustive_list_edges(ctx, cap, bound):
+    """The matrix-core scan at its edges: lists that overflow twice their
+    capacity (capacities 1, 2 and 64), bounds whose popcount window is one
+    side of the range or all of it (600: every pair matches), levels of a few
+    to a few thousand nodes (partial 32-row tiles and stages, one and several
+    chunks)."""
+    codes, L = random_codes(6, 20000, 3), 6
+    g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
+    st_g = g.lossy_merge(1, L - 2, max_diff=bound, list_cap=cap)
+    st_o = o.lossy_merge(1, L - 2, max_diff=bound, list_cap=cap)
+    assert_same_stats(st_g, st_o)
+    assert_same_dag(g, o, L)
+
+
+def test_lossy_exhaustive_lists_of_a_large_level(ctx):
+    """A level of some 260K nodes takes the two-tile workgroups.  At bound 1 no
+    list fills, so the ranked proposer (its own kernel, every earlier node)
+    lists the same pairs: the listed and verified counts agree."""
+    codes, L = random_codes(9, 1500000, 5), 9
+    st = []
+    for ranked in (False, True):
+        g = gpu_dag(ctx, codes, L)
+        assert g.level_size(S.VIEW_DAG, 6) > 200000
+        st.append(g.lossy_merge(6, 6, max_diff=1, list_cap=64, ranked=ranked))
+        g.free()
+    assert st[0]["listed"][0] > 0
+    for f in ("candidates", "listed", "verified"):
+        np.testing.assert_array_equal(st[0][f], st[1][f], err_msg=f)
+
+
 def test_lossy_error_within_accounted_bound(ctx):
     codes, L = W.cave_codes(7, seed=3), 7
     g = gpu_dag(ctx, codes, L)
