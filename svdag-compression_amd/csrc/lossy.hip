@@ -21,6 +21,7 @@
 //   5. compact the level, remap the parent level's child pointers.
 // Finally the whole DAG is re-deduplicated exactly (:1176).
 #include <algorithm>
+#include <type_traits>
 #include "svd_internal.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -29,11 +30,14 @@ namespace svd {
 namespace {
 
 constexpr int kB = 256;
+constexpr uint32_t kRounds = 3;      // resolution rounds between two looks at the unresolved flag
 constexpr uint8_t kUnres = 0, kRep = 1, kMerged = 2;
 
 struct LevelView {
   const uint32_t* rec[kMaxLevels];
   const uint64_t* vox[kMaxLevels];
+  const uint32_t* occ;            // 512-bit occupancies (16 words) of every node of level occLev
+  uint32_t occLev;
   uint32_t L;
 };
 
@@ -484,79 +488,150 @@ __global__ void k_lists_from_sorted(const uint64_t* __restrict__ keys, uint64_t 
   counts[hi] = cnt;
 }
 
-// Exact voxel difference of the subtrees a0, b0 at level lev0, capped at
-// bound + 1 (the running total only grows, so the capped value does not depend
-// on the visiting order).
-__device__ uint32_t subtree_diff(const LevelView& v, uint32_t lev0, uint32_t a0, uint32_t b0, uint32_t bound) {
-  if (a0 == b0) return 0;
-  const uint32_t L = v.L;
-  if (lev0 == L - 1) {
-    const uint32_t d = __popc(mask_of(v, lev0, a0) ^ mask_of(v, lev0, b0));
-    return d > bound ? bound + 1 : d;
+__device__ __forceinline__ uint32_t occ_diff(const LevelView& v, uint32_t a, uint32_t b) {
+  const uint4* pa = reinterpret_cast<const uint4*>(v.occ + (uint64_t)a * 16);
+  const uint4* pb = reinterpret_cast<const uint4*>(v.occ + (uint64_t)b * 16);
+  uint32_t h = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint4 x = pa[q], y = pb[q];
+    h += __popc(x.x ^ y.x) + __popc(x.y ^ y.y) + __popc(x.z ^ y.z) + __popc(x.w ^ y.w);
   }
+  return h;
+}
+
+// Adds the voxel difference of the subtrees a, b (level lev, D levels above
+// v.occLev) to acc; true once it exceeds the bound.  One nested loop per level
+// keeps every index in registers.
+template <int D>
+__device__ __forceinline__ bool add_diff(const LevelView& v, uint32_t lev, uint32_t a, uint32_t b, uint32_t bound,
+                                         uint64_t& acc) {
+  if constexpr (D == 0) {
+    acc += occ_diff(v, a, b);
+  } else {
+    const uint32_t* ra = v.rec[lev] + (uint64_t)a * kRecWords;
+    const uint32_t* rb = v.rec[lev] + (uint64_t)b * kRecWords;
+    const uint32_t ma = ra[0] & 0xFFu, mb = rb[0] & 0xFFu;
+    for (uint32_t m = ma ^ mb; m; m &= m - 1) {          // one-sided children
+      const int c = __ffs(m) - 1;
+      acc += v.vox[lev + 1][((ma >> c) & 1u) ? ra[1 + c] : rb[1 + c]];
+    }
+    if (acc > bound) return true;
+    for (uint32_t m = ma & mb; m; m &= m - 1) {
+      const int c = __ffs(m) - 1;
+      const uint32_t ca = ra[1 + c], cb = rb[1 + c];
+      if (ca != cb && add_diff<D - 1>(v, lev + 1, ca, cb, bound, acc)) return true;
+    }
+  }
+  return acc > bound;
+}
+
+// The same for any depth, with the path on a stack.
+__device__ bool add_diff_deep(const LevelView& v, uint32_t lev0, uint32_t a0, uint32_t b0, uint32_t bound,
+                              uint64_t& acc) {
   uint32_t sa[kMaxLevels], sb[kMaxLevels];
   uint8_t sc[kMaxLevels];
   int top = 0;
   sa[0] = a0; sb[0] = b0; sc[0] = 0;
-  uint64_t acc = 0;
   while (top >= 0) {
-    const uint32_t lev = lev0 + (uint32_t)top;     // < L - 1 for every frame on the stack
+    const uint32_t lev = lev0 + (uint32_t)top;     // < occLev for every frame on the stack
     const uint32_t a = sa[top], b = sb[top];
     const uint32_t ma = mask_of(v, lev, a), mb = mask_of(v, lev, b);
     int c = sc[top];
     bool pushed = false;
-    for (; c < 8; ++c) {
+    for (; c < 8 && !pushed; ++c) {
       const bool ea = (ma >> c) & 1u, eb = (mb >> c) & 1u;
       if (ea && eb) {
         const uint32_t ca = child_of(v, lev, a, c), cb = child_of(v, lev, b, c);
-        if (ca != cb) {
-          if (lev + 1 == L - 1) {
-            acc += __popc(mask_of(v, lev + 1, ca) ^ mask_of(v, lev + 1, cb));
-          } else {
-            sc[top] = (uint8_t)(c + 1);
-            ++top;
-            sa[top] = ca; sb[top] = cb; sc[top] = 0;
-            pushed = true;
-            break;
-          }
+        if (ca == cb) continue;
+        if (lev + 1 == v.occLev) {
+          acc += occ_diff(v, ca, cb);
+        } else {
+          sc[top] = (uint8_t)(c + 1);
+          ++top;
+          sa[top] = ca; sb[top] = cb; sc[top] = 0;
+          pushed = true;
         }
-      } else if (ea) {
-        acc += v.vox[lev + 1][child_of(v, lev, a, c)];
-      } else if (eb) {
-        acc += v.vox[lev + 1][child_of(v, lev, b, c)];
+      } else if (ea || eb) {
+        acc += v.vox[lev + 1][child_of(v, lev, ea ? a : b, c)];
       }
-      if (acc > bound) return bound + 1;
+      if (acc > bound) return true;
     }
     if (!pushed) --top;
   }
-  return (uint32_t)acc;
+  return false;
 }
 
-__global__ void k_verify(LevelView v, uint32_t lev, const uint32_t* __restrict__ lists,
-                         const uint32_t* __restrict__ counts, uint64_t n, uint32_t cap, uint32_t bound,
-                         uint32_t* __restrict__ dv, unsigned long long* __restrict__ stats) {
-  uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n * cap) return;
-  const uint64_t j = e / cap;
-  const uint32_t t = (uint32_t)(e - j * cap);
-  if (t >= counts[j]) return;
-  const uint32_t d = subtree_diff(v, lev, lists[e], (uint32_t)j, bound);
-  dv[e] = d;
-  atomicAdd(&stats[0], 1ull);
-  if (d <= bound) atomicAdd(&stats[1], 1ull);
+// Exact voxel difference of the subtrees a, b at level lev, capped at bound +
+// 1 (the running total only grows, so the capped value does not depend on the
+// visiting order).  The descent ends at level occLev: three levels above the
+// bottom a node's occupancy is its voxels, so the difference of two such nodes
+// is one 64-byte XOR/popcount instead of up to 73 records.  D = occLev - lev
+// for up to kMaxD levels (0 from occLev down), D = kDeep beyond.
+constexpr int kMaxD = 4, kDeep = kMaxD + 1;
+template <int D>
+__device__ __forceinline__ uint32_t subtree_diff(const LevelView& v, uint32_t lev, uint32_t a, uint32_t b,
+                                                 uint32_t bound) {
+  if (a == b) return 0;
+  uint64_t acc = 0;
+  bool over;
+  if constexpr (D == kDeep) over = add_diff_deep(v, lev, a, b, bound, acc);
+  else over = add_diff<D>(v, lev, a, b, bound, acc);
+  return over ? bound + 1 : (uint32_t)acc;
+}
+
+// Sums of a workgroup of 256 added to two words, one atomic each: a grid
+// strides over its work so that few workgroups meet at the address.
+__device__ __forceinline__ void add_block(unsigned long long a, unsigned long long b, unsigned long long* da,
+                                          unsigned long long* db) {
+  __shared__ unsigned long long part[2][4];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    a += __shfl_xor(a, o, 64);
+    b += __shfl_xor(b, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) { part[0][threadIdx.x >> 6] = a; part[1][threadIdx.x >> 6] = b; }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    a = part[0][0] + part[0][1] + part[0][2] + part[0][3];
+    b = part[1][0] + part[1][1] + part[1][2] + part[1][3];
+    if (a) atomicAdd(da, a);
+    if (b) atomicAdd(db, b);
+  }
+}
+
+template <int D>
+__global__ void __launch_bounds__(256) k_verify(LevelView v, uint32_t lev, const uint32_t* __restrict__ lists,
+                                                const uint32_t* __restrict__ counts, uint64_t n, uint32_t cap,
+                                                uint32_t bound, uint32_t* __restrict__ dv,
+                                                unsigned long long* __restrict__ stats) {
+  unsigned long long listed = 0, kept = 0;
+  for (uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x; e < n * cap; e += (uint64_t)gridDim.x * 256) {
+    const uint64_t j = e / cap;
+    const uint32_t t = (uint32_t)(e - j * cap);
+    if (t >= counts[j]) continue;
+    const uint32_t d = subtree_diff<D>(v, lev, lists[e], (uint32_t)j, bound);
+    dv[e] = d;
+    ++listed;
+    kept += d <= bound ? 1 : 0;
+  }
+  add_block(listed, kept, &stats[0], &stats[1]);
 }
 
 // Node state word: state << 32 | target node (one 64-bit word, so a reader
 // that sees "merged" also sees the target).
 constexpr uint64_t kStRep = (uint64_t)kRep << 32, kStMerged = (uint64_t)kMerged << 32;
 
-__global__ void k_resolve_init(uint64_t n, const uint64_t* __restrict__ refs, uint64_t maxRefs,
-                               unsigned long long* __restrict__ st, unsigned long long* __restrict__ stats) {
-  uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const bool cand = refs[j] <= maxRefs;
-  st[j] = cand ? (unsigned long long)kUnres << 32 : (unsigned long long)(kStRep | j);
-  if (cand) atomicAdd(&stats[2], 1ull);
+__global__ void __launch_bounds__(256) k_resolve_init(uint64_t n, const uint64_t* __restrict__ refs, uint64_t maxRefs,
+                                                      unsigned long long* __restrict__ st,
+                                                      unsigned long long* __restrict__ stats) {
+  unsigned long long cands = 0;
+  for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < n; j += (uint64_t)gridDim.x * 256) {
+    const bool cand = refs[j] <= maxRefs;
+    st[j] = cand ? (unsigned long long)kUnres << 32 : (unsigned long long)(kStRep | j);
+    cands += cand ? 1 : 0;
+  }
+  add_block(cands, 0, &stats[2], &stats[2]);
 }
 
 // One round: an unresolved j walks its verified entries in order.  A
@@ -564,7 +639,8 @@ __global__ void k_resolve_init(uint64_t n, const uint64_t* __restrict__ refs, ui
 // target (a representative), taken when the exact difference to j is within
 // the bound; an unresolved entry makes j wait.  States only move away from
 // "unresolved", so a stale read delays a node by one round and never changes
-// its outcome.
+// its outcome.  *unresolved is set while a node waits.
+template <int D>
 __global__ void k_resolve(LevelView v, uint32_t lev, const uint32_t* __restrict__ lists,
                           const uint32_t* __restrict__ dv, const uint32_t* __restrict__ counts, uint64_t n,
                           uint32_t cap, uint32_t bound, unsigned long long* st, uint32_t* __restrict__ tdist,
@@ -586,7 +662,7 @@ __global__ void k_resolve(LevelView v, uint32_t lev, const uint32_t* __restrict_
     }
     if (s == kMerged) {
       const uint32_t r = (uint32_t)w;
-      const uint32_t d = subtree_diff(v, lev, r, (uint32_t)j, bound);
+      const uint32_t d = subtree_diff<D>(v, lev, r, (uint32_t)j, bound);
       if (d <= bound) {
         tdist[j] = d;
         __atomic_store_n(&st[j], (unsigned long long)(kStMerged | r), __ATOMIC_RELAXED);
@@ -594,7 +670,7 @@ __global__ void k_resolve(LevelView v, uint32_t lev, const uint32_t* __restrict_
       }
       continue;
     }
-    atomicAdd(unresolved, 1u);
+    __atomic_store_n(unresolved, 1u, __ATOMIC_RELAXED);
     return;
   }
   __atomic_store_n(&st[j], (unsigned long long)(kStRep | j), __ATOMIC_RELAXED);
@@ -610,30 +686,31 @@ __global__ void k_rep_flag(const unsigned long long* __restrict__ st, uint64_t n
   hit[j] = 0u;
 }
 
-__global__ void k_lossy_compact(const uint32_t* __restrict__ rec, const uint64_t* __restrict__ vox,
-                                const unsigned long long* __restrict__ st, const uint32_t* __restrict__ tdist,
-                                const uint32_t* __restrict__ pos, const uint64_t* __restrict__ refs, uint64_t n,
-                                uint32_t* __restrict__ out, uint64_t* __restrict__ outVox,
-                                uint32_t* __restrict__ corr, uint32_t* __restrict__ hit,
-                                unsigned long long* __restrict__ stats) {
-  uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const unsigned long long w = st[j];
-  if ((w >> 32) == kRep) {
-    const uint32_t p = pos[j];
-    const uint32_t* s = rec + j * kRecWords;
-    uint32_t* d = out + (uint64_t)p * kRecWords;
+__global__ void __launch_bounds__(256)
+k_lossy_compact(const uint32_t* __restrict__ rec, const uint64_t* __restrict__ vox,
+                const unsigned long long* __restrict__ st, const uint32_t* __restrict__ tdist,
+                const uint32_t* __restrict__ pos, const uint64_t* __restrict__ refs, uint64_t n,
+                uint32_t* __restrict__ out, uint64_t* __restrict__ outVox, uint32_t* __restrict__ corr,
+                uint32_t* __restrict__ hit, unsigned long long* __restrict__ stats) {
+  unsigned long long err = 0, clusters = 0;
+  for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < n; j += (uint64_t)gridDim.x * 256) {
+    const unsigned long long w = st[j];
+    if ((w >> 32) == kRep) {
+      const uint32_t p = pos[j];
+      const uint32_t* s = rec + j * kRecWords;
+      uint32_t* d = out + (uint64_t)p * kRecWords;
 #pragma unroll
-    for (int k = 0; k < kRecWords; ++k) d[k] = s[k];
-    outVox[p] = vox[j];
-    corr[j] = p;
-  } else {
-    corr[j] = pos[(uint32_t)w];
-    atomicAdd(&stats[3], 1ull);
-    atomicAdd(&stats[4], (unsigned long long)tdist[j] * refs[j]);
-    // clusters: representatives with at least one member
-    if (atomicExch(&hit[(uint32_t)w], 1u) == 0u) atomicAdd(&stats[8], 1ull);
+      for (int k = 0; k < kRecWords; ++k) d[k] = s[k];
+      outVox[p] = vox[j];
+      corr[j] = p;
+    } else {
+      corr[j] = pos[(uint32_t)w];
+      err += (unsigned long long)tdist[j] * refs[j];
+      // clusters: representatives with at least one member
+      if (atomicExch(&hit[(uint32_t)w], 1u) == 0u) ++clusters;
+    }
   }
+  add_block(err, clusters, &stats[4], &stats[8]);
 }
 
 __global__ void k_remap_inplace(uint32_t* __restrict__ rec, uint64_t n, const uint32_t* __restrict__ corr) {
@@ -682,6 +759,21 @@ LevelView make_view(const svd_octree* o, const std::vector<uint64_t*>& vox) {
   v.L = o->levels;
   for (uint32_t l = 0; l < o->levels; ++l) { v.rec[l] = o->dag[l].rec; v.vox[l] = vox[l]; }
   return v;
+}
+
+// fn(std::integral_constant<int, D>) for the level's depth above v.occLev
+template <class F>
+void with_depth(const LevelView& v, uint32_t lev, F fn) {
+  const uint32_t d = lev < v.occLev ? v.occLev - lev : 0;
+  static_assert(kMaxD == 4, "the cases below");
+  switch (d) {
+    case 0: return fn(std::integral_constant<int, 0>());
+    case 1: return fn(std::integral_constant<int, 1>());
+    case 2: return fn(std::integral_constant<int, 2>());
+    case 3: return fn(std::integral_constant<int, 3>());
+    case 4: return fn(std::integral_constant<int, 4>());
+    default: return fn(std::integral_constant<int, kDeep>());
+  }
 }
 
 struct PhaseClock {
@@ -765,7 +857,10 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
   }
   check_launch("voxel counts");
   unsigned long long* dstats = dalloc<unsigned long long>(c, 9);
-  uint32_t* unresolved = dalloc<uint32_t>(c, 1);
+  uint32_t* unresolved = dalloc<uint32_t>(c, kRounds);
+  uint32_t* bottom = nullptr;          // occupancies of level L-3, once the level is final
+  // grid of the counting kernels: a resident wave of workgroups, one atomic each
+  auto grid = [&](uint64_t work) { return std::min<uint32_t>(div_up(work, 256), 8 * (uint32_t)std::max(c->numCU, 1)); };
   PhaseClock clk(c, 7);
 
   for (int lev = (int)p->lev_hi; lev >= (int)p->lev_lo; --lev) {
@@ -838,26 +933,45 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
     }
     if (!learned) clk.mark(3);
     clk.mark(4);
-    if (n) k_verify<<<div_up(n * cap, kB), kB, 0, c->stream>>>(v, (uint32_t)lev, lists, counts, n, cap, bound, dv,
-                                                             dstats + 5);
-    check_launch("k_verify");
-    clk.mark(5);
-    if (n) k_resolve_init<<<div_up(n, kB), kB, 0, c->stream>>>(n, refs[lev], maxRefs, state, dstats + 5);
-    check_launch("k_resolve_init");
-    for (uint64_t round = 0; n; ++round) {
-      fill_u32(c, unresolved, 0u, 1);
-      k_resolve<<<div_up(n, kB), kB, 0, c->stream>>>(v, (uint32_t)lev, lists, dv, counts, n, cap, bound, state, tdist,
-                                                     unresolved);
-      check_launch("k_resolve");
-      if (read_u32(c, unresolved) == 0) break;
-      if (round > n) throw Error{SVD_ERR_DEVICE, "lossy resolution did not converge"};
+    // the exact difference ends at the occupancies of level L-3 (or at the
+    // level's own from there down)
+    v.occ = sig;
+    v.occLev = (uint32_t)lev;
+    if ((uint32_t)lev + 3 < L) {
+      if (!bottom) {
+        const uint64_t nb = o->dag[L - 3].n;
+        bottom = dalloc<uint32_t>(c, (nb + 1) * 16);
+        if (nb) k_signatures<<<div_up(nb, kB), kB, 0, c->stream>>>(v, L - 3, nb, bottom);
+        check_launch("k_signatures");
+      }
+      v.occ = bottom;
+      v.occLev = L - 3;
     }
+    with_depth(v, (uint32_t)lev, [&](auto d) {
+      if (n) k_verify<d()><<<grid(n * cap), 256, 0, c->stream>>>(v, (uint32_t)lev, lists, counts, n, cap, bound, dv,
+                                                                 dstats + 5);
+      check_launch("k_verify");
+      clk.mark(5);
+      if (n) k_resolve_init<<<grid(n), 256, 0, c->stream>>>(n, refs[lev], maxRefs, state, dstats + 5);
+      check_launch("k_resolve_init");
+      // kRounds rounds between looks: a round over settled nodes costs less
+      // than a read-back (2 to 6 rounds settle the levels measured)
+      for (uint64_t round = 0; n; round += kRounds) {
+        fill_u32(c, unresolved, 0u, kRounds);
+        for (uint32_t r = 0; r < kRounds; ++r)
+          k_resolve<d()><<<div_up(n, kB), kB, 0, c->stream>>>(v, (uint32_t)lev, lists, dv, counts, n, cap, bound, state,
+                                                              tdist, unresolved + r);
+        check_launch("k_resolve");
+        if (read_u32(c, unresolved + kRounds - 1) == 0) break;
+        if (round > n) throw Error{SVD_ERR_DEVICE, "lossy resolution did not converge"};
+      }
+    });
     if (n) k_rep_flag<<<div_up(n, kB), kB, 0, c->stream>>>(state, n, pos, hit);
     scan_exclusive(c, pos, pos, n, total);
     const uint64_t kept = n ? read_u32(c, total) : 0;
     uint32_t* newRec = dalloc<uint32_t>(c, (kept + 1) * kRecWords);
     uint64_t* newVox = dalloc<uint64_t>(c, kept + 1);
-    if (n) k_lossy_compact<<<div_up(n, kB), kB, 0, c->stream>>>(lv.rec, vox[lev], state, tdist, pos, refs[lev], n,
+    if (n) k_lossy_compact<<<grid(n), 256, 0, c->stream>>>(lv.rec, vox[lev], state, tdist, pos, refs[lev], n,
                                                               newRec, newVox, corr, hit, dstats);
     check_launch("k_lossy_compact");
     const uint64_t np = o->dag[lev - 1].n;
@@ -867,7 +981,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
     uint64_t hs[9];
     SVD_HIP(hipMemcpyAsync(hs, dstats, sizeof(hs), hipMemcpyDeviceToHost, c->stream));
     SVD_HIP(hipStreamSynchronize(c->stream));
-    st.merged = hs[3];
+    st.merged = n - kept;
     st.error_bound = hs[4];
     st.listed = hs[5];
     st.verified = hs[6];
@@ -891,7 +1005,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
   }
   for (auto* r : refs) dfree(c, r);
   for (auto* x : vox) dfree(c, x);
-  dfree(c, dstats); dfree(c, unresolved);
+  dfree(c, dstats); dfree(c, unresolved); dfree(c, bottom);
   // final exact dedup of every level (geom_octree_extension.cpp:1176)
   std::vector<Level> reduced;
   const uint64_t nn = dedup_all(c, L, o->dag, reduced);

@@ -120,6 +120,29 @@ def test_lossy_exhaustive_list_edges(ctx, cap, bound):
     assert_same_dag(g, o, L)
 
 
+@pytest.mark.parametrize("L", [4, 7, 8, 9, 10])
+def test_lossy_exact_difference_depths(ctx, L):
+    """Octants that are copies of one another but for a few voxels, so that
+    nodes of every level are compared down to the occupancies three levels
+    above the bottom: each nesting depth of the difference (level 1 of 4 to 8
+    levels) and the stack walk beyond (9 and 10 levels)."""
+    rng = np.random.default_rng(L)
+    sub = 3 * (L - 1)
+    base = np.unique(rng.integers(0, 1 << sub, 2500, dtype=np.uint64))
+    parts = []
+    for o in range(6):
+        keep = np.ones(base.size, bool)
+        keep[rng.choice(base.size, 2 * o, replace=False)] = False
+        parts.append(base[keep] | np.uint64(o << sub))
+    codes = np.unique(np.concatenate(parts))
+    for bound in (3, 9):
+        g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
+        st_g = g.lossy_merge(1, L - 2, max_diff=bound)
+        st_o = o.lossy_merge(1, L - 2, max_diff=bound)
+        assert_same_stats(st_g, st_o)
+        assert_same_dag(g, o, L)
+
+
 def test_lossy_exhaustive_lists_of_a_large_level(ctx):
     """A level of some 260K nodes takes the two-tile workgroups.  At bound 1 no
     list fills, so the ranked proposer (its own kernel, every earlier node)
