@@ -58,6 +58,16 @@ def test_points_svo_equals_oracle(ctx, L, n, seed):
     assert g.encoded_bytes(S.FMT_SSVDAG) == o.encode(2)
 
 
+def test_points_deep_creation_keys(ctx):
+    """21 levels: the creation key (first point, 60 path bits) takes more than
+    64 bits from 32 points on, so it is sorted in two steps; 300 points in a
+    few clumps share paths down to the last levels."""
+    rng = np.random.default_rng(3)
+    bmin, bmax = (0.0, 0.0, 0.0), (1.0, 1.0, 1.0)
+    pts = rng.random((12, 3))[rng.integers(0, 12, 300)] + rng.integers(-3, 4, (300, 3)) * 2.0 ** -21
+    _compare(ctx, np.ascontiguousarray(np.clip(pts, 0.0, 1.0)), 21, bmin, bmax)
+
+
 def test_points_dyadic_box_device_input(ctx):
     """A dyadic box (exact arithmetic) with points on every kind of face, the
     points given on the device."""
