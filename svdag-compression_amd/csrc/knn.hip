@@ -10,6 +10,7 @@
 // With signatures given, the candidates are scored by the exact Hamming
 // distance of the 512-bit occupancies instead (the embedding only decides
 // which nodes meet in a window): the learned proposer's re-ranking.
+#include <algorithm>
 #include "svd_internal.hpp"
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -22,23 +23,219 @@ constexpr int kMaxK = 32;
 constexpr int kTile = 256;
 constexpr int kRow = kDim + 1;             // padded LDS row (no bank conflicts)
 
+// Keys of `tables` orderings of every point: keys[t n + i] = t << bits | sign
+// bits, so that one stable sort orders all of them.
 __global__ void k_lsh_keys(const float* __restrict__ e, uint64_t n, const float* __restrict__ h, uint32_t bits,
-                           uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                           uint32_t tables, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   float x[kDim];
 #pragma unroll
   for (int d = 0; d < kDim; ++d) x[d] = e[i * kDim + d];
-  uint32_t key = 0;
-  for (uint32_t b = 0; b < bits; ++b) {
-    const float* hp = h + (uint64_t)b * kDim;
-    float s = 0.f;
+  for (uint32_t t = 0; t < tables; ++t) {
+    uint32_t key = t << bits;
+    for (uint32_t b = 0; b < bits; ++b) {
+      const float* hp = h + ((uint64_t)t * bits + b) * kDim;
+      float s = 0.f;
 #pragma unroll
-    for (int d = 0; d < kDim; ++d) { const float q = x[d] * hp[d]; s = s + q; }
-    if (s > 0.f) key |= 1u << b;
+      for (int d = 0; d < kDim; ++d) { const float q = x[d] * hp[d]; s = s + q; }
+      if (s > 0.f) key |= 1u << b;
+    }
+    keys[t * n + i] = key;
+    vals[t * n + i] = (uint32_t)i;
   }
-  keys[i] = key;
-  vals[i] = (uint32_t)i;
+}
+
+// ---- windows on the matrix cores (signatures, k <= 16, n <= 2^22) --------------
+// The running list of a node is 16 ascending keys (Hamming << 22 | node), so
+// (distance, index) order is integer order: 10 + 22 bits.
+constexpr uint32_t kIdBits = 22, kIdMask = (1u << kIdBits) - 1u;
+constexpr int kList = 16;
+constexpr int kQ = 128;                    // queries per workgroup, 32 per wavefront
+constexpr int kMaxW = 96;                  // the widest window
+constexpr int kWinRows = kQ + 2 * kMaxW;   // rows a workgroup meets
+constexpr int kSigRow = 20;                // dwords per LDS row (eight lanes' 16-byte reads in distinct banks)
+constexpr int kHash = 1024;                // >= 3 x kWinRows
+constexpr int kMaxTiles = (32 + 2 * kMaxW + 31) / 32;
+
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// One signature word as 32 fp4 values, bit 0 -> +1.0, 1 -> -1.0; bit 4p + d is
+// nibble p of dword d (any order of the 512 positions serves).
+__device__ __forceinline__ i32x4_t bits_to_fp4(uint32_t w) {
+  constexpr uint32_t kOne = 0x22222222u, kSign = 0x88888888u;
+  i32x4_t r;
+  r[0] = (int)(((w << 3) & kSign) | kOne);
+  r[1] = (int)(((w << 2) & kSign) | kOne);
+  r[2] = (int)(((w << 1) & kSign) | kOne);
+  r[3] = (int)((w & kSign) | kOne);
+  return r;
+}
+__device__ __forceinline__ uint32_t med3(uint32_t a, uint32_t b, uint32_t c) {
+  return max(min(a, b), min(max(a, b), c));
+}
+
+// One table's windows: a wavefront's 32 consecutive sorted positions (the
+// columns) meet the 32 + 2W rows around them.  With bits as +-1 the dot
+// product is 512 - 2 Hamming; a tile of 32 x 32 distances is 8 of
+// v_mfma_f32_32x32x64_f8f6f4 (fp4, exact sums), which costs next to nothing.
+// Accumulator element v of lane l is row 8 (v/4) + 4 (l/32) + v%4, column
+// l%32: the two lanes of a column insert half of its rows each into a sorted
+// list of 16 keys (16 medians, skipped while no lane has a key below its
+// worst), the first starting from the running list, the second from copies of
+// its worst key, and the 16 smallest of both are the new list.  Candidates
+// that the running list already holds are masked out: the rows' ids are in a
+// hash set, which every list entry looks itself up in.  Bound by the inserts.
+// One lane per point with the window's XOR/popcounts took 0.66-1.22 ms per
+// table on 466K nodes (W = 64), bound by a chain of some 2500 cycles per row.
+__global__ void __launch_bounds__(256) k_window_keys(const uint32_t* __restrict__ sig,
+                                                     const uint32_t* __restrict__ order, uint32_t n, uint32_t W,
+                                                     int first, uint32_t* __restrict__ best) {
+  __shared__ __attribute__((aligned(16))) uint32_t rows[kWinRows * kSigRow];
+  __shared__ __attribute__((aligned(16))) uint32_t ids[kWinRows + 32];
+  __shared__ uint32_t setId[kHash];
+  __shared__ uint32_t setRow[kHash];
+  __shared__ uint32_t dup[kQ][kMaxTiles];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+  const int64_t lo = (int64_t)blockIdx.x * kQ - (int64_t)W;     // sorted position of row 0
+  const int nrows = kQ + 2 * (int)W;
+  const int tiles = (32 + 2 * (int)W + 31) / 32;
+  for (int r = tid; r < kWinRows + 32; r += 256) {
+    const int64_t q = lo + r;
+    ids[r] = r < nrows && q >= 0 && q < (int64_t)n ? order[q] : kNone;
+  }
+  if (!first) {
+    for (int s = tid; s < kHash; s += 256) setId[s] = kNone;
+    for (int s = tid; s < kQ * kMaxTiles; s += 256) (&dup[0][0])[s] = 0u;
+  }
+  __syncthreads();
+  for (int t = tid; t < kWinRows * 4; t += 256) {
+    const int r = t >> 2;
+    const uint32_t id = ids[r];
+    *reinterpret_cast<uint4*>(&rows[r * kSigRow + 4 * (t & 3)]) =
+        id != kNone ? reinterpret_cast<const uint4*>(sig + (uint64_t)id * 16)[t & 3] : make_uint4(0, 0, 0, 0);
+  }
+  if (!first) {
+    for (int r = tid; r < nrows; r += 256) {
+      const uint32_t id = ids[r];
+      if (id == kNone) continue;
+      uint32_t h = (id * 2654435761u) >> 22;
+      while (atomicCAS(&setId[h], kNone, id) != kNone) h = (h + 1) & (kHash - 1);   // ids are distinct
+      setRow[h] = (uint32_t)r;
+    }
+  }
+  __syncthreads();
+  const int base = 32 * wave;                    // the wavefront's first row
+  const uint32_t x = ids[base + col + (int)W];   // kNone past the last point
+  uint32_t b[kList];
+#pragma unroll
+  for (int t = 0; t < kList; ++t) b[t] = kNone;
+  if (!first && x != kNone) {
+    const uint4* p = reinterpret_cast<const uint4*>(best + (uint64_t)x * kList);
+#pragma unroll
+    for (int t = 0; t < kList / 4; ++t) {
+      const uint4 u = p[t];
+      b[4 * t] = u.x; b[4 * t + 1] = u.y; b[4 * t + 2] = u.z; b[4 * t + 3] = u.w;
+    }
+    // each half looks its eight entries up
+    const uint4 u = p[2 * half], w = p[2 * half + 1];
+    const uint32_t mine[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const uint32_t key = mine[t];
+      if (key == kNone) continue;
+      const uint32_t id = key & kIdMask;
+      uint32_t h = (id * 2654435761u) >> 22, got;
+      while ((got = setId[h]) != kNone && got != id) h = (h + 1) & (kHash - 1);
+      if (got == kNone) continue;
+      const int r = (int)setRow[h] - base;
+      if (r >= 0 && r < 32 * tiles) atomicOr(&dup[base + col][r >> 5], 1u << (r & 31));
+    }
+  }
+  if (half) {
+#pragma unroll
+    for (int t = 0; t < kList; ++t) b[t] = b[kList - 1];
+  }
+  __syncthreads();
+  i32x4_t qf[8];
+  {
+    const uint4* p = reinterpret_cast<const uint4*>(&rows[(base + col + (int)W) * kSigRow + 8 * half]);
+    const uint4 u = p[0], w = p[1];
+    const uint32_t q[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) qf[k] = bits_to_fp4(q[k]);
+  }
+  for (int t = 0; t < tiles; ++t) {
+    const int r0 = base + 32 * t;                // first row of the tile
+    f32x16_t acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+    {
+      const uint4* p = reinterpret_cast<const uint4*>(&rows[(r0 + col) * kSigRow + 8 * half]);
+      const uint4 u = p[0], w = p[1];
+      const uint32_t q[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const i32x4_t a = bits_to_fp4(q[k]);
+        acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
+            __builtin_shufflevector(a, a, 0, 1, 2, 3, -1, -1, -1, -1),
+            __builtin_shufflevector(qf[k], qf[k], 0, 1, 2, 3, -1, -1, -1, -1), acc, 4, 4, 0, 0, 0, 0);
+      }
+    }
+    // rows of the tile that this column may take: within W of it, not itself,
+    // not listed already
+    const int c = col - 32 * t;                  // row of the window's start, relative to the tile
+    const int e = c + 2 * (int)W;                // and of its end
+    uint32_t ok = 0;
+    if (x != kNone && e >= 0 && c < 32)
+      ok = (c > 0 ? 0xFFFFFFFFu << c : 0xFFFFFFFFu) & (e < 31 ? 0xFFFFFFFFu >> (31 - e) : 0xFFFFFFFFu);
+    const int self = c + (int)W;
+    if (self >= 0 && self < 32) ok &= ~(1u << self);
+    if (!first) ok &= ~dup[base + col][t];
+    const uint32_t bad = ~ok >> (4 * half);      // bit 8 (v/4) + v%4: accumulator element v is out
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const uint4 id4 = *reinterpret_cast<const uint4*>(&ids[r0 + 8 * g + 4 * half]);
+      const uint32_t id[4] = {id4.x, id4.y, id4.z, id4.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t d = (uint32_t)(1073741824.f - 2097152.f * acc[4 * g + i]);   // Hamming << 22
+        const uint32_t out = (uint32_t)((int)(bad << (31 - (8 * g + i))) >> 31);
+        const uint32_t key = d | id[i] | out;    // an absent row's id is all ones
+        if (!__any(key < b[kList - 1])) continue;
+#pragma unroll
+        for (int q = kList - 1; q > 0; --q) b[q] = med3(b[q - 1], key, b[q]);
+        b[0] = min(b[0], key);
+      }
+    }
+  }
+  // the 16 smallest of the two halves' lists (a bitonic sequence), sorted
+  uint32_t m[kList];
+#pragma unroll
+  for (int t = 0; t < kList; ++t) m[t] = min(b[t], (uint32_t)__shfl_xor(b[kList - 1 - t], 32, 64));
+#pragma unroll
+  for (int o = kList / 2; o >= 1; o >>= 1)
+#pragma unroll
+    for (int t = 0; t < kList; ++t)
+      if (!(t & o)) {
+        const uint32_t u = min(m[t], m[t + o]), w = max(m[t], m[t + o]);
+        m[t] = u;
+        m[t + o] = w;
+      }
+  if (half == 0 && x != kNone) {
+    uint4* p = reinterpret_cast<uint4*>(best + (uint64_t)x * kList);
+#pragma unroll
+    for (int t = 0; t < kList / 4; ++t) p[t] = make_uint4(m[4 * t], m[4 * t + 1], m[4 * t + 2], m[4 * t + 3]);
+  }
+}
+
+// The lists' first k nodes.
+__global__ void k_window_ids(const uint32_t* __restrict__ best, uint64_t n, uint32_t k, uint32_t* __restrict__ out) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n * k) return;
+  const uint32_t key = best[e / k * kList + e % k];
+  out[e] = key == kNone ? kNone : key & kIdMask;
 }
 
 // Block = 256 consecutive sorted positions; the window's rows are staged in
@@ -236,27 +433,49 @@ void knn_lsh(svd_ctx* c, const float* emb, uint64_t n, uint32_t k, uint32_t tabl
   }
   float* dh = dalloc<float>(c, h.size());
   SVD_HIP(hipMemcpyAsync(dh, h.data(), h.size() * 4, hipMemcpyHostToDevice, c->stream));
-  uint32_t* keys = dalloc<uint32_t>(c, n);
-  uint32_t* keys2 = dalloc<uint32_t>(c, n);
-  uint32_t* vals = dalloc<uint32_t>(c, n);
-  uint32_t* order = dalloc<uint32_t>(c, n);
-  float* bd = dalloc<float>(c, n * k);
-  size_t bytes = 0;
-  SVD_HIP(rocprim::radix_sort_pairs(nullptr, bytes, keys, keys2, vals, order, (size_t)n, 0, bits, c->stream));
+  // orderings are sorted several at a time, up to 2^22 keys (table << bits | key)
+  const uint32_t group = (uint32_t)std::min<uint64_t>(std::min<uint64_t>(tables, 1ull << (32 - bits)),
+                                                      std::max<uint64_t>(1, (1ull << 22) / n));
+  uint32_t gbits = bits;
+  while ((group - 1) >> (gbits - bits)) ++gbits;
+  uint32_t* keys = dalloc<uint32_t>(c, n * group);
+  uint32_t* keys2 = dalloc<uint32_t>(c, n * group);
+  uint32_t* vals = dalloc<uint32_t>(c, n * group);
+  uint32_t* orders = dalloc<uint32_t>(c, n * group);
+  // the matrix-core windows need (distance, node) in 32 bits
+  const bool mm = sig && k <= (uint32_t)kList && n <= (1ull << kIdBits);
+  float* bd = mm ? nullptr : dalloc<float>(c, n * k);
+  uint32_t* best = mm ? dalloc<uint32_t>(c, n * kList) : nullptr;
+  size_t bytes = 0, last = 0;
+  SVD_HIP(rocprim::radix_sort_pairs(nullptr, bytes, keys, keys2, vals, orders, (size_t)(n * group), 0, gbits, c->stream));
+  if (tables % group)
+    SVD_HIP(rocprim::radix_sort_pairs(nullptr, last, keys, keys2, vals, orders, (size_t)(n * (tables % group)), 0, gbits,
+                                      c->stream));
+  bytes = std::max(bytes, last);
   void* tmp = c->arena->get(bytes + 16);
   const size_t lds = (size_t)(kTile + 2 * window) * (sig ? 17 : kRow) * sizeof(float);
   for (uint32_t t = 0; t < tables; ++t) {
-    k_lsh_keys<<<div_up(n, 256), 256, 0, c->stream>>>(emb, n, dh + (size_t)t * bits * kDim, bits, keys, vals);
-    SVD_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, vals, order, (size_t)n, 0, bits, c->stream));
+    const uint32_t inGroup = t % group;
+    if (inGroup == 0) {
+      const uint32_t m = std::min(group, tables - t);
+      k_lsh_keys<<<div_up(n, 256), 256, 0, c->stream>>>(emb, n, dh + (size_t)t * bits * kDim, bits, m, keys, vals);
+      SVD_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, vals, orders, (size_t)(n * m), 0, gbits, c->stream));
+    }
+    const uint32_t* order = orders + (uint64_t)inGroup * n;
     const dim3 g(div_up(n, kTile));
-    if (sig && k == 16) k_window_topk<1, 16><<<g, kTile, lds, c->stream>>>(emb, sig, order, n, window, k, t == 0, bd, out);
+    if (mm) k_window_keys<<<div_up(n, kQ), 256, 0, c->stream>>>(sig, order, (uint32_t)n, window, t == 0, best);
+    else if (sig && k == 16) k_window_topk<1, 16><<<g, kTile, lds, c->stream>>>(emb, sig, order, n, window, k, t == 0, bd, out);
     else if (sig) k_window_topk<1, kMaxK><<<g, kTile, lds, c->stream>>>(emb, sig, order, n, window, k, t == 0, bd, out);
     else if (k == 16) k_window_topk<0, 16><<<g, kTile, lds, c->stream>>>(emb, sig, order, n, window, k, t == 0, bd, out);
     else k_window_topk<0, kMaxK><<<g, kTile, lds, c->stream>>>(emb, sig, order, n, window, k, t == 0, bd, out);
     check_launch("knn table");
   }
+  if (mm) {
+    k_window_ids<<<div_up(n * k, 256), 256, 0, c->stream>>>(best, n, k, out);
+    check_launch("k_window_ids");
+  }
   c->arena->put(tmp);
-  dfree(c, dh); dfree(c, keys); dfree(c, keys2); dfree(c, vals); dfree(c, order); dfree(c, bd);
+  dfree(c, dh); dfree(c, keys); dfree(c, keys2); dfree(c, vals); dfree(c, orders); dfree(c, bd); dfree(c, best);
 }
 
 }  // namespace svd

@@ -281,6 +281,27 @@ def test_knn_matches_oracle(ctx):
                                   O.knn_lsh(e, 16, 4, 12, 48, 9, sig=sig))
 
 
+@pytest.mark.parametrize("n,k,tables,bits,window", [(1, 16, 2, 4, 64), (31, 16, 2, 4, 3), (33, 1, 3, 4, 1),
+                                                    (128, 16, 2, 3, 96), (129, 7, 2, 3, 95), (300, 16, 9, 5, 63),
+                                                    (1000, 15, 3, 24, 96), (1000, 17, 2, 6, 40)])
+def test_knn_signature_windows(ctx, n, k, tables, bits, window):
+    """The matrix-core windows at their edges: fewer points than a workgroup,
+    one or a partial query tile, windows of 1 to 96 positions (partial row
+    tiles), several tables over the same neighbours (candidates the list
+    already holds), many equal distances and equal signatures, and k = 17
+    (the general kernel)."""
+    rng = np.random.default_rng(n + k)
+    sig = _rand_sigs(max(n // 3, 1), 11 + n, density=0.02)[rng.integers(0, max(n // 3, 1), n)]
+    e = rng.standard_normal((n, 32)).astype(np.float32)
+    de, dsig = torch.from_numpy(e).to(DEV), _dev_u32(sig)
+    out = torch.zeros(n * k, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+    ctx.knn(de.data_ptr(), n, k, tables, bits, window, 9, out.data_ptr(), sig_ptr=dsig.data_ptr())
+    ctx.sync()
+    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32).reshape(n, k),
+                                  O.knn_lsh(e, k, tables, bits, window, 9, sig=sig))
+
+
 def test_knn_full_window_is_brute_force(ctx):
     rng = np.random.default_rng(5)
     n = 90                               # every point within +-96 positions of every other
