@@ -6,6 +6,7 @@
 // min/max follow the GLSL definitions: min(x,y) = y<x ? y : x.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include "svd_internal.hpp"
 
 namespace svd {
@@ -67,6 +68,20 @@ __device__ __forceinline__ Stack make_stack(uint32_t* mem, int depth, int lane) 
   return Stack{mem, mem + depth * kBT, kStackWords<FMT> == 3 ? mem + 2 * depth * kBT : nullptr, lane, 0};
 }
 
+// An SSVDAG's level offsets in LDS behind the stacks: every fetch adds its
+// level's, and a read from memory would stand in front of each of them.  All
+// threads of the workgroup call it before any leaves.
+template <int FMT>
+__device__ __forceinline__ const uint32_t* stage_offsets(const Dev& s, uint32_t* mem) {
+  uint32_t* l = mem + kStackWords<FMT> * (s.innerLevels + 1) * kBT;
+  if (FMT == SVD_FMT_SSVDAG) {
+    const int t = threadIdx.y * blockDim.x + threadIdx.x;
+    if (t < s.innerLevels) l[t] = s.levelOffsets[t];
+    __syncthreads();
+  }
+  return l;
+}
+
 // INSTR: keep the per-ray descent-path hash and the fetched-byte count (the
 // test and byte-count variant); without it the two stay at their initial
 // values and cost no instructions.
@@ -74,11 +89,13 @@ template <int FMT, bool INSTR = true>
 struct Tracer {
   const Dev& s;
   Stack st;
+  const uint32_t* lofs;   // level offsets (LDS)
   uint32_t path;
   uint32_t bytes;
   bool bad;   // a fetch fell outside the scene arrays (malformed file)
 
-  __device__ Tracer(const Dev& d, Stack k) : s(d), st(k), path(2166136261u), bytes(0), bad(false) {}
+  __device__ Tracer(const Dev& d, Stack k, const uint32_t* offsets)
+      : s(d), st(k), lofs(offsets), path(2166136261u), bytes(0), bad(false) {}
 
   __device__ __forceinline__ uint32_t word(uint32_t i) {
     if (i < s.nWords) return s.nodes[i];
@@ -135,7 +152,7 @@ struct Tracer {
     // the two in scratch memory
     uint32_t lo, hi = ts.leaf_hi;
     if ((int)ts.level < s.innerLevels) {
-      lo = half((uint32_t)(ts.node_index + (int)s.levelOffsets[ts.level]));
+      lo = half((uint32_t)(ts.node_index + (int)lofs[ts.level]));
       if (INSTR) bytes += 2;
     } else {
       uint2 v = make_uint2(0u, 0u);
@@ -163,17 +180,17 @@ struct Tracer {
     // plus one more per code with its high bit set
     const uint32_t lo = ts.hdr & 0x5555u, hi = (ts.hdr >> 1) & 0x5555u;
     const uint32_t above = 0xFFFFu & ~((2u << (2 * ts.cli + 1)) - 1u);   // fields cli+1 .. 7
-    int off = 1 + (int)s.levelOffsets[ts.level] + ts.node_index +
-              __popc((lo | hi) & above) + __popc(hi & above);
+    const uint32_t off = (uint32_t)(1 + (int)lofs[ts.level] + ts.node_index +
+                                    __popc((lo | hi) & above) + __popc(hi & above));
     const int cm = (int)((ts.hdr >> (ts.cli << 1)) & 3u);
-    int cx = (int)half((uint32_t)off);
-    if (INSTR) bytes += 2;
-    const uint32_t mf = ((uint32_t)cx >> 13) & 7u;
-    cx &= -57345;
+    // both words of a pointer at once; a one-word pointer reads its own twice
+    const uint32_t off2 = off + (cm > 1 ? 1u : 0u);
+    const uint32_t w0 = half(off), w1 = half(off2);
+    if (INSTR) bytes += cm > 1 ? 4 : 2;
+    const uint32_t mf = (w0 >> 13) & 7u;
+    int cx = (int)(w0 & ~0xE000u);
     if (cm > 1) {
-      const int cy = (int)half((uint32_t)off + 1);
-      if (INSTR) bytes += 2;
-      cx = (cx << 16) | cy;
+      cx = (cx << 16) | (int)w1;
       cx |= (cm & 1) << 29;
     }
     ts.mm ^= mf;
@@ -208,7 +225,8 @@ struct Tracer {
   __device__ __forceinline__ static bool in_bounds(const int li[3], int sz) {
     return (uint32_t)li[0] < (uint32_t)sz && (uint32_t)li[1] < (uint32_t)sz && (uint32_t)li[2] < (uint32_t)sz;
   }
-  __device__ __forceinline__ void up_in(const float o[3], TS& ts) {
+  // Up to the pushed node; settle() follows, as after down_in.
+  __device__ __forceinline__ void up_in(TS& ts) {
     uint32_t dl = ts.level;
     pop(ts);
     dl -= ts.level;
@@ -216,9 +234,6 @@ struct Tracer {
     for (int a = 0; a < 3; ++a) ts.idx[a] >>= dl;
     ts.cell *= (float)(1 << dl);
     ts.cns = (int)ts.level < s.innerLevels ? 2 : s.leafSize;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & 1;
-    next_crossing(ts, o);
   }
   // The position step of go_down_one_level (octree_dda.frag.glsl:434-451).
   // Its next-crossing and local-index updates read nothing this step reads,
@@ -245,13 +260,18 @@ struct Tracer {
       int vc = s.leafSize / 2;
       while (vc > 1) { step_down(o, d, ts); vc >>= 1; }
     }
-    next_crossing(ts, o);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & (ts.cns - 1);
     if (INSTR) {
       path = (path ^ (uint32_t)ts.node_index) * 16777619u;
       path = (path ^ ts.level) * 16777619u;
     }
+  }
+  // The next crossings and the local index in a node just entered: the same
+  // for a step up (into a node of side 2) and a step down, so a wavefront whose
+  // lanes do both runs it once.
+  __device__ __forceinline__ static void settle(TS& ts, const float o[3]) {
+    next_crossing(ts, o);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & (ts.cns - 1);
   }
 
   // Per-ray state between iterations of the traversal loop.
@@ -342,12 +362,14 @@ struct Tracer {
 #pragma unroll
     for (int a = 0; a < 3; ++a) { delta[a] = m[a] ? ts.di[a] : 0; nl[a] = ts.li[a] + delta[a]; }
     const bool next_in_node = in_bounds(nl, ts.cns);
+    bool entered = full;
     if (!full) {
       r.stepm = (uint32_t)(m[0] | (m[1] << 1) | (m[2] << 2));
       dda_next(ts, m, delta);
       if (!next_in_node) {
         if (st.size == 0) { out[0] = -1.f; out[1] = 0.f; out[2] = (float)r.it; out[3] = -1.f; return true; }
-        up_in(r.o, ts);
+        up_in(ts);
+        entered = true;
       }
     } else {
       const bool hit = (ts.level >= r.maxLevel) || ((ts.cell * r.projf) < ts.t_current);
@@ -359,6 +381,7 @@ struct Tracer {
       down_in(r.o, r.d, ts, next_in_node);
       fetch_data(ts);
     }
+    if (entered) settle(ts, r.o);
     ts.cli = lin_idx(ts, ts.cns);
     ++r.it;
     if ((ts.t_current < r.tmax) && ((uint32_t)r.it < r.maxIters)) return false;
@@ -483,14 +506,15 @@ __device__ __forceinline__ float min_t(const MinDepth& md, uint32_t px, uint32_t
 // shadow ray is cast.
 template <int FMT, bool INSTR = true>
 __device__ __forceinline__ void trace_pixel(const Dev& s, const svd_trace_params& p, uint32_t px, uint32_t py,
-                                            uint32_t* stackMem, svd_ray_result* __restrict__ prim,
+                                            uint32_t* stackMem, const uint32_t* lofs,
+                                            svd_ray_result* __restrict__ prim,
                                             svd_ray_result* __restrict__ shad, MinDepth md = MinDepth{nullptr, 0, 0},
                                             float4* __restrict__ primHit = nullptr,
                                             float4* __restrict__ shadHit = nullptr) {
   const int depth = s.innerLevels + 1;
   const int lane = threadIdx.y * blockDim.x + threadIdx.x;
   Stack stk = make_stack<FMT>(stackMem, depth, lane);
-  Tracer<FMT, INSTR> tr(s, stk);
+  Tracer<FMT, INSTR> tr(s, stk, lofs);
   float o[3], d[3];
   camera_ray(p, px, py, (float)p.width, (float)p.height, o, d);
   float res[4];
@@ -591,12 +615,12 @@ struct ViewArgs {
 // intensity, the normal samples of the pretty mode, the highlight / frequency /
 // random colouring and the shadow ray.  rgb gets the colour the fragment
 // writes; a fragment the shader discards gets 0.
-template <int FMT>
+template <int FMT, bool INSTR>
 __device__ __forceinline__ void render_pixel(const Dev& s, const svd_trace_params& p, const ViewArgs& va,
-                                             uint32_t px, uint32_t py, uint32_t* stackMem, float* __restrict__ rgb,
-                                             svd_ray_result* __restrict__ prim, MinDepth md) {
+                                             uint32_t px, uint32_t py, uint32_t* stackMem, const uint32_t* lofs,
+                                             float* __restrict__ rgb, svd_ray_result* __restrict__ prim, MinDepth md) {
   const int lane = threadIdx.y * blockDim.x + threadIdx.x;
-  Tracer<FMT> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane));
+  Tracer<FMT, INSTR> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane), lofs);
   const float sw = (float)p.width, sh = (float)p.height;
   const float scx = screen_coord(px, sw), scy = screen_coord(py, sh);
   float o[3], d[3];
@@ -607,7 +631,7 @@ __device__ __forceinline__ void render_pixel(const Dev& s, const svd_trace_param
   tr.trace(o, d, tmin, 1e30f, p.projection_factor, p.max_iters, p.draw_level, res, step);
   if (tr.bad) { res[0] = -6.f; res[1] = 0.f; res[3] = -1.f; }
   const size_t k = (size_t)py * p.width + px;
-  if (prim) prim[k] = svd_ray_result{res[0], res[1], res[2], res[3], tr.path, tr.bytes};
+  if (INSTR) prim[k] = svd_ray_result{res[0], res[1], res[2], res[3], tr.path, tr.bytes};
   float col[3];
   if (res[0] >= 0.f) {
     const float hit[3] = {o[0] + res[0] * d[0], o[1] + res[0] * d[1], o[2] + res[0] * d[2]};
@@ -725,13 +749,12 @@ struct AOEntry {
   uint32_t pixel;
 };
 
-template <int FMT>
-__device__ __forceinline__ void ao_gbuffer(const Dev& s, const svd_trace_params& p, uint32_t px, uint32_t py,
-                                           uint32_t* stackMem, float* __restrict__ vis, uint32_t* __restrict__ cnt,
-                                           AOEntry* __restrict__ entries, uint32_t* __restrict__ nEntries,
-                                           svd_ray_result* __restrict__ prim) {
+template <int FMT, bool INSTR>
+__device__ __forceinline__ bool ao_gbuffer(const Dev& s, const svd_trace_params& p, uint32_t px, uint32_t py,
+                                           uint32_t* stackMem, const uint32_t* lofs, float* __restrict__ vis,
+                                           uint32_t* __restrict__ cnt, svd_ray_result* __restrict__ prim, AOEntry& e) {
   const int lane = threadIdx.y * blockDim.x + threadIdx.x;
-  Tracer<FMT> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane));
+  Tracer<FMT, INSTR> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane), lofs);
   float o[3], d[3];
   camera_ray(p, px, py, (float)p.width, (float)p.height, o, d);
   float res[4];
@@ -739,17 +762,16 @@ __device__ __forceinline__ void ao_gbuffer(const Dev& s, const svd_trace_params&
   tr.trace(o, d, 0.0f, 1e30f, p.projection_factor, p.max_iters, p.draw_level, res, step);
   if (tr.bad) { res[0] = -6.f; res[1] = 0.f; res[3] = -1.f; }
   const size_t k = (size_t)py * p.width + px;
-  if (prim) prim[k] = svd_ray_result{res[0], res[1], res[2], res[3], tr.path, tr.bytes};
+  if (INSTR) prim[k] = svd_ray_result{res[0], res[1], res[2], res[3], tr.path, tr.bytes};
   float hit[3] = {0.f, 0.f, 0.f};
   if (res[0] >= 0.f) {
     hit[0] = o[0] + res[0] * d[0];
     hit[1] = o[1] + res[0] * d[1];
     hit[2] = o[2] + res[0] * d[2];
   }
-  if (hit[0] == 0.f && hit[1] == 0.f && hit[2] == 0.f) { vis[k] = -1.0f; return; }
+  if (hit[0] == 0.f && hit[1] == 0.f && hit[2] == 0.f) { vis[k] = -1.0f; return false; }
   const float hn[3] = {-(float)step[0], -(float)step[1], -(float)step[2]};
   const float cellSize = (2.0f * s.rootHalfSide) / ldexpf(1.0f, (int)res[1]);
-  AOEntry e;
   e.hit[0] = hit[0] + hn[0] * 1e-3f;
   e.hit[1] = hit[1] + hn[1] * 1e-3f;
   e.hit[2] = hit[2] + hn[2] * 1e-3f;
@@ -762,7 +784,7 @@ __device__ __forceinline__ void ao_gbuffer(const Dev& s, const svd_trace_params&
   e.pixel = (uint32_t)k;
   vis[k] = 0.0f;
   cnt[k] = 0u;
-  entries[atomicAdd(nEntries, 1u)] = e;
+  return true;
 }
 
 // Persistent form: lanes that finished their rays take new ones from a
@@ -791,7 +813,7 @@ k_trace_persist(Dev s, svd_trace_params p, svd_ray_result* __restrict__ prim, sv
   const int depth = s.innerLevels + 1;
   const uint32_t lane = threadIdx.x & 63u;
   Stack stk = make_stack<FMT>(stackMem, depth, (int)threadIdx.x);
-  Tracer<FMT> tr(s, stk);
+  Tracer<FMT> tr(s, stk, stage_offsets<FMT>(s, stackMem));
   typename Tracer<FMT>::Ray ray;
   const uint32_t th = kBT / tw;
   uint32_t state = kIdle, px = 0, py = 0;
@@ -897,8 +919,9 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_trace(Dev s, svd_trace_pa
   extern __shared__ uint32_t stackMem[];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
   if (px >= p.width || py >= p.height) return;
-  trace_pixel<FMT>(s, p, px, py, stackMem, prim, shad, md);
+  trace_pixel<FMT>(s, p, px, py, stackMem, lofs, prim, shad, md);
 }
 
 // The same frame without instrumentation: traceRay's vec4 per ray (16 bytes),
@@ -909,8 +932,9 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_trace_hits(Dev s, svd_tra
   extern __shared__ uint32_t stackMem[];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
   if (px >= p.width || py >= p.height) return;
-  trace_pixel<FMT, false>(s, p, px, py, stackMem, nullptr, nullptr, md, prim, shad);
+  trace_pixel<FMT, false>(s, p, px, py, stackMem, lofs, nullptr, nullptr, md, prim, shad);
 }
 
 // DEPTH_MODE pre-pass (octree_dda.frag.glsl:862-872) over the (w x h)
@@ -923,9 +947,10 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_trace_depth(Dev s, svd_tr
   extern __shared__ uint32_t stackMem[];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
   if (px >= w || py >= h) return;
   const int lane = threadIdx.y * blockDim.x + threadIdx.x;
-  Tracer<FMT, false> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane));
+  Tracer<FMT, false> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, lane), lofs);
   float o[3], d[3];
   camera_ray(p, px, py, sw, sh, o, d);
   float res[4];
@@ -946,24 +971,27 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_trace_batch(const Dev* __
   const svd_trace_params p = cams[cam];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
-  if (px >= p.width || py >= p.height) return;
   const Dev s = scenes[camScene[cam]];
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
+  if (px >= p.width || py >= p.height) return;
   const size_t off = (size_t)cam * p.width * p.height;
-  trace_pixel<FMT>(s, p, px, py, stackMem, prim + off, shad ? shad + off : nullptr);
+  trace_pixel<FMT>(s, p, px, py, stackMem, lofs, prim + off, shad ? shad + off : nullptr);
 }
 
-template <int FMT>
+// prim (primary records with path and bytes) only with INSTR, here and below.
+template <int FMT, bool INSTR>
 __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_render(Dev s, svd_trace_params p, ViewArgs va,
                                                                 float* __restrict__ rgb,
                                                                 svd_ray_result* __restrict__ prim, MinDepth md) {
   extern __shared__ uint32_t stackMem[];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
   if (px >= p.width || py >= p.height) return;
-  render_pixel<FMT>(s, p, va, px, py, stackMem, rgb, prim, md);
+  render_pixel<FMT, INSTR>(s, p, va, px, py, stackMem, lofs, rgb, prim, md);
 }
 
-template <int FMT>
+template <int FMT, bool INSTR>
 __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_gbuffer(Dev s, svd_trace_params p, float* __restrict__ vis,
                                                                     uint32_t* __restrict__ cnt,
                                                                     AOEntry* __restrict__ entries,
@@ -972,8 +1000,23 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_gbuffer(Dev s, svd_tra
   extern __shared__ uint32_t stackMem[];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
-  if (px >= p.width || py >= p.height) return;
-  ao_gbuffer<FMT>(s, p, px, py, stackMem, vis, cnt, entries, nEntries, prim);
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
+  AOEntry e;
+  const bool has = px < p.width && py < p.height && ao_gbuffer<FMT, INSTR>(s, p, px, py, stackMem, lofs, vis, cnt, prim, e);
+  // one atomic per workgroup: from every wavefront of a 1080p frame they took
+  // a good part of the pass at that one address
+  __shared__ uint32_t waveN[kBT / 64], wgBase;
+  const int tid = threadIdx.y * blockDim.x + threadIdx.x, wave = tid >> 6;
+  const uint64_t b = __ballot(has);
+  if ((tid & 63) == 0) waveN[wave] = (uint32_t)__popcll(b);
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t n = 0;
+    for (int w = 0; w < kBT / 64; ++w) { const uint32_t x = waveN[w]; waveN[w] = n; n += x; }
+    wgBase = n ? atomicAdd(nEntries, n) : 0u;
+  }
+  __syncthreads();
+  if (has) entries[wgBase + waveN[wave] + (uint32_t)__popcll(b & ((1ull << (tid & 63)) - 1ull))] = e;
 }
 
 // Grid-stride over the (entry, ray) pairs; consecutive lanes take the rays
@@ -984,7 +1027,7 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_rays(Dev s, svd_trace_
                                                                  const uint32_t* __restrict__ nEntries,
                                                                  uint32_t* __restrict__ cnt) {
   extern __shared__ uint32_t stackMem[];
-  Tracer<FMT> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, threadIdx.x));
+  Tracer<FMT, false> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, threadIdx.x), stage_offsets<FMT>(s, stackMem));
   const uint64_t total = (uint64_t)(*nEntries) * nrays;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < total; w += stride) {
@@ -1051,10 +1094,10 @@ Dev scene_dev(const svd_scene* sc) {
 
 namespace {
 
-// LDS of one workgroup: the descent stacks of its kBT lanes
+// LDS of one workgroup: the descent stacks of its kBT lanes, the level offsets
 size_t stack_bytes(const svd_scene* sc, const Dev& d) {
-  return (size_t)(sc->fmt == SVD_FMT_USSVDAG ? kStackWords<SVD_FMT_USSVDAG> : 2) * (d.innerLevels + 1) * kBT *
-         sizeof(uint32_t);
+  return ((size_t)(sc->fmt == SVD_FMT_USSVDAG ? kStackWords<SVD_FMT_USSVDAG> : 2) * (d.innerLevels + 1) * kBT +
+          kMaxLevels) * sizeof(uint32_t);
 }
 
 // The DEPTH_MODE pre-pass into `depth` ((width/8) x (height/8) floats).  The
@@ -1237,12 +1280,14 @@ void render_frame(svd_scene* sc, const svd_trace_params* p, const svd_view_param
     depth = depthBuf ? depthBuf : dalloc<float>(c, (uint64_t)(p->width / 8) * (p->height / 8) + 1);
     md = depth_prepass(sc, d, p, beamProjf, depth);
   }
+  auto render = [&](auto fmt) {
+    if (prim) k_render<fmt(), true><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md);
+    else k_render<fmt(), false><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, nullptr, md);
+  };
   switch (sc->fmt) {
-    case SVD_FMT_SVDAG: k_render<SVD_FMT_SVDAG><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md); break;
-    case SVD_FMT_USSVDAG:
-      k_render<SVD_FMT_USSVDAG><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md);
-      break;
-    default: k_render<SVD_FMT_SSVDAG><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md); break;
+    case SVD_FMT_SVDAG: render(std::integral_constant<int, SVD_FMT_SVDAG>()); break;
+    case SVD_FMT_USSVDAG: render(std::integral_constant<int, SVD_FMT_USSVDAG>()); break;
+    default: render(std::integral_constant<int, SVD_FMT_SSVDAG>()); break;
   }
   check_launch("k_render");
   if (depth != depthBuf) dfree(c, depth);
@@ -1326,21 +1371,15 @@ void ao_frame(svd_scene* sc, const svd_trace_params* p, uint32_t nrays, float* v
   const size_t shmem = stack_bytes(sc, d);
   // as many workgroups as run at once at six wavefronts per SIMD
   const uint32_t rayBlocks = (uint32_t)std::max(1, c->numCU > 0 ? c->numCU : 256) * 6u;
+  auto ao = [&](auto fmt) {
+    if (prim) k_ao_gbuffer<fmt(), true><<<grid, block, shmem, c->stream>>>(d, *p, vis, cnt, entries, nEntries, prim);
+    else k_ao_gbuffer<fmt(), false><<<grid, block, shmem, c->stream>>>(d, *p, vis, cnt, entries, nEntries, nullptr);
+    if (nrays) k_ao_rays<fmt()><<<rayBlocks, kBT, shmem, c->stream>>>(d, *p, dhs, nrays, entries, nEntries, cnt);
+  };
   switch (sc->fmt) {
-    case SVD_FMT_SVDAG:
-      k_ao_gbuffer<SVD_FMT_SVDAG><<<grid, block, shmem, c->stream>>>(d, *p, vis, cnt, entries, nEntries, prim);
-      if (nrays) k_ao_rays<SVD_FMT_SVDAG><<<rayBlocks, kBT, shmem, c->stream>>>(d, *p, dhs, nrays, entries, nEntries, cnt);
-      break;
-    case SVD_FMT_USSVDAG:
-      k_ao_gbuffer<SVD_FMT_USSVDAG><<<grid, block, shmem, c->stream>>>(d, *p, vis, cnt, entries, nEntries, prim);
-      if (nrays)
-        k_ao_rays<SVD_FMT_USSVDAG><<<rayBlocks, kBT, shmem, c->stream>>>(d, *p, dhs, nrays, entries, nEntries, cnt);
-      break;
-    default:
-      k_ao_gbuffer<SVD_FMT_SSVDAG><<<grid, block, shmem, c->stream>>>(d, *p, vis, cnt, entries, nEntries, prim);
-      if (nrays)
-        k_ao_rays<SVD_FMT_SSVDAG><<<rayBlocks, kBT, shmem, c->stream>>>(d, *p, dhs, nrays, entries, nEntries, cnt);
-      break;
+    case SVD_FMT_SVDAG: ao(std::integral_constant<int, SVD_FMT_SVDAG>()); break;
+    case SVD_FMT_USSVDAG: ao(std::integral_constant<int, SVD_FMT_USSVDAG>()); break;
+    default: ao(std::integral_constant<int, SVD_FMT_SSVDAG>()); break;
   }
   k_ao_finish<<<div_up(npix, 256), 256, 0, c->stream>>>(vis, cnt, npix, nrays);
   check_launch("ao passes");
