@@ -278,12 +278,16 @@ class Context:
         else:
             a = np.ascontiguousarray(attrs, dtype=np.uint8)
             src, n, on_dev = a.ctypes.data_as(C.c_void_p), a.size, 0
+        # one call into a buffer no blob exceeds: a plane's tree has at most n - 1
+        # mixed nodes and as many uniform parts plus one, 2 n bits in all, and up
+        # to three per level of the padding
         size = C.c_uint64()
-        self.check(self.L.svd_attr_bittree_encode(self.h, src, n, int(gray), on_dev, None, 0, C.byref(size)))
-        buf = np.zeros(size.value, np.uint8)
+        buf = np.empty(48 + 8 * 4 * ((2 * n + 3 * 64 + 31) // 32), np.uint8)
         self.check(self.L.svd_attr_bittree_encode(self.h, src, n, int(gray), on_dev, buf.ctypes.data_as(C.c_void_p),
-                                                  size.value, C.byref(size)))
-        return buf.tobytes()
+                                                  buf.size, C.byref(size)))
+        if size.value > buf.size:
+            raise SvdError(OK, "bit-tree larger than its bound")
+        return buf[:size.value].tobytes()
 
     def knn(self, emb_ptr: int, n: int, k: int = 16, tables: int = 4, bits: int = 16, window: int = 32,
             seed: int = 7, out_ptr: int = 0, sig_ptr: int = 0):

@@ -215,6 +215,13 @@ __global__ void __launch_bounds__(kBT) k_bt_count(const uint8_t* __restrict__ a,
   }
 }
 
+// 3. one scan runs over the counts of all planes (plane-major; a plane has
+// fewer than 2^32 bits, so differences within it are exact): bits per plane
+__global__ void k_bt_bits(const uint32_t* __restrict__ offs, uint32_t nb, uint32_t* __restrict__ bits) {
+  const uint32_t k = threadIdx.x;   // bits[8]: the scan's total
+  if (k < 8) bits[k] = (k < 7 ? offs[(uint64_t)(k + 1) * nb] : bits[8]) - offs[(uint64_t)k * nb];
+}
+
 struct PlaneWords { uint64_t w[8]; };
 
 // 4. emit at pre-order offsets
@@ -238,7 +245,7 @@ __global__ void __launch_bounds__(kBT) k_bt_emit(const uint8_t* __restrict__ a, 
   }
   if (lane >= 56) s[w][lane - 56] = x;   // wave totals per plane
   __syncthreads();
-  uint32_t pos = offs[(uint64_t)k * g.nb + blockIdx.x] + x - cn.n;
+  uint32_t pos = offs[(uint64_t)k * g.nb + blockIdx.x] - offs[(uint64_t)k * g.nb] + x - cn.n;
   for (uint32_t v = 0; v < w; ++v) pos += s[v][k];
   if (j < g.C && cn.n) {
     Writer wr{words + pw.w[k], pos, pos >> 5, 0u};
@@ -267,7 +274,7 @@ uint64_t attr_bittree(svd_ctx* c, const uint8_t* dattrs, uint64_t V, int gray, u
   uint32_t bits[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   uint16_t* pyr = nullptr;
   uint32_t* sums = nullptr;
-  uint32_t* total = dalloc<uint32_t>(c, 8);
+  uint32_t* total = dalloc<uint32_t>(c, 9);
   if (V) {
     pyr = dalloc<uint16_t>(c, at + 1);
     sums = dalloc<uint32_t>(c, 8ull * g.nb + 1);
@@ -282,7 +289,9 @@ uint64_t attr_bittree(svd_ctx* c, const uint8_t* dattrs, uint64_t V, int gray, u
     }
     k_bt_count<<<g.nb, kBT, 0, c->stream>>>(dattrs, g, pyr, sums);
     check_launch("k_bt_count");
-    for (int k = 0; k < 8; ++k) scan_exclusive(c, sums + (uint64_t)k * g.nb, sums + (uint64_t)k * g.nb, g.nb, total + k);
+    scan_exclusive(c, sums, sums, 8ull * g.nb, total + 8);
+    k_bt_bits<<<1, 8, 0, c->stream>>>(sums, g.nb, total);
+    check_launch("k_bt_bits");
     read_u32s(c, total, bits, 8);
   }
   uint64_t nwords = 0;

@@ -23,6 +23,10 @@
 // node, the smallest matching frontier index and then the largest path
 // (path * 8 + slot), and the winning parent writes B's descendant on the same
 // path.  No subtree is walked per thread.
+//
+// The state of all levels lies in flat arrays (level l from base[l] on), so a
+// step over several levels is one launch: a merge is bound by its launches
+// and read-backs (2.8 us per launch at 200K nodes), not by its work.
 #include "svd_internal.hpp"
 
 namespace svd {
@@ -35,8 +39,17 @@ constexpr uint32_t kMaxL = 21;
 struct LevelPtrs {
   const uint32_t* rec[kMaxL];   // 9-word records (leaf level: 1 word)
   uint32_t n[kMaxL];
+  uint64_t base[kMaxL + 1];     // flat index of a level's first node
   uint32_t leafLevel;
 };
+
+// Level and node of a flat index between levels lo and hi.
+__device__ __forceinline__ uint32_t level_of(const LevelPtrs& P, uint64_t e, uint32_t lo, uint32_t hi, uint32_t& i) {
+  uint32_t l = lo;
+  while (l < hi && e >= P.base[l + 1]) ++l;
+  i = (uint32_t)(e - P.base[l]);
+  return l;
+}
 
 __device__ __forceinline__ uint32_t node_mask(const LevelPtrs& P, uint32_t lev, uint32_t i) {
   return lev == P.leafLevel ? (P.rec[lev][i] & 0xFFu) : (P.rec[lev][(uint64_t)i * kRecWords] & 0xFFu);
@@ -46,21 +59,25 @@ __device__ __forceinline__ uint32_t node_child(const LevelPtrs& P, uint32_t lev,
 }
 
 // ---- truncated-subtree classes ---------------------------------------------
-// keys of level lev for depth d >= 1: mask, then the children's cls_{d-1}
-// (clsChild == nullptr: d == 1, the children's masks)
-__global__ void k_class_keys(LevelPtrs P, uint32_t lev, const uint32_t* __restrict__ clsChild,
+// keys of levels 1..top for depth d >= 1: mask, then the children's cls_{d-1}
+// (clsChild == nullptr: d == 1, the children's masks).  Class and key arrays
+// start at level 1.
+__global__ void k_class_keys(LevelPtrs P, uint32_t top, const uint32_t* __restrict__ clsChild,
                              uint32_t* __restrict__ keys) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.n[lev]) return;
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= P.base[top + 1] - P.base[1]) return;
+  uint32_t i;
+  const uint32_t lev = level_of(P, e + P.base[1], 1, top, i);
   const uint32_t m = node_mask(P, lev, i);
-  uint32_t* k = keys + (uint64_t)i * kRecWords;
+  const uint64_t below = P.base[lev + 1] - P.base[1];
+  uint32_t* k = keys + e * kRecWords;
   k[0] = m;
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     uint32_t v = kNull;
     if ((m >> c) & 1u) {
       const uint32_t ch = node_child(P, lev, i, c);
-      v = clsChild ? clsChild[ch] : node_mask(P, lev + 1, ch);
+      v = clsChild ? clsChild[below + ch] : node_mask(P, lev + 1, ch);
     }
     k[1 + c] = v;
   }
@@ -95,13 +112,15 @@ __device__ __forceinline__ uint32_t class_of(const LevelPtrs& P, uint32_t lev, u
   return cls ? cls[i] : node_mask(P, lev, i);
 }
 
-// bestOf[class] = min over the nodes of level levB of (levB << 32 | index)
-__global__ void k_class_best(LevelPtrs P, uint32_t levB, const uint32_t* __restrict__ cls,
+// bestOf[class] = min over the nodes of levels 1..top of (level << 32 | index)
+__global__ void k_class_best(LevelPtrs P, uint32_t top, const uint32_t* __restrict__ cls,
                              unsigned long long* __restrict__ bestOf) {
-  const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= P.n[levB]) return;
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= P.base[top + 1] - P.base[1]) return;
+  uint32_t j;
+  const uint32_t levB = level_of(P, e + P.base[1], 1, top, j);
   const unsigned long long key = ((unsigned long long)levB << 32) | j;
-  unsigned long long* b = &bestOf[class_of(P, levB, j, cls)];
+  unsigned long long* b = &bestOf[cls ? cls[e] : node_mask(P, levB, j)];
   if (key < __atomic_load_n(b, __ATOMIC_RELAXED)) atomicMin(b, key);
 }
 
@@ -119,7 +138,7 @@ __global__ void k_frontier_best(LevelPtrs P, uint32_t levA, const uint8_t* __res
   sa[a] = b != ~0ull ? a : kNone;
   sp[a] = 0;
   sb[a] = b;
-  if (b != ~0ull) atomicAdd(nMatched, 1u);
+  if (b != ~0ull) __atomic_store_n(nMatched, 1u, __ATOMIC_RELAXED);   // any match: the levels below are recorded
 }
 
 // One level of the recording pass: children (level lev+1) of recorded nodes.
@@ -185,8 +204,8 @@ __global__ void k_merge_self(uint32_t n, const uint8_t* __restrict__ front, cons
     if ((r[0] >> c) & 1u) nextFront[r[1 + c]] = 1;
 }
 
-__global__ void k_merge_sub(uint32_t n, const uint64_t* __restrict__ cand, uint64_t* __restrict__ mlc) {
-  uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_merge_sub(uint64_t n, const uint64_t* __restrict__ cand, uint64_t* __restrict__ mlc) {
+  const uint64_t x = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (x >= n) return;
   if (cand[x] != ~0ull && mlc[x] == ~0ull) mlc[x] = cand[x];
 }
@@ -195,64 +214,73 @@ __global__ void k_fill64(uint64_t* d, uint64_t v, uint64_t n) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) d[i] = v;
 }
-__global__ void k_fill8(uint8_t* d, uint8_t v, uint64_t n) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) d[i] = v;
+// empty correspondences; the frontier holds level 1
+__global__ void k_init(uint64_t* __restrict__ mlc, uint8_t* __restrict__ front, uint64_t n, uint64_t f0, uint64_t f1) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  mlc[i] = ~0ull;
+  front[i] = i >= f0 && i < f1 ? 1 : 0;
+}
+// an empty recording state
+__global__ void k_clear_record(uint32_t* __restrict__ sa, uint64_t* __restrict__ sp, uint64_t* __restrict__ cand,
+                               uint64_t n) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  sa[i] = kNone;
+  sp[i] = 0;
+  cand[i] = ~0ull;
 }
 
 // ---- compaction (geom_octree_extension.cpp:1428-1498) ------------------------
-__global__ void k_keep_flags(const uint64_t* __restrict__ mlc, uint32_t n, uint32_t* __restrict__ flag) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// The reference compacts bottom-up and rewrites pointers after every level.
+// A pointer's last value depends only on the final correspondences: a child
+// with one becomes its B (level and compacted index), any other its own
+// compacted index.  So all levels are numbered by one scan and written at once.
+__global__ void k_keep_flags(const uint64_t* __restrict__ mlc, uint64_t n, uint32_t* __restrict__ flag) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) flag[i] = mlc[i] == ~0ull ? 1u : 0u;
 }
-
-__global__ void k_compact_level(const uint32_t* __restrict__ rec, const uint32_t* __restrict__ cl, uint32_t n, int leaf,
-                                const uint64_t* __restrict__ mlc, const uint32_t* __restrict__ pos,
-                                uint32_t* __restrict__ outRec, uint32_t* __restrict__ outCl, uint32_t* __restrict__ corr) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (mlc[i] != ~0ull) { corr[i] = kNone; return; }
-  const uint32_t p = pos[i];
-  corr[i] = p;
-  if (leaf) { outRec[p] = rec[i]; return; }
-  for (int k = 0; k < kRecWords; ++k) outRec[(uint64_t)p * kRecWords + k] = rec[(uint64_t)i * kRecWords + k];
-  for (int k = 0; k < 8; ++k) outCl[(uint64_t)p * 8 + k] = cl[(uint64_t)i * 8 + k];
+// kept[l] = the scan at level l's start (l <= L; the total past the last level)
+__global__ void k_level_starts(LevelPtrs P, uint32_t L, const uint32_t* __restrict__ pos,
+                               const uint32_t* __restrict__ total, uint32_t* __restrict__ kept) {
+  const uint32_t l = threadIdx.x;
+  if (l <= L) kept[l] = P.base[l] < P.base[L] ? pos[P.base[l]] : *total;
 }
 
-// Parents (level lev-1) of the nodes of level lev: redirect or renumber.
-__global__ void k_fix_parents(uint32_t* __restrict__ rec, uint32_t* __restrict__ cl, uint32_t n,
-                              const uint64_t* __restrict__ mlc, const uint32_t* __restrict__ corr) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint32_t* r = rec + (uint64_t)i * kRecWords;
-  uint32_t* l = cl + (uint64_t)i * 8;
+struct OutLevels {
+  uint32_t* rec[kMaxL];
+  uint32_t* cl[kMaxL];
+};
+// pos: the scan of the keep flags; kept: its value at every level's start
+__global__ void k_compact(LevelPtrs P, uint32_t L, const uint64_t* __restrict__ mlc, const uint32_t* __restrict__ pos,
+                          const uint32_t* __restrict__ kept, OutLevels out, uint32_t* __restrict__ missing) {
+  const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= P.base[L] || mlc[e] != ~0ull) return;
+  uint32_t i;
+  const uint32_t lev = level_of(P, e, 0, L - 1, i);
+  const uint32_t p = pos[e] - kept[lev];
+  if (lev == P.leafLevel) { out.rec[lev][p] = P.rec[lev][i]; return; }
+  const uint32_t* r = P.rec[lev] + (uint64_t)i * kRecWords;
+  uint32_t* o = out.rec[lev] + (uint64_t)p * kRecWords;
+  uint32_t* l = out.cl[lev] + (uint64_t)p * 8;
+  const uint32_t m = r[0];
+  o[0] = m;
   for (int c = 0; c < 8; ++c) {
-    if (!((r[0] >> c) & 1u)) continue;
-    const uint32_t ch = r[1 + c];
-    const uint64_t m = mlc[ch];
-    if (m != ~0ull) { l[c] = (uint32_t)(m >> 32); r[1 + c] = (uint32_t)m; }
-    else r[1 + c] = corr[ch];
+    uint32_t v = r[1 + c], to = lev + 1;
+    if ((m >> c) & 1u) {
+      const uint64_t w = mlc[P.base[to] + v];
+      if (w != ~0ull) { to = (uint32_t)(w >> 32); v = (uint32_t)w; }
+      const uint64_t t = P.base[to] + v;
+      if (mlc[t] == ~0ull) {
+        v = pos[t] - kept[to];
+      } else {
+        v = kNone;
+        atomicAdd(missing, 1u);
+      }
+    }
+    o[1 + c] = v;
+    l[c] = to;
   }
-}
-
-// Nodes of a lower level whose pointers were redirected into level lev.
-__global__ void k_fix_redirected(uint32_t* __restrict__ rec, const uint32_t* __restrict__ cl, uint32_t n, uint32_t lev,
-                                 const uint32_t* __restrict__ corr, uint32_t* __restrict__ missing) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint32_t* r = rec + (uint64_t)i * kRecWords;
-  const uint32_t* l = cl + (uint64_t)i * 8;
-  for (int c = 0; c < 8; ++c) {
-    if (!((r[0] >> c) & 1u) || l[c] != lev) continue;
-    const uint32_t v = corr[r[1 + c]];
-    if (v == kNone) atomicAdd(missing, 1u);
-    r[1 + c] = v;
-  }
-}
-
-__global__ void k_init_cl(uint32_t* __restrict__ cl, uint32_t n, uint32_t lev) {
-  uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n * 8) cl[i] = lev + 1;
 }
 
 }  // namespace
@@ -262,156 +290,120 @@ void cross_level_merge(svd_octree* o) {
   if (o->state != SVD_S_DAG) throw Error{SVD_ERR_STATE, "cross-level merge needs a DAG"};
   const uint32_t L = o->levels;
   if (L > kMaxL) throw Error{SVD_ERR_LEVELS, "too many levels"};
-  std::vector<Level>& D = o->dag;
-  // working copy of the DAG view with childLevels (the merge rewrites pointers)
-  std::vector<Level> W(L);
   LevelPtrs P{};
   P.leafLevel = L - 1;
   for (uint32_t l = 0; l < L; ++l) {
-    W[l].n = D[l].n;
-    W[l].leaf = D[l].leaf;
-    const uint64_t words = D[l].leaf ? D[l].n : D[l].n * kRecWords;
-    W[l].rec = dalloc<uint32_t>(c, words + 1);
-    if (words) SVD_HIP(hipMemcpyAsync(W[l].rec, D[l].rec, 4 * words, hipMemcpyDeviceToDevice, c->stream));
-    if (!D[l].leaf) {
-      W[l].childLevels = dalloc<uint32_t>(c, 8 * D[l].n + 1);
-      if (D[l].n) k_init_cl<<<div_up(8 * D[l].n, kB), kB, 0, c->stream>>>(W[l].childLevels, (uint32_t)D[l].n, l);
-    }
-    P.rec[l] = W[l].rec;
-    P.n[l] = (uint32_t)W[l].n;
+    P.rec[l] = o->dag[l].rec;
+    P.n[l] = (uint32_t)o->dag[l].n;
+    P.base[l + 1] = P.base[l] + o->dag[l].n;
   }
-  // per-level state
-  std::vector<uint64_t*> mlc(L, nullptr), cand(L, nullptr), sp(L, nullptr);
-  std::vector<uint32_t*> sa(L, nullptr);
-  std::vector<uint8_t*> front(L, nullptr);
-  for (uint32_t l = 0; l < L; ++l) {
-    const uint64_t n = W[l].n + 1;
-    mlc[l] = dalloc<uint64_t>(c, n);
-    cand[l] = dalloc<uint64_t>(c, n);
-    sp[l] = dalloc<uint64_t>(c, n);
-    sa[l] = dalloc<uint32_t>(c, n);
-    front[l] = dalloc<uint8_t>(c, n);
-    k_fill64<<<div_up(n, kB), kB, 0, c->stream>>>(mlc[l], ~0ull, n);
-    k_fill8<<<div_up(n, kB), kB, 0, c->stream>>>(front[l], 0, n);
-  }
-  // classes: cls[d] covers levels 1..L-1-d, level l at base[l]
-  std::vector<uint64_t> base(L + 1, 0);
-  for (uint32_t l = 1; l < L; ++l) base[l + 1] = base[l] + P.n[l];
+  const uint64_t N = P.base[L];
+  uint64_t* mlc = dalloc<uint64_t>(c, N + 1);
+  uint64_t* cand = dalloc<uint64_t>(c, N + 1);
+  uint64_t* sp = dalloc<uint64_t>(c, N + 1);
+  uint32_t* sa = dalloc<uint32_t>(c, N + 1);
+  uint8_t* front = dalloc<uint8_t>(c, N + 1);
+  if (N) k_init<<<div_up(N, kB), kB, 0, c->stream>>>(mlc, front, N, P.base[1], L > 1 ? P.base[2] : P.base[1]);
+  // classes: cls[d] covers levels 1..L-1-d
   std::vector<uint32_t*> cls(L, nullptr);
   std::vector<uint32_t> capOf(L, 256);
+  auto nodes = [&](uint32_t top) { return P.base[top + 1] - P.base[1]; };   // of levels 1..top
   if (L >= 3) {
-    uint32_t* keys = dalloc<uint32_t>(c, (base[L - 1] + 1) * kRecWords);
+    uint32_t* keys = dalloc<uint32_t>(c, (nodes(L - 2) + 1) * kRecWords);
     for (uint32_t d = 1; d + 2 <= L; ++d) {
       const uint32_t top = L - 1 - d;   // deepest level with d levels below it
-      const uint64_t nd = base[top + 1];
+      const uint64_t nd = nodes(top);
       uint64_t cap = 1024;
       while (cap < 2 * nd) cap <<= 1;
       if (cap > (1ull << 31)) throw Error{SVD_ERR_CAPACITY, "cross-level merge: too many nodes"};
       capOf[d] = (uint32_t)cap;
       cls[d] = dalloc<uint32_t>(c, nd + 1);
-      for (uint32_t l = 1; l <= top; ++l)
-        if (P.n[l])
-          k_class_keys<<<div_up(P.n[l], kB), kB, 0, c->stream>>>(P, l, d == 1 ? nullptr : cls[d - 1] + base[l + 1],
-                                                                 keys + base[l] * kRecWords);
       uint32_t* table = dalloc<uint32_t>(c, cap);
       fill_u32(c, table, kNone, cap);
-      if (nd) k_class_insert<<<div_up(nd, kB), kB, 0, c->stream>>>(keys, nd, table, (uint32_t)(cap - 1), cls[d]);
+      if (nd) {
+        k_class_keys<<<div_up(nd, kB), kB, 0, c->stream>>>(P, top, d == 1 ? nullptr : cls[d - 1], keys);
+        k_class_insert<<<div_up(nd, kB), kB, 0, c->stream>>>(keys, nd, table, (uint32_t)(cap - 1), cls[d]);
+      }
       check_launch("k_class");
       dfree(c, table);
     }
     dfree(c, keys);
   }
-  auto clsAt = [&](uint32_t d, uint32_t l) -> const uint32_t* { return d == 0 ? nullptr : cls[d] + base[l]; };
 
-  if (P.n[1]) k_fill8<<<div_up(P.n[1], kB), kB, 0, c->stream>>>(front[1], 1, P.n[1]);
-  uint32_t* nMatched = dalloc<uint32_t>(c, 1);
+  uint32_t* matched = dalloc<uint32_t>(c, L);     // per levA: any match
+  fill_u32(c, matched, 0u, L);
   for (uint32_t levA = 1; levA < L; ++levA) {
     const uint32_t D = L - 1 - levA;   // levels below A
     const uint32_t nA = P.n[levA];
     if (!nA) continue;
+    const uint64_t bA = P.base[levA];
     unsigned long long* best = dalloc<unsigned long long>(c, nA);
     unsigned long long* bestOf = dalloc<unsigned long long>(c, capOf[D]);
     k_fill64<<<div_up(capOf[D], kB), kB, 0, c->stream>>>((uint64_t*)bestOf, ~0ull, capOf[D]);
-    for (uint32_t levB = 1; levB < levA; ++levB)
-      if (P.n[levB]) k_class_best<<<div_up(P.n[levB], kB), kB, 0, c->stream>>>(P, levB, clsAt(D, levB), bestOf);
-    fill_u32(c, nMatched, 0u, 1);
-    k_frontier_best<<<div_up(nA, kB), kB, 0, c->stream>>>(P, levA, front[levA], clsAt(D, levA), bestOf, best,
-                                                            sa[levA], sp[levA], cand[levA], nMatched);
+    const uint32_t* cl = D ? cls[D] : nullptr;
+    const uint64_t nb = nodes(levA - 1);
+    if (nb) k_class_best<<<div_up(nb, kB), kB, 0, c->stream>>>(P, levA - 1, cl, bestOf);
+    k_frontier_best<<<div_up(nA, kB), kB, 0, c->stream>>>(P, levA, front + bA, cl ? cl + (bA - P.base[1]) : nullptr,
+                                                            bestOf, best, sa + bA, sp + bA, cand + bA, matched + levA);
     check_launch("k_frontier_best");
-    if (levA + 1 < L && read_u32(c, nMatched)) {
+    if (levA + 1 < L && read_u32(c, matched + levA)) {
+      const uint64_t b0 = P.base[levA + 1], nBelow = N - b0;
+      if (nBelow) k_clear_record<<<div_up(nBelow, kB), kB, 0, c->stream>>>(sa + b0, sp + b0, cand + b0, nBelow);
       for (uint32_t l = levA; l + 1 < L; ++l) {
-        const uint32_t nc = P.n[l + 1];
-        fill_u32(c, sa[l + 1], kNone, nc);
-        k_fill64<<<div_up(nc + 1, kB), kB, 0, c->stream>>>(sp[l + 1], 0ull, nc + 1);
-        k_fill64<<<div_up(nc + 1, kB), kB, 0, c->stream>>>(cand[l + 1], ~0ull, nc + 1);
         if (!P.n[l]) continue;
         const uint32_t g = div_up(P.n[l], kB);
-        k_prop_min<<<g, kB, 0, c->stream>>>(P, l, sa[l], sa[l + 1]);
-        k_prop_path<<<g, kB, 0, c->stream>>>(P, l, sa[l], sp[l], sa[l + 1], (unsigned long long*)sp[l + 1]);
-        k_prop_write<<<g, kB, 0, c->stream>>>(P, l, sa[l], sp[l], cand[l], sa[l + 1], sp[l + 1], cand[l + 1]);
+        const uint64_t x = P.base[l], y = P.base[l + 1];
+        k_prop_min<<<g, kB, 0, c->stream>>>(P, l, sa + x, sa + y);
+        k_prop_path<<<g, kB, 0, c->stream>>>(P, l, sa + x, sp + x, sa + y, (unsigned long long*)sp + y);
+        k_prop_write<<<g, kB, 0, c->stream>>>(P, l, sa + x, sp + x, cand + x, sa + y, sp + y, cand + y);
         check_launch("cross-level record");
       }
-      for (uint32_t l = levA + 1; l < L; ++l)
-        if (P.n[l]) k_merge_sub<<<div_up(P.n[l], kB), kB, 0, c->stream>>>(P.n[l], cand[l], mlc[l]);
+      if (nBelow) k_merge_sub<<<div_up(nBelow, kB), kB, 0, c->stream>>>(nBelow, cand + b0, mlc + b0);
     }
-    k_merge_self<<<div_up(nA, kB), kB, 0, c->stream>>>(nA, front[levA], best, mlc[levA],
-                                                        levA + 1 < L ? front[levA + 1] : nullptr, W[levA].rec,
+    k_merge_self<<<div_up(nA, kB), kB, 0, c->stream>>>(nA, front + bA, best, mlc + bA,
+                                                        levA + 1 < L ? front + P.base[levA + 1] : nullptr, P.rec[levA],
                                                         levA == L - 1 ? 1 : 0);
     check_launch("cross-level round");
     dfree(c, best); dfree(c, bestOf);
   }
-  dfree(c, nMatched);
+  dfree(c, matched);
   for (auto* p : cls) dfree(c, p);
 
-  // compaction, bottom-up
-  uint32_t* missing = dalloc<uint32_t>(c, 1);
-  uint32_t* total = dalloc<uint32_t>(c, 1);
-  fill_u32(c, missing, 0u, 1);
+  // compaction: kept counts of every level (one read), then every level at once
+  uint32_t* pos = dalloc<uint32_t>(c, N + 1);
+  uint32_t* kept = dalloc<uint32_t>(c, L + 2);
+  uint32_t* missing = dalloc<uint32_t>(c, 2);     // and the scan's total
+  fill_u32(c, missing, 0u, 2);
+  if (N) k_keep_flags<<<div_up(N, kB), kB, 0, c->stream>>>(mlc, N, pos);
+  scan_exclusive(c, pos, pos, N, missing + 1);
+  k_level_starts<<<1, 64, 0, c->stream>>>(P, L, pos, missing + 1, kept);
+  check_launch("k_level_starts");
+  std::vector<uint32_t> h(L + 1);
+  read_u32s(c, kept, h.data(), L + 1);
   std::vector<Level> X(L);
-  X[0] = W[0];
+  OutLevels out{};
   uint64_t nNodes = 1, merged = 0;
-  for (uint32_t lev = L - 1; lev > 0; --lev) {
-    const uint32_t n = P.n[lev];
-    uint32_t* pos = dalloc<uint32_t>(c, n + 1);
-    uint32_t* corr = dalloc<uint32_t>(c, n + 1);
-    if (n) k_keep_flags<<<div_up(n, kB), kB, 0, c->stream>>>(mlc[lev], n, pos);
-    scan_exclusive(c, pos, pos, n, total);
-    const uint64_t keep = read_u32(c, total);
-    merged += n - keep;
-    Level& x = X[lev];
-    x.n = keep;
-    x.leaf = W[lev].leaf;
-    x.rec = dalloc<uint32_t>(c, (x.leaf ? keep : keep * kRecWords) + 1);
-    if (!x.leaf) x.childLevels = dalloc<uint32_t>(c, 8 * keep + 1);
-    if (n) k_compact_level<<<div_up(n, kB), kB, 0, c->stream>>>(W[lev].rec, W[lev].childLevels, n, x.leaf ? 1 : 0,
-                                                                mlc[lev], pos, x.rec, x.childLevels, corr);
-    check_launch("k_compact_level");
-    nNodes += keep;
-    // parents in level lev-1: for lev-1 >= 1 they live in W (not yet compacted)
-    const uint32_t np = P.n[lev - 1];
-    if (np) k_fix_parents<<<div_up(np, kB), kB, 0, c->stream>>>(W[lev - 1].rec, W[lev - 1].childLevels, np,
-                                                                mlc[lev], corr);
-    // already compacted levels [lev, L-2] that were redirected into level lev
-    for (uint32_t low = lev; low + 1 < L; ++low) {
-      if (X[low].n) k_fix_redirected<<<div_up(X[low].n, kB), kB, 0, c->stream>>>(X[low].rec, X[low].childLevels,
-                                                                                   (uint32_t)X[low].n, lev, corr, missing);
-    }
-    check_launch("k_fix");
-    dfree(c, pos); dfree(c, corr);
+  for (uint32_t l = 0; l < L; ++l) {
+    Level& x = X[l];
+    x.n = h[l + 1] - h[l];
+    x.leaf = o->dag[l].leaf;
+    x.rec = dalloc<uint32_t>(c, (x.leaf ? x.n : x.n * kRecWords) + 1);
+    if (!x.leaf) x.childLevels = dalloc<uint32_t>(c, 8 * x.n + 1);
+    out.rec[l] = x.rec;
+    out.cl[l] = x.childLevels;
+    if (l) { nNodes += x.n; merged += P.n[l] - x.n; }
   }
-  X[0] = W[0];
+  if (N) k_compact<<<div_up(N, kB), kB, 0, c->stream>>>(P, L, mlc, pos, kept, out, missing);
+  check_launch("k_compact");
   const uint64_t nMissing = read_u32(c, missing);
   // replace the cross-level view
   for (auto& lv : o->xdag) { dfree(c, lv.rec); dfree(c, lv.childLevels); }
   o->xdag = X;
-  for (uint32_t l = 1; l < L; ++l) { dfree(c, W[l].rec); dfree(c, W[l].childLevels); }
   o->hasX = true;
   o->nNodesX = nNodes;
   o->crossMerged = merged;
-  for (uint32_t l = 0; l < L; ++l) {
-    dfree(c, mlc[l]); dfree(c, cand[l]); dfree(c, sp[l]); dfree(c, sa[l]); dfree(c, front[l]);
-  }
-  dfree(c, missing); dfree(c, total);
+  dfree(c, mlc); dfree(c, cand); dfree(c, sp); dfree(c, sa); dfree(c, front);
+  dfree(c, pos); dfree(c, kept); dfree(c, missing);
   for (auto& e : o->enc) e.valid = false;
   if (nMissing)
     throw Error{SVD_ERR_POINTER, "cross-level merge: " + std::to_string(nMissing) +
