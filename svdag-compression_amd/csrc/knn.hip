@@ -327,32 +327,60 @@ __global__ void __launch_bounds__(kTile) k_window_topk(const float* __restrict__
     if (t < (int)k) { best_d[(uint64_t)x * k + t] = bd[t]; best_i[(uint64_t)x * k + t] = bi[t]; }
 }
 
+// The smallest x of the wavefront, in every lane: a reduction by the VALU's
+// lane shifts (rows of 16, then across rows), the result read from lane 63.
+__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
+#define SVD_DPP_MIN(ctrl, rows) \
+  x = min(x, (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, ctrl, rows, 0xf, false))
+  SVD_DPP_MIN(0x111, 0xf);   // row_shr:1, 2, 4, 8
+  SVD_DPP_MIN(0x112, 0xf);
+  SVD_DPP_MIN(0x114, 0xf);
+  SVD_DPP_MIN(0x118, 0xf);
+  SVD_DPP_MIN(0x142, 0xa);   // row_bcast:15 into rows 1 and 3
+  SVD_DPP_MIN(0x143, 0xc);   // row_bcast:31 into rows 2 and 3
+#undef SVD_DPP_MIN
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+__device__ __forceinline__ uint64_t wave_min(uint64_t m) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const uint32_t lo = __shfl_xor((uint32_t)m, off, 64), hi = __shfl_xor((uint32_t)(m >> 32), off, 64);
+    const uint64_t o = ((uint64_t)hi << 32) | lo;
+    m = o < m ? o : m;
+  }
+  return m;
+}
+
 // One neighbour-of-neighbour round (NN-descent) on the signature Hamming
 // metric: node x keeps the k smallest distinct (distance, index) among its
 // own list and the lists of its neighbours.  Reads `in`, writes `out`.
 // One wavefront per node: the k + k*k candidate ids are deduplicated through
 // a hash set in LDS, each distinct candidate's signature is read once (by the
-// lane whose insert won), and k wave-wide minimum reductions over
-// (distance << 32 | index) take the k smallest.
-template <int KM>
+// lane whose insert won), and k wave-wide minima over the keys (distance <<
+// IDB | index) take the k smallest.  The minima bound it: 32-bit keys (IDB =
+// 22, up to 2^22 nodes) reduced by lane shifts took a round over 466K nodes
+// from 1.28 ms (64-bit keys by shuffles, IDB = 32) to 0.85 - 1.03 ms.
+template <int KM, typename Key>
 __global__ void __launch_bounds__(256) k_knn_refine_wave(const uint32_t* __restrict__ sig, uint64_t n, uint32_t k,
                                                          const uint32_t* __restrict__ in, uint32_t* __restrict__ out) {
   constexpr int kCand = KM * (KM + 1);
   constexpr int kPer = (kCand + 63) / 64;                 // candidates per lane
   constexpr int kSlots = KM <= 16 ? 1024 : 4096;          // >= 2 * kCand, power of two
   constexpr int kShift = KM <= 16 ? 22 : 20;              // 32 - log2(kSlots): the product's high bits
-  __shared__ uint32_t set[4][kSlots];
+  constexpr int IDB = sizeof(Key) == 4 ? (int)kIdBits : 32;
+  constexpr Key kNoKey = ~(Key)0;
+  __shared__ __attribute__((aligned(16))) uint32_t set[4][kSlots];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const uint64_t x = (uint64_t)blockIdx.x * 4 + wave;
   const bool live = x < n;
   uint32_t* S = set[wave];
-  for (int j = lane; j < kSlots; j += 64) S[j] = 0xFFFFFFFFu;
+  for (int j = lane; j < kSlots / 4; j += 64) reinterpret_cast<uint4*>(S)[j] = make_uint4(kNone, kNone, kNone, kNone);
   __syncthreads();
   const uint32_t nc = k + k * k;
-  uint64_t key[kPer];
+  Key key[kPer];
 #pragma unroll
   for (int p = 0; p < kPer; ++p) {
-    key[p] = ~0ull;
+    key[p] = kNoKey;
     const uint32_t c = (uint32_t)(lane + 64 * p);
     if (!live || c >= nc) continue;
     uint32_t z;
@@ -360,14 +388,14 @@ __global__ void __launch_bounds__(256) k_knn_refine_wave(const uint32_t* __restr
       z = in[x * k + c];
     } else {
       const uint32_t y = in[x * k + (c - k) / k];
-      z = (y == 0xFFFFFFFFu || (uint64_t)y >= n) ? 0xFFFFFFFFu : in[(uint64_t)y * k + (c - k) % k];
+      z = (y == kNone || (uint64_t)y >= n) ? kNone : in[(uint64_t)y * k + (c - k) % k];
     }
-    if (z == 0xFFFFFFFFu || (uint64_t)z == x || (uint64_t)z >= n) continue;
+    if (z == kNone || (uint64_t)z == x || (uint64_t)z >= n) continue;
     uint32_t h = (z * 2654435761u) >> kShift;
     bool mine = false;
     while (true) {
-      const uint32_t old = atomicCAS(&S[h], 0xFFFFFFFFu, z);
-      if (old == 0xFFFFFFFFu) { mine = true; break; }
+      const uint32_t old = atomicCAS(&S[h], kNone, z);
+      if (old == kNone) { mine = true; break; }
       if (old == z) break;
       h = (h + 1) & (kSlots - 1);
     }
@@ -380,23 +408,21 @@ __global__ void __launch_bounds__(256) k_knn_refine_wave(const uint32_t* __restr
       const uint4 a = px[q], b = pz[q];
       d += __popc(a.x ^ b.x) + __popc(a.y ^ b.y) + __popc(a.z ^ b.z) + __popc(a.w ^ b.w);
     }
-    key[p] = ((uint64_t)d << 32) | z;
+    key[p] = ((Key)d << IDB) | z;
   }
+  Key mine = kNoKey;                 // lane t: the t-th smallest
   for (uint32_t t = 0; t < k; ++t) {
-    uint64_t m = key[0];
+    Key m = key[0];
 #pragma unroll
     for (int p = 1; p < kPer; ++p) m = key[p] < m ? key[p] : m;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      const uint32_t lo = __shfl_xor((uint32_t)m, off, 64), hi = __shfl_xor((uint32_t)(m >> 32), off, 64);
-      const uint64_t o = ((uint64_t)hi << 32) | lo;
-      m = o < m ? o : m;
-    }
-    if (live && lane == 0) out[x * k + t] = m == ~0ull ? 0xFFFFFFFFu : (uint32_t)m;
+    m = wave_min(m);
+    if ((uint32_t)lane == t) mine = m;
 #pragma unroll
     for (int p = 0; p < kPer; ++p)
-      if (key[p] == m) key[p] = ~0ull;   // candidates are distinct: one lane holds m
+      if (key[p] == m) key[p] = kNoKey;   // candidates are distinct: one lane holds m
   }
+  if (live && (uint32_t)lane < k)
+    out[x * k + lane] = mine == kNoKey ? kNone : (uint32_t)(mine & (((Key)1 << (IDB - 1) << 1) - 1));
 }
 
 }  // namespace
@@ -406,11 +432,15 @@ void knn_refine(svd_ctx* c, const uint32_t* sig, uint64_t n, uint32_t k, uint32_
   if (k < 1 || k > (uint32_t)kMaxK) throw Error{SVD_ERR_ARG, "knn: k must be 1..32"};
   uint32_t* tmp = dalloc<uint32_t>(c, n * k);
   for (uint32_t r = 0; r < rounds; ++r) {
-    if (k <= 16) k_knn_refine_wave<16><<<div_up(n, 4), 256, 0, c->stream>>>(sig, n, k, knn, tmp);
-    else k_knn_refine_wave<kMaxK><<<div_up(n, 4), 256, 0, c->stream>>>(sig, n, k, knn, tmp);
-    SVD_HIP(hipMemcpyAsync(knn, tmp, n * k * 4, hipMemcpyDeviceToDevice, c->stream));
+    const uint32_t* in = r & 1 ? tmp : knn;
+    uint32_t* out = r & 1 ? knn : tmp;
+    if (k <= 16 && n <= (1ull << kIdBits))
+      k_knn_refine_wave<16, uint32_t><<<div_up(n, 4), 256, 0, c->stream>>>(sig, n, k, in, out);
+    else if (k <= 16) k_knn_refine_wave<16, uint64_t><<<div_up(n, 4), 256, 0, c->stream>>>(sig, n, k, in, out);
+    else k_knn_refine_wave<kMaxK, uint64_t><<<div_up(n, 4), 256, 0, c->stream>>>(sig, n, k, in, out);
   }
   check_launch("k_knn_refine");
+  if (rounds & 1) SVD_HIP(hipMemcpyAsync(knn, tmp, n * k * 4, hipMemcpyDeviceToDevice, c->stream));
   dfree(c, tmp);
 }
 

@@ -447,15 +447,16 @@ __global__ void __launch_bounds__(256) k_ranked_lists(const uint32_t* __restrict
   counts[j] = m;
 }
 
-// Learned proposals -> (hi << 32 | lo) keys; invalid entries get ~0.
+// Learned proposals -> keys hi << nb | lo (nodes below 2^nb); invalid entries
+// get the bit above, so that the sort reads 2 nb + 1 bits.
 __global__ void k_proposal_keys(const uint32_t* __restrict__ knn, uint64_t n, uint32_t k,
                                 const uint32_t* __restrict__ sig, const uint64_t* __restrict__ refs, uint64_t maxRefs,
-                                uint32_t bound, uint64_t* __restrict__ keys) {
+                                uint32_t bound, int nb, uint64_t* __restrict__ keys) {
   uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * k) return;
   const uint64_t x = e / k;
   const uint32_t y = knn[e];
-  uint64_t key = ~0ull;
+  uint64_t key = 1ull << (2 * nb);
   if (y != kNone && (uint64_t)y != x && (uint64_t)y < n) {
     const uint64_t lo = x < y ? x : y, hi = x < y ? y : x;
     if (refs[hi] <= maxRefs) {
@@ -463,27 +464,27 @@ __global__ void k_proposal_keys(const uint32_t* __restrict__ knn, uint64_t n, ui
       const uint4* p = reinterpret_cast<const uint4*>(sig + hi * 16);
 #pragma unroll
       for (int q = 0; q < 4; ++q) { const uint4 t = p[q]; s[4 * q] = t.x; s[4 * q + 1] = t.y; s[4 * q + 2] = t.z; s[4 * q + 3] = t.w; }
-      if (hamming512(reinterpret_cast<const uint4*>(sig + lo * 16), s) <= bound) key = (hi << 32) | lo;
+      if (hamming512(reinterpret_cast<const uint4*>(sig + lo * 16), s) <= bound) key = (hi << nb) | lo;
     }
   }
   keys[e] = key;
 }
 
 // Sorted keys -> per hi node its first cap distinct lo (ascending).
-__global__ void k_lists_from_sorted(const uint64_t* __restrict__ keys, uint64_t m, uint32_t cap,
+__global__ void k_lists_from_sorted(const uint64_t* __restrict__ keys, uint64_t m, uint32_t cap, int nb,
                                     uint32_t* __restrict__ lists, uint32_t* __restrict__ counts) {
   uint64_t p = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= m) return;
   const uint64_t key = keys[p];
-  if (key == ~0ull) return;
-  const uint64_t hi = key >> 32;
-  if (p > 0 && (keys[p - 1] >> 32) == hi) return;
+  if (key >> (2 * nb)) return;
+  const uint64_t hi = key >> nb;
+  if (p > 0 && (keys[p - 1] >> nb) == hi) return;
   uint32_t cnt = 0;
   uint64_t prev = ~0ull;
   for (uint64_t q = p; q < m && cnt < cap; ++q) {
     const uint64_t kq = keys[q];
-    if (kq == ~0ull || (kq >> 32) != hi) break;
-    if (kq != prev) { lists[hi * cap + cnt++] = (uint32_t)kq; prev = kq; }
+    if ((kq >> nb) != hi) break;           // an invalid key's is above every node
+    if (kq != prev) { lists[hi * cap + cnt++] = (uint32_t)(kq & ((1ull << nb) - 1)); prev = kq; }
   }
   counts[hi] = cnt;
 }
@@ -794,17 +795,18 @@ struct PhaseClock {
 
 }  // namespace
 
-// Sort n u64 keys ascending in place (rocPRIM radix sort through a scratch copy).
-void sort_u64(svd_ctx* c, uint64_t* keys, uint64_t n) {
-  if (n < 2) return;
-  uint64_t* tmpKeys = dalloc<uint64_t>(c, n);
+// n u64 keys ascending by their low bits, through a scratch copy that takes
+// their place: returns the array that holds them and frees the other.
+static uint64_t* sort_u64(svd_ctx* c, uint64_t* keys, uint64_t n, int bits) {
+  if (n < 2) return keys;
+  uint64_t* sorted = dalloc<uint64_t>(c, n);
   size_t bytes = 0;
-  SVD_HIP(rocprim::radix_sort_keys(nullptr, bytes, keys, tmpKeys, (size_t)n, 0, 64, c->stream));
+  SVD_HIP(rocprim::radix_sort_keys(nullptr, bytes, keys, sorted, (size_t)n, 0, bits, c->stream));
   void* tmp = c->arena->get(bytes + 16);
-  SVD_HIP(rocprim::radix_sort_keys(tmp, bytes, keys, tmpKeys, (size_t)n, 0, 64, c->stream));
-  SVD_HIP(hipMemcpyAsync(keys, tmpKeys, n * 8, hipMemcpyDeviceToDevice, c->stream));
+  SVD_HIP(rocprim::radix_sort_keys(tmp, bytes, keys, sorted, (size_t)n, 0, bits, c->stream));
   c->arena->put(tmp);
-  dfree(c, tmpKeys);
+  dfree(c, keys);
+  return sorted;
 }
 
 void lossy_signatures(svd_octree* o, uint32_t lev, uint32_t* sig) {
@@ -923,10 +925,13 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
       uint64_t* keys = dalloc<uint64_t>(c, n * k + 1);
       fill_u32(c, counts, 0u, n + 1);
       if (n) {
-        k_proposal_keys<<<div_up(n * k, kB), kB, 0, c->stream>>>(knn, n, k, sig, refs[lev], maxRefs, bound, keys);
+        int nb = 1;                        // n < 2^32 (32-bit node ids): at most 31 bits keep the flag in the key
+        while (n >> nb) ++nb;
+        if (nb > 31) throw Error{SVD_ERR_CAPACITY, "too many nodes in one level for the learned proposer"};
+        k_proposal_keys<<<div_up(n * k, kB), kB, 0, c->stream>>>(knn, n, k, sig, refs[lev], maxRefs, bound, nb, keys);
         check_launch("k_proposal_keys");
-        sort_u64(c, keys, n * k);
-        k_lists_from_sorted<<<div_up(n * k, kB), kB, 0, c->stream>>>(keys, n * k, cap, lists, counts);
+        keys = sort_u64(c, keys, n * k, 2 * nb + 1);
+        k_lists_from_sorted<<<div_up(n * k, kB), kB, 0, c->stream>>>(keys, n * k, cap, nb, lists, counts);
         check_launch("k_lists_from_sorted");
       }
       dfree(c, keys); dfree(c, knn); dfree(c, emb);

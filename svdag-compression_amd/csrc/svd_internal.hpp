@@ -274,7 +274,6 @@ void render_scratch_init(svd_ctx* c);
 void ao_frame(svd_scene* s, const svd_trace_params* p, uint32_t nrays, float* vis, svd_ray_result* prim);
 
 // ---- lossy DAG (lossy.hip), learned encoder (mlp.hip), kNN (knn.hip) ----------
-void sort_u64(svd_ctx* c, uint64_t* keys, uint64_t n);
 void lossy_signatures(svd_octree* o, uint32_t lev, uint32_t* sig);
 void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy_level_stats>& out);
 void mlp_embed(svd_mlp* m, const uint32_t* sig, uint64_t n, float* emb);

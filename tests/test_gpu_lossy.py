@@ -320,6 +320,25 @@ def test_knn_full_window_is_brute_force(ctx):
 
 
 # ---------------------------------------------------------------- learned lossy
+@pytest.mark.parametrize("k,rounds", [(1, 1), (15, 2), (16, 1), (16, 3), (17, 2), (32, 1)])
+def test_knn_refine_list_sizes(ctx, k, rounds):
+    """Refinement with 32-bit keys (k <= 16) and 64-bit ones, after an odd and
+    an even number of rounds: the recorded lists equal the oracle's."""
+    codes, L = W.cave_codes(6, seed=4), 6
+    g, m = gpu_dag(ctx, codes, L), S.MLP(ctx, seed=1)
+    n = g.level_size(S.VIEW_DAG, L - 2)
+    dsig = torch.zeros(n * 16, dtype=torch.int32, device=DEV)
+    demb = torch.zeros(n * 32, dtype=torch.float32, device=DEV)
+    torch.cuda.synchronize()
+    g.lossy_signatures(L - 2, dsig.data_ptr())
+    m.embed(dsig.data_ptr(), n, demb.data_ptr())
+    ctx.sync()
+    sig, emb = dsig.cpu().numpy().view(np.uint32).reshape(n, 16), demb.cpu().numpy().reshape(n, 32)
+    _, rec = g.lossy_merge(L - 2, L - 2, max_diff=10, model=m, k=k, refine=rounds, record_knn=True)
+    want = O.knn_refine(sig, O.knn_lsh(emb, k, 8, 16, 64, 7, sig=sig), rounds)
+    np.testing.assert_array_equal(rec[:n * k].reshape(n, k), want)
+
+
 def test_lossy_learned_matches_oracle_given_knn(ctx):
     codes, L = W.cave_codes(7, seed=3), 7
     g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
