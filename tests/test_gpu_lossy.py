@@ -179,6 +179,21 @@ def test_lossy_signatures_match_oracle(ctx):
         np.testing.assert_array_equal(sig.cpu().numpy().view(np.uint32).reshape(n, 16), o.lossy_signatures(lev))
 
 
+@pytest.mark.parametrize("L", [3, 4, 6])
+def test_lossy_signatures_every_level(ctx, L):
+    """The root and the two levels above the voxels, whose occupancies end
+    before 512 bits."""
+    codes = random_codes(L, 40 * L, seed=L)
+    g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
+    for lev in range(L):
+        n = g.level_size(S.VIEW_DAG, lev)
+        sig = torch.full((n * 16,), -1, dtype=torch.int32, device=DEV)
+        torch.cuda.synchronize()
+        g.lossy_signatures(lev, sig.data_ptr())
+        ctx.sync()
+        np.testing.assert_array_equal(sig.cpu().numpy().view(np.uint32).reshape(n, 16), o.lossy_signatures(lev))
+
+
 def test_lossy_argument_errors(ctx):
     codes, L = W.terrain_codes(6, seed=1), 6
     g = gpu_dag(ctx, codes, L)
