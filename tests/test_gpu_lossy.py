@@ -241,10 +241,12 @@ def test_mlp_forward_matches_oracle(ctx):
     assert np.corrcoef(e_g.ravel(), e_o.ravel())[0, 1] > 0.9999
 
 
-def test_mlp_gradients_match_oracle(ctx):
+@pytest.mark.parametrize("P", [16, 48, 256, 4112])
+def test_mlp_gradients_match_oracle(ctx, P):
+    """Batches of one workgroup, a partial split of the weight gradients, several
+    splits, and more workgroups than compute units."""
     m = S.MLP(ctx, seed=9)
     p = M.init_params(9)
-    P = 256
     sig = _rand_sigs(2 * P, 2)
     sig[1::2] = sig[0::2] ^ (_rand_sigs(P, 3, density=0.02))     # near pairs
     H = M.hamming(sig[0::2], sig[1::2])
