@@ -26,6 +26,21 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// x of the lane below; lane 0 gets `zero` (a wavefront shift of the VALU, no
+// LDS round trip as a shuffle needs).
+__device__ __forceinline__ uint32_t lane_below(uint32_t x, uint32_t zero) {
+  constexpr int kWaveShr1 = 0x138;
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)zero, (int)x, kWaveShr1, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint64_t lane_below(uint64_t x, uint64_t zero) {
+  return ((uint64_t)lane_below((uint32_t)(x >> 32), (uint32_t)(zero >> 32)) << 32) |
+         lane_below((uint32_t)x, (uint32_t)zero);
+}
+__device__ __forceinline__ uint64_t last_lane(uint64_t x) {
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), 63) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, 63);
+}
+
 // Sources of the codes the one-pass level builds read: plain codes, or a
 // batch's per-scene codes tagged on the fly with their scene id above bit
 // kSceneTagShift (scene-major, so the tagged list ascends when each scene's
@@ -81,13 +96,14 @@ struct TaggedCodes {
   }
 };
 
-// A tile of sorted codes for the one-pass level builds: thread (wave w, lane
+// A tile of sorted codes for the level builds: thread (wave w, lane
 // j) holds codes w * 64 * PER + 64 * k + j (k < PER) of the tile, so every
 // load is coalesced; a run of codes sharing code >> 3 is one parent node.
 // After run_tile: head bit k = code k starts a run, rank[k] = the run's
 // number within the tile counted from the tile's first head (-1: the code
-// continues the previous tile's last run), agg = the tile's runs.
-// 512 threads per run tile: tile numbers come from one device counter whose
+// continues the previous tile's last run), agg = the tile's runs, bad = the
+// thread's codes that do not ascend or have a bit of hiMask set.
+// 512 threads per run tile: in one pass, tile numbers come from one device counter whose
 // same-address atomics serialise, so fewer, larger tiles start sooner.
 constexpr int kRunT = 512;
 template <int PER>
@@ -96,10 +112,11 @@ struct RunTile {
   int32_t rank[PER];
   uint32_t heads = 0;
   uint32_t agg = 0;
+  uint32_t bad = 0;
 };
 template <int PER, typename Src>
 __device__ __forceinline__ void run_tile(Src& code, uint64_t n, uint64_t tileBase, RunTile<PER>& t,
-                                         uint32_t* wtot) {
+                                         uint32_t* wtot, uint64_t hiMask) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t wbase = tileBase + (uint64_t)wave * (64 * PER) + lane;
 #pragma unroll
@@ -114,15 +131,15 @@ __device__ __forceinline__ void run_tile(Src& code, uint64_t n, uint64_t tileBas
     if (i < n) t.v[k] = code.tag(i, t.v[k]);
   }
   const uint64_t first = tileBase + (uint64_t)wave * (64 * PER);
-  const uint64_t before = (lane == 0 && first > 0 && first - 1 < n) ? code(first - 1) : 0ull;
+  uint64_t before = (lane == 0 && first > 0 && first - 1 < n) ? code(first - 1) : 0ull;   // of use to lane 0
   uint32_t c = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const uint64_t i = wbase + 64 * k;
-    const uint64_t up = __shfl_up(t.v[k], 1, 64);
-    const uint64_t wrap = k ? __shfl(t.v[k - 1], 63, 64) : before;
-    const uint64_t u = lane ? up : wrap;
+    const uint64_t u = lane_below(t.v[k], before);
+    before = last_lane(t.v[k]);
     const bool h = i < n && (i == 0 || (t.v[k] >> 3) != (u >> 3));
+    t.bad += (i < n && ((t.v[k] & hiMask) != 0 || (i > 0 && t.v[k] <= u))) ? 1u : 0u;
     const uint64_t b = __ballot(h);
     t.heads |= (h ? 1u : 0u) << k;
     // inclusive head count up to this code, minus one
@@ -162,182 +179,258 @@ __device__ __forceinline__ uint32_t run_tail_bits(const Src& code, uint64_t n, u
 // Input contract: strictly ascending codes with no bit of hiMask set (plain
 // codes: every bit from 3 * levels up; scene-tagged codes: bit 63, which
 // TaggedCodes sets on a code beyond its scene's depth).
-// One pass over the codes for the finest level: the input check, every
-// level's node count, the run heads, their numbering by a single-pass scan,
-// and the leaf masks and parent codes.  Code i starts a node of the level k
-// steps above the voxels (prefix code >> 3k) exactly when k <= K_i =
-// floor(msb(code[i] ^ code[i-1]) / 3) (K_0 = L), so the level k steps up has
-// #{i : K_i >= k} nodes; part[tile * (L + 1) + k] = that count over the tile
-// (k >= 1), part[tile * (L + 1)] = the tile's bad codes.  Counts go per tile
-// rather than to device atomics, whose same-address updates from thousands
-// of workgroups would queue.  Each code ORs its bit into its run's LDS mask;
-// a run that crosses the tile's end reads the codes past it.  With bad input
-// the writes stay below n and the caller throws on the bad count.
+// A batch's node scenes as a level is written: scene[i] = parent code >> shift
+// (none when null).
+struct SceneOut { uint32_t* scene; int shift; };
+
+// The finest level: the leaf masks and parent codes of the runs that start in
+// one tile of codes, the tile's first head being leaf `prefix`.  Each code ORs
+// its bit into its run's LDS mask (cleared); a run that crosses the tile's end
+// reads the codes past it.
+template <int PER>
+__device__ __forceinline__ void leaf_masks(uint64_t n, uint64_t tileBase, const RunTile<PER>& t, uint32_t* lmask) {
+  const uint64_t wbase = tileBase + (uint64_t)(threadIdx.x >> 6) * (64 * PER) + (threadIdx.x & 63);
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (wbase + 64 * k < n && t.rank[k] >= 0) atomicOr(&lmask[t.rank[k]], 1u << (uint32_t)(t.v[k] & 7u));
+}
+template <int PER, typename Src>
+__device__ __forceinline__ void leaf_write(const Src& code, uint64_t n, uint64_t tileBase, const RunTile<PER>& t,
+                                           uint32_t prefix, const uint32_t* lmask, uint32_t* __restrict__ mask,
+                                           uint64_t* __restrict__ pcode) {
+  uint64_t last = ~0ull;               // parent code of the tile's last run, in the thread of its head
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if (!((t.heads >> k) & 1u)) continue;
+    const uint32_t r = (uint32_t)t.rank[k];
+    const uint64_t pc = t.v[k] >> 3;
+    if (r + 1 == t.agg) last = pc;
+    mask[prefix + r] = lmask[r];
+    pcode[prefix + r] = pc;
+  }
+  const uint64_t tileEnd = tileBase + (uint64_t)kRunT * PER;
+  if (last != ~0ull && tileEnd < n)
+    mask[prefix + t.agg - 1] = lmask[t.agg - 1] | run_tail_bits(code, n, tileEnd, last);
+}
+
+// A level in one pass over the codes below it (run heads numbered by a
+// look-back scan), or, from this many codes, in two: a pass that counts each
+// tile's heads, a scan of the counts and a pass that writes.  One pass reads
+// the codes once, but holds every tile until its predecessors are known: the
+// leaves of 463M codes (a batch) took 1.84 ms in one pass and 1.03 + 0.60 ms in
+// two, of 13.7M codes 63 and 58 us; of 12K codes the two launches more cost
+// 40 us of a build's 400.
+constexpr uint64_t kTwoPassCodes = 4ull << 20;
+
+// The leaves in one pass; bad codes are added to bad[0] (zero between builds;
+// with bad input the writes stay below n and the caller throws on the count),
+// *leaves = the level's nodes.
 constexpr int kLeafPer = 16;
 constexpr uint32_t kLeafTile = kRunT * kLeafPer;
 template <typename Src>
-__global__ void __launch_bounds__(kRunT) k_leaf_build(Src src, uint64_t n, uint32_t L, uint64_t hiMask, LbPass p,
-                                                      uint32_t* __restrict__ part, uint32_t* __restrict__ hist,
-                                                      uint32_t* __restrict__ mask, uint64_t* __restrict__ pcode) {
+__global__ void __launch_bounds__(kRunT) k_leaf_build(Src src, uint64_t n, uint64_t hiMask, LbPass p, uint32_t* bad,
+                                                      uint32_t* __restrict__ leaves, uint32_t* __restrict__ mask,
+                                                      uint64_t* __restrict__ pcode) {
   __shared__ uint32_t lds[kRunT / 64 + 2];
   __shared__ uint32_t word;
-  __shared__ uint32_t cpart[kMaxLevels + 1][kRunT / 64];
   __shared__ uint32_t lmask[kLeafTile];
   const uint32_t tile = lb_take_tile(p, &word);
   const uint64_t tileBase = (uint64_t)tile * kLeafTile;
-  if (tile == 0 && threadIdx.x <= L) hist[threadIdx.x] = 0;   // k_level_counts adds to it
   for (uint32_t j = threadIdx.x; j < kLeafTile; j += kRunT) lmask[j] = 0;
   Src code = src;
   RunTile<kLeafPer> t;
-  run_tile(code, n, tileBase, t, lds);   // its barrier also orders the clearing
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t wbase = tileBase + (uint64_t)wave * (64 * kLeafPer) + lane;
-  // per-thread histogram of K over the good codes, 6-bit bins packed in three
-  // 64-bit words (bins 0-9, 10-19, 20-21; at most kLeafPer < 64 per bin):
-  // a few operations per code instead of one counter per level
-  static_assert(kLeafPer < 64, "6-bit histogram bins");
-  uint64_t hA = 0, hB = 0, hC = 0;
-  uint32_t nBad = 0;
-#pragma unroll
-  for (int k = 0; k < kLeafPer; ++k) {
-    const uint64_t i = wbase + 64 * k;
-    const uint64_t x = t.v[k];
-    const uint64_t up = __shfl_up(x, 1, 64);
-    const uint64_t wrap = k ? __shfl(t.v[k - 1], 63, 64) : (lane == 0 && i > 0 && i - 1 < n ? code(i - 1) : 0ull);
-    const uint64_t u = lane ? up : wrap;
-    if (i >= n) continue;
-    uint32_t K = L;
-    bool bad = (x & hiMask) != 0;
-    if (i > 0) {
-      if (x <= u) bad = true;
-      else K = min(L, (uint32_t)(63 - __clzll((long long)(x ^ u))) / 3u);
-    }
-    nBad += bad ? 1u : 0u;
-    const uint32_t kb = K < 10 ? K : (K < 20 ? K - 10 : K - 20);
-    const uint64_t one = bad ? 0ull : 1ull << (6 * kb);
-    hA += K < 10 ? one : 0ull;
-    hB += (K >= 10 && K < 20) ? one : 0ull;
-    hC += K >= 20 ? one : 0ull;
-    if (t.rank[k] >= 0) atomicOr(&lmask[t.rank[k]], 1u << (uint32_t)(x & 7u));
-  }
-  // level q (q >= 1) counts the good codes with K >= q: suffix sums of the bins
-  uint32_t cnt[kMaxLevels + 1];
-  cnt[0] = nBad;
-  {
-    uint32_t run = 0;
-#pragma unroll
-    for (int q = (int)kMaxLevels; q >= 1; --q) {
-      const uint64_t w = q < 10 ? hA : (q < 20 ? hB : hC);
-      const int sh = 6 * (q < 10 ? q : (q < 20 ? q - 10 : q - 20));
-      run += (uint32_t)(w >> sh) & 63u;
-      cnt[q] = run;
-    }
-  }
-#pragma unroll
-  for (int q = 0; q <= (int)kMaxLevels; ++q) {
-    uint32_t x = cnt[q];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-    if (lane == 0) cpart[q][wave] = x;
-  }
+  run_tile(code, n, tileBase, t, lds, hiMask);   // its barrier also orders the clearing
+  if (t.bad) atomicAdd(bad, t.bad);
+  leaf_masks(n, tileBase, t, lmask);
+  const uint32_t prefix = lb_exclusive(p, tile, t.agg, lds);   // its barriers also order the masks
+  if (threadIdx.x == 0 && tile == p.tiles - 1) *leaves = prefix + t.agg;
+  leaf_write(code, n, tileBase, t, prefix, lmask, mask, pcode);
+}
+
+// The two passes: smaller tiles, as nothing waits for a tile here and more
+// workgroups fit on a CU.
+constexpr int kScanPer = 8;
+constexpr uint32_t kScanTile = kRunT * kScanPer;
+template <typename Src>
+__global__ void __launch_bounds__(kRunT) k_run_count(Src src, uint64_t n, uint64_t hiMask, uint32_t* bad,
+                                                     uint32_t* __restrict__ heads) {
+  __shared__ uint32_t lds[kRunT / 64];
+  Src code = src;
+  RunTile<kScanPer> t;
+  run_tile(code, n, (uint64_t)blockIdx.x * kScanTile, t, lds, hiMask);
+  if (t.bad) atomicAdd(bad, t.bad);
+  if (threadIdx.x == 0) heads[blockIdx.x] = t.agg;
+}
+template <typename Src>
+__global__ void __launch_bounds__(kRunT) k_leaf_scanned(Src src, uint64_t n, const uint32_t* __restrict__ before,
+                                                        uint32_t* __restrict__ mask, uint64_t* __restrict__ pcode) {
+  __shared__ uint32_t lds[kRunT / 64];
+  __shared__ uint32_t lmask[kScanTile];
+  const uint64_t tileBase = (uint64_t)blockIdx.x * kScanTile;
+  for (uint32_t j = threadIdx.x; j < kScanTile; j += kRunT) lmask[j] = 0;
+  Src code = src;
+  RunTile<kScanPer> t;
+  run_tile(code, n, tileBase, t, lds, 0ull);
+  leaf_masks(n, tileBase, t, lmask);
+  const uint32_t prefix = before[blockIdx.x];
   __syncthreads();
-  if (threadIdx.x <= L) {
-    uint32_t x = 0;
+  leaf_write(code, n, tileBase, t, prefix, lmask, mask, pcode);
+}
+
+// An inner level: the records of the nodes whose runs start in one tile of
+// child codes (child pointer = the child's position in its level) and the
+// parent codes.  The children of a run are neighbours, so its record follows
+// from its first child's position and its mask: lrun[r] = position in the tile
+// << 8 | mask, filled by run_words (cleared before).  inner_write then stores
+// the tile's records, 36 bytes each and one after another, as one run of
+// words: every store of a wavefront is a full line, where a thread per code and
+// head storing its own words of a record touched each line nine times
+// (123M codes of a batch: 0.90 -> 0.42 ms; 3.9M codes in one pass: 43 -> 27 us).
+template <int PER>
+__device__ __forceinline__ void run_words(uint64_t n, uint64_t tileBase, const RunTile<PER>& t, uint32_t* lrun) {
+  const uint32_t at = (threadIdx.x >> 6) * (64 * PER) + (threadIdx.x & 63);
 #pragma unroll
-    for (int w = 0; w < kRunT / 64; ++w) x += cpart[threadIdx.x][w];
-    part[(uint64_t)tile * (L + 1) + threadIdx.x] = x;
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t j = at + 64 * k;
+    if (tileBase + j < n && t.rank[k] >= 0)
+      atomicOr(&lrun[t.rank[k]], (1u << (uint32_t)(t.v[k] & 7u)) | (((t.heads >> k) & 1u) ? j << 8 : 0u));
   }
-  const uint32_t prefix = lb_exclusive(p, tile, t.agg, lds);
-  const uint64_t tileEnd = tileBase + kLeafTile;
+}
+template <int PER>
+__device__ __forceinline__ void inner_write(const PlainCodes& src, uint64_t n, uint64_t tileBase, const RunTile<PER>& t,
+                                            uint32_t prefix, uint32_t* lrun, uint32_t* __restrict__ rec,
+                                            uint64_t* __restrict__ pcode, SceneOut sc) {
+  uint64_t last = ~0ull;               // parent code of the tile's last run, in the thread of its head
 #pragma unroll
-  for (int k = 0; k < kLeafPer; ++k) {
+  for (int k = 0; k < PER; ++k) {
     if (!((t.heads >> k) & 1u)) continue;
     const uint32_t r = (uint32_t)t.rank[k];
-    uint32_t m = lmask[r];
     const uint64_t pc = t.v[k] >> 3;
-    if (r + 1 == t.agg && tileEnd < n) m |= run_tail_bits(code, n, tileEnd, pc);
-    mask[prefix + r] = m;
-    pcode[prefix + r] = pc;
+    if (r + 1 == t.agg) last = pc;
+    if (pcode) pcode[prefix + r] = pc;
+    if (sc.scene) sc.scene[prefix + r] = (uint32_t)(pc >> sc.shift);
+  }
+  const uint64_t tileEnd = tileBase + (uint64_t)kRunT * PER;
+  if (last != ~0ull && tileEnd < n) lrun[t.agg - 1] |= run_tail_bits(src, n, tileEnd, last);
+  __syncthreads();
+  uint32_t* o = rec + (uint64_t)prefix * kRecWords;
+  for (uint32_t w = threadIdx.x; w < t.agg * kRecWords; w += kRunT) {
+    const uint32_t r = w / kRecWords, c = w - r * kRecWords, run = lrun[r], m = run & 0xFFu;
+    const uint32_t bit = c ? 1u << (c - 1) : 0u;
+    const uint32_t child = (uint32_t)tileBase + (run >> 8) + __popc(m & (bit - 1));
+    o[w] = c == 0 ? m : ((m & bit) ? child : kNull);
   }
 }
 
-// An inner level in one pass: run heads of the child codes, their numbering
-// by a single-pass scan, the records (child pointer = the child's position
-// in its level) and the parent codes.  Every code stores its own child
-// pointer into its parent's record and ORs its slot into the run's LDS mask;
-// the head writes the mask and kNull into the other slots.
+// In one pass: the run heads are numbered by a look-back scan.
 constexpr int kInnerPer = 16;
 constexpr uint32_t kInnerTile = kRunT * kInnerPer;
 __global__ void __launch_bounds__(kRunT) k_inner_build(const uint64_t* __restrict__ ccode, uint64_t n, LbPass p,
-                                                       uint32_t* __restrict__ rec, uint64_t* __restrict__ pcode) {
+                                                       uint32_t* __restrict__ rec, uint64_t* __restrict__ pcode,
+                                                       SceneOut sc) {
   __shared__ uint32_t lds[kRunT / 64 + 2];
   __shared__ uint32_t word;
-  __shared__ uint32_t lmask[kInnerTile];
+  __shared__ uint32_t lrun[kInnerTile];
   const uint32_t tile = lb_take_tile(p, &word);
   const uint64_t tileBase = (uint64_t)tile * kInnerTile;
-  for (uint32_t j = threadIdx.x; j < kInnerTile; j += kRunT) lmask[j] = 0;
+  for (uint32_t j = threadIdx.x; j < kInnerTile; j += kRunT) lrun[j] = 0;
   RunTile<kInnerPer> t;
   PlainCodes src{ccode};
-  run_tile(src, n, tileBase, t, lds);
-  const uint32_t prefix = lb_exclusive(p, tile, t.agg, lds);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint64_t wbase = tileBase + (uint64_t)wave * (64 * kInnerPer) + lane;
-#pragma unroll
-  for (int k = 0; k < kInnerPer; ++k) {
-    const uint64_t i = wbase + 64 * k;
-    if (i >= n) continue;
-    const uint32_t sl = (uint32_t)(t.v[k] & 7u);
-    // rank -1: the run began in the previous tile, whose last node is prefix - 1
-    rec[(uint64_t)(prefix + t.rank[k]) * kRecWords + 1 + sl] = (uint32_t)i;
-    if (t.rank[k] >= 0) atomicOr(&lmask[t.rank[k]], 1u << sl);
-  }
+  run_tile(src, n, tileBase, t, lds, 0ull);      // its barrier also orders the clearing
+  run_words(n, tileBase, t, lrun);
+  const uint32_t prefix = lb_exclusive(p, tile, t.agg, lds);   // its barriers also order the words
+  inner_write(src, n, tileBase, t, prefix, lrun, rec, pcode, sc);
+}
+// In two passes, after k_run_count and its scan, as k_leaf_scanned.
+__global__ void __launch_bounds__(kRunT) k_inner_scanned(const uint64_t* __restrict__ ccode, uint64_t n,
+                                                         const uint32_t* __restrict__ before,
+                                                         uint32_t* __restrict__ rec, uint64_t* __restrict__ pcode,
+                                                         SceneOut sc) {
+  __shared__ uint32_t lds[kRunT / 64];
+  __shared__ uint32_t lrun[kScanTile];
+  const uint64_t tileBase = (uint64_t)blockIdx.x * kScanTile;
+  for (uint32_t j = threadIdx.x; j < kScanTile; j += kRunT) lrun[j] = 0;
+  RunTile<kScanPer> t;
+  PlainCodes src{ccode};
+  run_tile(src, n, tileBase, t, lds, 0ull);
+  run_words(n, tileBase, t, lrun);
+  const uint32_t prefix = before[blockIdx.x];
   __syncthreads();
-  const uint64_t tileEnd = tileBase + kInnerTile;
-#pragma unroll
-  for (int k = 0; k < kInnerPer; ++k) {
-    if (!((t.heads >> k) & 1u)) continue;
-    const uint32_t r = (uint32_t)t.rank[k];
-    uint32_t m = lmask[r];
-    const uint64_t pc = t.v[k] >> 3;
-    if (r + 1 == t.agg && tileEnd < n) m |= run_tail_bits(src, n, tileEnd, pc);
-    uint32_t* o = rec + (uint64_t)(prefix + r) * kRecWords;
-    o[0] = m;
-#pragma unroll
-    for (int c = 0; c < 8; ++c)
-      if (!((m >> c) & 1u)) o[1 + c] = kNull;
-    if (pcode) pcode[prefix + r] = pc;
-  }
+  inner_write(src, n, tileBase, t, prefix, lrun, rec, pcode, sc);
 }
 
-// Level counts of k_leaf_build: hist[k] = sum over tiles of part[t][k], all
-// counters in one pass over the tiles; each workgroup adds its tiles' sums
-// to hist, which k_leaf_build's first tile cleared.
-constexpr uint32_t kCountTilesPerWg = 8192;
-__global__ void __launch_bounds__(1024) k_level_counts(const uint32_t* __restrict__ part, uint32_t tiles, uint32_t L,
-                                                       uint32_t* __restrict__ hist) {
-  __shared__ uint32_t red[kMaxLevels + 1][1024 / 64];
-  uint32_t s[kMaxLevels + 1];
-#pragma unroll
-  for (int q = 0; q <= (int)kMaxLevels; ++q) s[q] = 0;
-  for (uint32_t t = blockIdx.x * 1024 + threadIdx.x; t < tiles; t += gridDim.x * 1024) {
-    const uint32_t* pt = part + (uint64_t)t * (L + 1);
-#pragma unroll
-    for (int q = 0; q <= (int)kMaxLevels; ++q)
-      if ((uint32_t)q <= L) s[q] += pt[q];
-  }
+// Level counts from the leaves' parent codes.  Leaf j starts a node q steps
+// above the leaves (prefix pcode >> 3q) exactly when q <= floor(msb(pcode[j] ^
+// pcode[j-1]) / 3), so hist[1 + q] = the leaves that reach q, hist[1] =
+// *leaves and hist[0] = the bad codes (state[0], which is cleared again).  A
+// wavefront takes 64 neighbouring leaves at a time and counts level after
+// level by ballots until none reaches on (two or three levels for most).  The
+// last of few workgroups (state[1] counts them) sums all parts.
+constexpr uint32_t kHistGrid = 256;
+__global__ void __launch_bounds__(1024) k_level_hist(const uint64_t* __restrict__ pcode,
+                                                     const uint32_t* __restrict__ leaves, uint32_t L, uint32_t* state,
+                                                     uint32_t* part, uint32_t* __restrict__ hist) {
+  __shared__ uint32_t red[1024 / 64][kMaxLevels + 1];
+  __shared__ uint32_t lastWg;
+  const uint32_t n = *leaves;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t mine = 0;                      // lane q: the leaves that reach q
+  constexpr int kChunks = 4;              // loads in flight per wavefront
+  for (uint64_t base = ((uint64_t)blockIdx.x * 16 + wave) * (64 * kChunks); base < n;
+       base += (uint64_t)gridDim.x * (1024 * kChunks)) {
+    uint64_t v[kChunks];
 #pragma unroll
-  for (int q = 0; q <= (int)kMaxLevels; ++q) {
-    uint32_t x = s[q];
+    for (int k = 0; k < kChunks; ++k) {
+      const uint64_t j = base + 64 * k + lane;
+      v[k] = j < n ? pcode[j] : 0ull;
+    }
+    uint64_t before = lane == 0 && base ? pcode[base - 1] : 0ull;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-    if (lane == 0) red[q][wave] = x;
+    for (int k = 0; k < kChunks; ++k) {
+      const uint64_t j = base + 64 * k + lane;
+      const uint64_t x = v[k] ^ lane_below(v[k], before);
+      before = last_lane(v[k]);
+      uint32_t K = 0;
+      if (j < n) K = j == 0 ? L : (x ? (uint32_t)(63 - __clzll((long long)x)) / 3u : 0u);
+      for (uint32_t q = 1; q < L; ++q) {
+        const uint64_t b = __ballot(K >= q);
+        if (!b) break;
+        if (lane == (int)q) mine += (uint32_t)__popcll(b);
+      }
+    }
+  }
+  if (lane <= (int)kMaxLevels) red[wave][lane] = mine;
+  __syncthreads();
+  if (threadIdx.x < L) {
+    uint32_t x = 0;
+    for (int w = 0; w < 1024 / 64; ++w) x += red[w][threadIdx.x];
+    __hip_atomic_store(&part[(uint64_t)blockIdx.x * kMaxLevels + threadIdx.x], x, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();
   }
   __syncthreads();
-  if (threadIdx.x <= L) {
-    uint32_t x = 0;
-    for (int v = 0; v < 1024 / 64; ++v) x += red[threadIdx.x][v];
-    atomicAdd(&hist[threadIdx.x], x);
+  if (threadIdx.x == 0) {
+    const uint32_t done = atomicAdd(&state[1], 1u);
+    lastWg = done == gridDim.x - 1 ? 1u : 0u;
+    if (lastWg) atomicExch(&state[1], 0u);
+  }
+  __syncthreads();
+  if (!lastWg) return;
+  __threadfence();
+  // lane l sums level l % 32 over every 32nd part
+  uint32_t x = 0;
+  if ((threadIdx.x & 31) < L)
+    for (uint32_t g = threadIdx.x >> 5; g < gridDim.x; g += 32)
+      x += __hip_atomic_load(&part[(uint64_t)g * kMaxLevels + (threadIdx.x & 31)], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+  x += __shfl_xor(x, 32, 64);
+  if (lane < (int)L) red[wave][lane] = x;      // red was last read before the barriers above
+  __syncthreads();
+  if (threadIdx.x < L) {
+    x = 0;
+    for (int w = 0; w < 1024 / 64; ++w) x += red[w][threadIdx.x];
+    hist[1 + threadIdx.x] = threadIdx.x ? x : n;
+    if (threadIdx.x == 0) hist[0] = atomicExch(&state[0], 0u);
   }
 }
 
@@ -1349,15 +1442,15 @@ __global__ void __launch_bounds__(256) k_sdag_leaves(const uint32_t* __restrict_
   }
 }
 
-// The scene s of code t * kLeafTile (the last s with off[s] <= it; every
+// The scene s of code t * tileSize (the last s with off[s] <= it; every
 // scene holds at least one code, so off ascends strictly), as 8 words per
 // tile: off[s], off[s + 1], off[s + 2] (64-bit, low word first; off[S] past
 // the last scene), s, 3 * levels[s] | 3 * levels[s + 1] << 8.
 __global__ void k_tile_scenes(const uint64_t* __restrict__ off, const uint32_t* __restrict__ levels, uint32_t S,
-                              uint64_t tiles, uint32_t* __restrict__ tileScene) {
+                              uint64_t tiles, uint32_t tileSize, uint32_t* __restrict__ tileScene) {
   const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= tiles) return;
-  const uint64_t i = t * kLeafTile;
+  const uint64_t i = t * tileSize;
   uint32_t lo = 0, hi = S;
   while (hi - lo > 1) {
     const uint32_t mid = (lo + hi) >> 1;
@@ -1413,13 +1506,6 @@ void build_svo_from_morton(svd_octree* o, const uint64_t* dcodes, uint64_t n) {
 uint64_t svo_inner_levels(svd_ctx* c, uint64_t* codeA, uint64_t nc, uint32_t L, std::vector<Level>& svo,
                           std::vector<uint32_t*>* levelScenes, const uint64_t* sizes) {
   uint64_t* codeB = dalloc<uint64_t>(c, nc ? nc : 1);
-  auto keep = [&](uint32_t lev, const uint64_t* codes, uint64_t m) {
-    if (!levelScenes) return;
-    (*levelScenes)[lev] = dalloc<uint32_t>(c, m + 1);
-    if (m)
-      k_code_scenes<<<div_up(m, kB), kB, 0, c->stream>>>(codes, m, kSceneTagShift - 3 * (L - lev),
-                                                         (*levelScenes)[lev]);
-  };
   uint64_t nNodes = 0;
   for (int lev = (int)L - 2; lev >= 0; --lev) {
     Level& lv = svo[lev];
@@ -1440,15 +1526,25 @@ uint64_t svo_inner_levels(svd_ctx* c, uint64_t* codeA, uint64_t nc, uint32_t L, 
     const uint64_t np = sizes[lev];
     lv.n = np;
     lv.rec = dalloc<uint32_t>(c, np * kRecWords);
+    SceneOut sc{nullptr, kSceneTagShift - 3 * (int)(L - lev)};
+    if (levelScenes) sc.scene = (*levelScenes)[lev] = dalloc<uint32_t>(c, np + 1);
     if (nc <= small_limit(c->smallSvo, kSvoSmall)) {
       k_inner_level_small<<<1, 1024, 0, c->stream>>>(codeA, (uint32_t)nc, lv.rec, codeB);
+      if (sc.scene && np) k_code_scenes<<<div_up(np, kB), kB, 0, c->stream>>>(codeB, np, sc.shift, sc.scene);
       check_launch("k_inner_level_small");
-    } else {
+    } else if (nc < kTwoPassCodes) {
       const uint64_t tiles = div_up(nc, kInnerTile);
-      k_inner_build<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(codeA, nc, lb_pass(c, tiles), lv.rec, codeB);
+      k_inner_build<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(codeA, nc, lb_pass(c, tiles), lv.rec, codeB, sc);
       check_launch("k_inner_build");
+    } else {
+      const uint64_t tiles = div_up(nc, kScanTile);
+      uint32_t* heads = dalloc<uint32_t>(c, tiles);
+      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(PlainCodes{codeA}, nc, 0ull, pass_counters(c) + 1, heads);
+      scan_exclusive(c, heads, heads, tiles, nullptr);
+      k_inner_scanned<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(codeA, nc, heads, lv.rec, codeB, sc);
+      check_launch("k_inner_scanned");
+      dfree(c, heads);
     }
-    keep((uint32_t)lev, codeB, lv.n);
     std::swap(codeA, codeB);
     nc = lv.n;
     if (lev > 0) nNodes += lv.n;
@@ -1471,29 +1567,44 @@ uint64_t svo_levels_from_codes(svd_ctx* c, const uint64_t* dcodes, uint64_t n, u
                                std::vector<uint32_t*>* levelScenes, uint64_t hiMask, const SceneTags* tags) {
   svo.assign(L, Level());
   if (levelScenes) levelScenes->assign(L, nullptr);
-  const uint64_t tiles = div_up(n, kLeafTile);
-  uint32_t* part = dalloc<uint32_t>(c, tiles * (L + 1));
-  uint32_t* hist = dalloc<uint32_t>(c, kMaxLevels + 1);
+  const bool scanned = n >= kTwoPassCodes;
+  const uint32_t tile = scanned ? kScanTile : kLeafTile;
+  const uint64_t tiles = div_up(n, tile);
+  uint32_t* part = dalloc<uint32_t>(c, (uint64_t)kHistGrid * kMaxLevels);
+  uint32_t* heads = scanned ? dalloc<uint32_t>(c, tiles) : nullptr;
+  uint32_t* hist = dalloc<uint32_t>(c, kMaxLevels + 2);
+  uint32_t* leaves = hist + kMaxLevels + 1;
   uint32_t* leafMask = dalloc<uint32_t>(c, n);
   uint64_t* codeA = dalloc<uint64_t>(c, n);
   uint32_t* tileScene = nullptr;
+  uint32_t* state = pass_counters(c) + 1;    // bad codes, workgroups done
+  auto finest = [&](auto src, uint64_t hi) {
+    if (scanned) {
+      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, hi, state, heads);
+      scan_exclusive(c, heads, heads, tiles, leaves);
+      k_leaf_scanned<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, heads, leafMask, codeA);
+    } else {
+      k_leaf_build<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, hi, lb_pass(c, tiles), state, leaves, leafMask,
+                                                             codeA);
+    }
+  };
   if (tags) {
     tileScene = dalloc<uint32_t>(c, 8 * tiles);
-    k_tile_scenes<<<div_up(tiles, kB), kB, 0, c->stream>>>(tags->off, tags->levels, tags->S, tiles, tileScene);
+    k_tile_scenes<<<div_up(tiles, kB), kB, 0, c->stream>>>(tags->off, tags->levels, tags->S, tiles, tile, tileScene);
     SceneTags t = *tags;
     t.tileScene = tileScene;
-    k_leaf_build<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(TaggedCodes{dcodes, t, kLeafTile}, n, L, 1ull << 63,
-                                                           lb_pass(c, tiles), part, hist, leafMask, codeA);
+    finest(TaggedCodes{dcodes, t, tile}, 1ull << 63);
   } else {
-    k_leaf_build<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(PlainCodes{dcodes}, n, L, hiMask, lb_pass(c, tiles), part,
-                                                           hist, leafMask, codeA);
+    finest(PlainCodes{dcodes}, hiMask);
   }
-  k_level_counts<<<(uint32_t)div_up(tiles, kCountTilesPerWg), 1024, 0, c->stream>>>(part, (uint32_t)tiles, L, hist);
+  const uint32_t grid = std::min<uint32_t>(kHistGrid, div_up(n, 4096));
+  k_level_hist<<<grid, 1024, 0, c->stream>>>(codeA, leaves, L, state, part, hist);
   check_launch("k_leaf_build");
   uint32_t h[kMaxLevels + 1];
   read_u32s(c, hist, h, L + 1);
   dfree(c, hist);
   dfree(c, part);
+  dfree(c, heads);
   dfree(c, tileScene);
   if (h[0]) {
     dfree(c, leafMask);

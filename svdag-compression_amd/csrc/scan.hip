@@ -131,6 +131,14 @@ void scan_exclusive2(svd_ctx* c, uint32_t* a, uint32_t* b, uint64_t n) {
   check_launch("scan_exclusive2");
 }
 
+uint32_t* pass_counters(svd_ctx* c) {
+  if (!c->lbCounter) {
+    c->lbCounter = dalloc<uint32_t>(c, 3);
+    fill_u32(c, c->lbCounter, 0u, 3);
+  }
+  return c->lbCounter;
+}
+
 LbPass lb_pass(svd_ctx* c, uint64_t tiles) {
   if (tiles >= (1ull << 31)) throw Error{SVD_ERR_CAPACITY, "single-pass scan: too many tiles"};
   bool clear = false;
@@ -140,10 +148,7 @@ LbPass lb_pass(svd_ctx* c, uint64_t tiles) {
     c->lbStatus = dalloc<unsigned long long>(c, c->lbCap);
     clear = true;
   }
-  if (!c->lbCounter) {
-    c->lbCounter = dalloc<uint32_t>(c, 1);
-    fill_u32(c, c->lbCounter, 0u, 1);
-  }
+  pass_counters(c);
   if (++c->lbEpoch >= (1u << 30)) {
     c->lbEpoch = 1;
     clear = true;

@@ -66,7 +66,7 @@ struct svd_ctx {
   hipError_t renderScratchErr = hipSuccess;  // why it is null, if it is
   unsigned long long* lbStatus = nullptr;    // single-pass scans: one published word per tile
   uint64_t lbCap = 0;                        // tiles lbStatus holds
-  uint32_t* lbCounter = nullptr;             // tile counter, zero between passes
+  uint32_t* lbCounter = nullptr;             // three counters, zero between passes (pass_counters)
   uint32_t lbEpoch = 0;                      // epoch of the last pass (words of older passes are stale)
 };
 
@@ -183,6 +183,9 @@ void read_u32s_2(svd_ctx* c, const uint32_t* d1, uint32_t* h1, size_t n1, const 
 // captured graph (its epoch would repeat).
 struct LbPass;
 LbPass lb_pass(svd_ctx* c, uint64_t tiles);
+// Device counters that every pass leaves at zero: [0] the look-back tile
+// counter, [1] bad codes and [2] finished workgroups of the leaf build.
+uint32_t* pass_counters(svd_ctx* c);
 // Exclusive prefix sum of n u32 values; out may alias in.  *total (device) gets
 // the sum (may be null).  Scratch comes from the context arena.
 void scan_exclusive(svd_ctx* c, const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* total);

@@ -86,6 +86,47 @@ def test_build_levels_and_files_bit_exact(ctx, name):
         assert got == want, f"format {fmt} differs at byte {next(i for i in range(len(got)) if got[i] != want[i])}"
 
 
+@pytest.mark.parametrize("L", [3, 6, 21])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 8191, 8192, 8193, 30011, (4 << 20) - 1, (4 << 20) + 4097])
+def test_leaf_pass_edges(ctx, n, L):
+    """The leaves from the voxel codes at the edges of a wavefront, of a tile
+    (8192 codes, with runs across its end), of several tiles and of the lists
+    that are read in two passes (from 4M codes, 4096 per tile; the sparse ones
+    have inner levels of that size too): every SVO level and the level counts
+    equal the oracle's, for dense codes (full runs) and sparse ones (every
+    code its own run)."""
+    top = 1 << (3 * L)
+    for step in (1, 3, 9973):
+        if (n - 1) * step + 5 >= top:
+            continue
+        codes = np.uint64(5) + np.arange(n, dtype=np.uint64) * np.uint64(step)
+        if L == 21 and step > 3:
+            codes = codes * np.uint64(((1 << 62) // (n * step)) | 1)
+        g, o = S.Octree.from_morton(ctx, codes, L), O.OracleOctree.from_morton(codes, L)
+        want = o.levels_words()
+        for l in range(L):
+            np.testing.assert_array_equal(g.level(S.VIEW_SVO, l), want[l], err_msg=f"level {l} step {step}")
+        assert g.counts() == (o.n_nodes, o.n_voxels)
+        g.free()
+
+
+@pytest.mark.parametrize("n,at", [(9001, 1), (9001, 64), (9001, 8191), (9001, 8192), (9001, 8193), (9001, 9000),
+                                  (4 << 20, 4095), (4 << 20, 4096), (4 << 20, (4 << 20) - 1)])
+def test_leaf_pass_rejects_bad_codes(ctx, n, at):
+    """One repeated, descending or too large code, on either side of a tile's
+    end (one pass and two), is refused; the context builds the corrected list
+    right after."""
+    good = (np.arange(n, dtype=np.uint64) + np.uint64(1)) * np.uint64(3)
+    for bad in (good[at - 1], good[at - 1] - np.uint64(1), np.uint64(1 << 30)):
+        codes = good.copy()
+        codes[at] = bad
+        with pytest.raises(S.SvdError):
+            S.Octree.from_morton(ctx, codes, 10)
+        g = S.Octree.from_morton(ctx, good, 10)
+        assert g.counts()[1] == good.size
+        g.free()
+
+
 def test_refcount_order_unfinished_batch_reruns_checked(ctx, monkeypatch):
     """The SSVDAG-layout encoder runs the refcount order's device rounds
     without reading the list size and finds out with its layout read whether
