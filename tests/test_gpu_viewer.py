@@ -139,6 +139,30 @@ def test_ao_matches_oracle(ctx, scene_files, fmt, nrays):
         assert (got[hit] < 1).any(), "no pixel is occluded"
 
 
+@pytest.mark.parametrize("size,samples,nrays", [((1, 1), 1, 1), ((17, 9), 64, 256), ((33, 47), 1, 3),
+                                                ((16, 16), 5, 64), ((70, 45), 3, 7)])
+def test_shared_out_rays_match_oracle(ctx, scene_files, size, samples, nrays):
+    """The rays that a workgroup or wavefront shares out over its lanes: fewer
+    than a wavefront, partial tiles and runs, the most rays a pixel takes, and
+    lanes that take a second ray (also with rays that end by max_iters)."""
+    import torch
+    L, files = scene_files
+    fmt = S.FMT_SSVDAG
+    for iters in (1000, 30):
+        p = W.trace_params(size[0], size[1], seed=4, levels=L, shadows=True, light=(1.0, 0.6, 1.0), max_iters=iters)
+        v = S.ViewParams.defaults(render_mode=3, norm_samples=samples, random_colors=0)
+        want, wprim = O.render_frame(files[fmt], fmt, p, v)
+        got, gprim = gpu_render(ctx, fmt, files[fmt], p, v, 0.0)
+        np.testing.assert_array_equal(gprim, wprim)
+        np.testing.assert_array_equal(got, want)
+        want, _ = O.trace_ao(files[fmt], fmt, p, nrays)
+        vis = torch.full((p.width * p.height,), float("nan"), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        S.Scene.from_bytes(ctx, fmt, files[fmt]).ao_device(p, nrays, vis.data_ptr())
+        ctx.sync()
+        np.testing.assert_array_equal(vis.cpu().numpy().reshape(p.height, p.width), want)
+
+
 def test_render_and_ao_reject_bad_arguments(ctx, scene_files):
     import torch
     L, files = scene_files
