@@ -990,8 +990,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
     check_launch("k_remap_inplace");
     clk.mark(6);
     uint64_t hs[9];
-    SVD_HIP(hipMemcpyAsync(hs, dstats, sizeof(hs), hipMemcpyDeviceToHost, c->stream));
-    SVD_HIP(hipStreamSynchronize(c->stream));
+    read_u32s(c, (const uint32_t*)dstats, (uint32_t*)hs, sizeof(hs) / 4);
     st.merged = n - kept;
     st.error_bound = hs[4];
     st.listed = hs[5];

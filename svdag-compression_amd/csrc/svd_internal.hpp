@@ -18,6 +18,7 @@ constexpr uint32_t kMaxLevels = 21;        // 3*21 = 63 Morton bits
 // svd_render_noalloc: texels of its static depth pre-pass texture (512 KiB),
 // enough for (width / 8) * (height / 8) of frames up to 4096 x 2048 or 3840 x 2160
 constexpr uint64_t kRenderScratchTexels = 131072;
+constexpr size_t kStageWords = 2048;       // words one size read-back brings over
 
 struct Error {
   int code;
@@ -45,7 +46,9 @@ struct svd_ctx {
   hipStream_t stream = nullptr;
   std::string err;
   svd::Arena* arena = nullptr;
-  uint64_t* pinned = nullptr;                // small pinned staging for size read-backs
+  uint64_t* pinned = nullptr;                // pinned staging for size read-backs: kStageWords words, a flag word
+  uint32_t* pinnedDev = nullptr;             // its device address
+  uint32_t readSeq = 0;                      // value of the flag word after the last read-back
   hipEvent_t ev[2] = {nullptr, nullptr};
   // per timed family: events around its last call (the elapsed time is read
   // when asked for, so a call need not wait for its own kernels)
