@@ -25,7 +25,8 @@ namespace {
 constexpr int kThreshold = 16;
 constexpr int kLdsN = 2048;           // segments up to this size finish in one workgroup
 constexpr int kBT = 256;              // threads per workgroup
-constexpr int kPer = kLdsN / kBT;     // elements per thread in the workgroup phase
+constexpr int kSortT = 512;           // threads per workgroup in the workgroup phase
+constexpr int kPer = kLdsN / kSortT;  // elements per thread in the workgroup phase
 constexpr int kTile = 2048;           // elements per workgroup in the device-wide rounds
 constexpr uint32_t kLeafTag = 0x8000u; // workgroup phase: segOf tags
 constexpr uint32_t kEqTag = 0xC000u;
@@ -377,7 +378,12 @@ __global__ void k_heap_sort(const Seg* __restrict__ segs, const uint32_t* __rest
 
 // ---------------------------------------------------------------- workgroup phase
 // One workgroup runs the complete introsort recursion of one segment of
-// 17..2048 elements in LDS, all subsegments of one depth together.
+// 17..2048 elements in LDS, all subsegments of one depth together.  The
+// recursion is a chain of barriers, so the longest segment bounds the launch:
+// eight wavefronts with four elements per thread took 52 us on the segments of
+// a 2048^3 terrain (29 us on the single one of a 64^3 scene), four with eight
+// 75 (42).  Segments of up to 4096 elements in sixteen wavefronts save one
+// device-wide round of 28 us but took 71 us (36).
 // Introsort of a segment of s equal values with depth budget d.  The median
 // of three is the middle element B = f + s/2 (no comparison holds), so the
 // front and B swap; every element stops both scanners, so the partition
@@ -417,9 +423,9 @@ __device__ __forceinline__ uint32_t blk_elem(int tid, int k) {
   return (uint32_t)((tid >> 6) * (64 * kPer) + 64 * k + (tid & 63));
 }
 
-__global__ void __launch_bounds__(kBT) k_block_sort(const Seg* __restrict__ segs, const uint32_t* __restrict__ nsp,
+__global__ void __launch_bounds__(kSortT) k_block_sort(const Seg* __restrict__ segs, const uint32_t* __restrict__ nsp,
                                                     uint32_t* val, uint32_t* idx) {
-  constexpr int kWaves = kBT / 64;
+  constexpr int kWaves = kSortT / 64;
   __shared__ uint32_t sv[kLdsN], si[kLdsN];
   __shared__ uint16_t segOf[kLdsN];
   __shared__ uint16_t exL[kLdsN + 1], exR[kLdsN + 1];
@@ -443,7 +449,7 @@ __global__ void __launch_bounds__(kBT) k_block_sort(const Seg* __restrict__ segs
   const int tid = threadIdx.x, wv = tid >> 6;
   const uint32_t v0 = val[g.first];
   bool differs = false;
-  for (uint32_t k = tid; k < n; k += kBT) {
+  for (uint32_t k = tid; k < n; k += kSortT) {
     sv[k] = val[g.first + k];
     si[k] = idx[g.first + k];
     segOf[k] = 0;
@@ -451,7 +457,7 @@ __global__ void __launch_bounds__(kBT) k_block_sort(const Seg* __restrict__ segs
   }
   if (!__syncthreads_or(differs) && eq_depth_ok(n, g.depth)) {
     // all values equal: only the indices move, each straight to its place
-    for (uint32_t k = tid; k < n; k += kBT) idx[g.first + eq_dest(k, n)] = si[k];
+    for (uint32_t k = tid; k < n; k += kSortT) idx[g.first + eq_dest(k, n)] = si[k];
     __syncthreads();   // the next segment reuses the LDS arrays
     continue;
   }
@@ -710,7 +716,7 @@ __global__ void __launch_bounds__(kBT) k_block_sort(const Seg* __restrict__ segs
   for (int k = 0; k < kPer; ++k)
     if (rp[k] != kDone) { sv[rp[k]] = rv[k]; si[rp[k]] = ri[k]; }
   __syncthreads();
-  for (uint32_t k = tid; k < n; k += kBT) { val[g.first + k] = sv[k]; idx[g.first + k] = si[k]; }
+  for (uint32_t k = tid; k < n; k += kSortT) { val[g.first + k] = sv[k]; idx[g.first + k] = si[k]; }
   __syncthreads();   // the next segment reuses the LDS arrays
   }
 }
@@ -835,7 +841,7 @@ void refsort_ranges(svd_ctx* c, uint32_t* idx, uint32_t* val, uint64_t n, const 
     dfree(c, Lpos); dfree(c, Rpos); dfree(c, st); dfree(c, blk0); dfree(c, cntL); dfree(c, cntR);
   }
   // finishers, sized without reading the list lengths (grid-stride)
-  k_block_sort<<<(uint32_t)std::max(c->numCU, 1) * 3, kBT, 0, c->stream>>>(L.small, L.nsmall, val, idx);
+  k_block_sort<<<(uint32_t)std::max(c->numCU, 1) * 3, kSortT, 0, c->stream>>>(L.small, L.nsmall, val, idx);
   k_heap_sort<<<64, 64, 0, c->stream>>>(L.heap, L.nheap, val, idx);
   k_leaf_sort<<<512, 64, 0, c->stream>>>(L.leaf, L.nleaf, val, idx);
   check_launch("refsort finish");
