@@ -179,8 +179,8 @@ __device__ __forceinline__ uint32_t run_tail_bits(const Src& code, uint64_t n, u
 // Input contract: strictly ascending codes with no bit of hiMask set (plain
 // codes: every bit from 3 * levels up; scene-tagged codes: bit 63, which
 // TaggedCodes sets on a code beyond its scene's depth).
-// A batch's node scenes as a level is written: scene[i] = parent code >> shift
-// (none when null).
+// A batch's node scenes as a pass holds their codes: scene[i] = code of node i
+// >> shift (none when null).
 struct SceneOut { uint32_t* scene; int shift; };
 
 // The finest level: the leaf masks and parent codes of the runs that start in
@@ -253,13 +253,18 @@ constexpr int kScanPer = 8;
 constexpr uint32_t kScanTile = kRunT * kScanPer;
 template <typename Src>
 __global__ void __launch_bounds__(kRunT) k_run_count(Src src, uint64_t n, uint64_t hiMask, uint32_t* bad,
-                                                     uint32_t* __restrict__ heads) {
+                                                     uint32_t* __restrict__ heads, SceneOut sc) {
   __shared__ uint32_t lds[kRunT / 64];
   Src code = src;
   RunTile<kScanPer> t;
   run_tile(code, n, (uint64_t)blockIdx.x * kScanTile, t, lds, hiMask);
   if (t.bad) atomicAdd(bad, t.bad);
   if (threadIdx.x == 0) heads[blockIdx.x] = t.agg;
+  if (!sc.scene) return;               // the codes' own scenes, while they are here
+  const uint64_t at = (uint64_t)blockIdx.x * kScanTile + (threadIdx.x >> 6) * (64 * kScanPer) + (threadIdx.x & 63);
+#pragma unroll
+  for (int k = 0; k < kScanPer; ++k)
+    if (at + 64 * k < n) sc.scene[at + 64 * k] = (uint32_t)(t.v[k] >> sc.shift);
 }
 template <typename Src>
 __global__ void __launch_bounds__(kRunT) k_leaf_scanned(Src src, uint64_t n, const uint32_t* __restrict__ before,
@@ -366,7 +371,7 @@ __global__ void __launch_bounds__(kRunT) k_inner_scanned(const uint64_t* __restr
 // wavefront takes 64 neighbouring leaves at a time and counts level after
 // level by ballots until none reaches on (two or three levels for most).  The
 // last of few workgroups (state[1] counts them) sums all parts.
-constexpr uint32_t kHistGrid = 256;
+constexpr uint32_t kHistGrid = 512;
 __global__ void __launch_bounds__(1024) k_level_hist(const uint64_t* __restrict__ pcode,
                                                      const uint32_t* __restrict__ leaves, uint32_t L, uint32_t* state,
                                                      uint32_t* part, uint32_t* __restrict__ hist) {
@@ -804,27 +809,30 @@ __global__ void __launch_bounds__(kSmallThreads) k_dedup_levels_small(DagTop a) 
 // pos[i] = number of representatives before node i (scan_op): a node is its
 // key's representative when the table slot holds its own index.
 struct RepFlagOp {
-  const uint32_t* __restrict__ slot;
+  uint32_t* __restrict__ slot;   // table slot, replaced by the representative's index
   const TEntry* __restrict__ table;
   uint32_t* __restrict__ pos;
   __device__ uint32_t value(uint64_t i, uint32_t&) const {
     const uint32_t s = slot[i];
-    return (s != kNone && entry_index(table[s]) == (uint32_t)i) ? 1u : 0u;
+    if (s == kNone) return 0u;
+    const uint32_t r = entry_index(table[s]);
+    slot[i] = r;                 // saves k_compact a second random read of the table
+    return r == (uint32_t)i ? 1u : 0u;
   }
   __device__ void apply(uint64_t i, uint32_t ex) const { pos[i] = ex; }
   __device__ void report(uint32_t) const {}
 };
 
-__global__ void k_compact(const uint32_t* __restrict__ rec, const uint32_t* __restrict__ slot,
-                          const TEntry* __restrict__ table, const uint32_t* __restrict__ pos, uint64_t n,
-                          uint32_t* __restrict__ out, uint32_t* __restrict__ remap) {
+// repOf[i]: node i's representative (kNone for an empty node)
+__global__ void k_compact(const uint32_t* __restrict__ rec, const uint32_t* __restrict__ repOf,
+                          const uint32_t* __restrict__ pos, uint64_t n, uint32_t* __restrict__ out,
+                          uint32_t* __restrict__ remap) {
   uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const uint32_t s = slot[i];
+  const uint32_t r = repOf[i];
   // an empty (skipped) node keeps correspondence 0, like the reference's
   // zero-initialised correspondences vector (geom_octree.cpp:489-495)
-  if (s == kNone) { remap[i] = 0; return; }
-  const uint32_t r = entry_index(table[s]);
+  if (r == kNone) { remap[i] = 0; return; }
   remap[i] = pos[r];
   if (r == (uint32_t)i) {
     const uint32_t* src = rec + i * kRecWords;
@@ -858,20 +866,28 @@ __global__ void k_remap_children(const uint32_t* __restrict__ in, uint64_t n, co
 // Each block folds a contiguous chunk of masks into an LDS table first, so the
 // global table sees at most 255 atomics per block instead of one per node
 // (all nodes hit the same 255 addresses).
-constexpr int kFoBlocks = 1024;
-__global__ void __launch_bounds__(256) k_leaf_firstocc(const uint32_t* __restrict__ mask, uint64_t n,
-                                                       uint32_t* __restrict__ firstocc) {
+// 256 blocks of 1024: the global atomics on one mask serialise at 11 ns each,
+// and eight masks in flight per thread hide the loads (3.9M masks: 26 -> 13 us).
+constexpr int kFoBlocks = 256, kFoT = 1024;
+__global__ void __launch_bounds__(kFoT) k_leaf_firstocc(const uint32_t* __restrict__ mask, uint64_t n,
+                                                        uint32_t* __restrict__ firstocc) {
   __shared__ uint32_t fo[256];
-  fo[threadIdx.x] = kNone;
+  if (threadIdx.x < 256) fo[threadIdx.x] = kNone;
   __syncthreads();
   const uint64_t chunk = (n + gridDim.x - 1) / gridDim.x;
   const uint64_t lo = (uint64_t)blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
-  for (uint64_t i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    const uint32_t m = mask[i] & 0xFFu;
-    if (m && fo[m] > (uint32_t)i) atomicMin(&fo[m], (uint32_t)i);
+  for (uint64_t i0 = lo + threadIdx.x; i0 < hi; i0 += 8 * kFoT) {
+    uint32_t m[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m[k] = i0 + k * kFoT < hi ? mask[i0 + k * kFoT] & 0xFFu : 0u;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t i = (uint32_t)(i0 + k * kFoT);
+      if (m[k] && fo[m[k]] > i) atomicMin(&fo[m[k]], i);
+    }
   }
   __syncthreads();
-  const uint32_t v = fo[threadIdx.x];
+  const uint32_t v = threadIdx.x < 256 ? fo[threadIdx.x] : kNone;
   if (v != kNone) atomicMin(&firstocc[threadIdx.x], v);
 }
 
@@ -1539,7 +1555,10 @@ uint64_t svo_inner_levels(svd_ctx* c, uint64_t* codeA, uint64_t nc, uint32_t L, 
     } else {
       const uint64_t tiles = div_up(nc, kScanTile);
       uint32_t* heads = dalloc<uint32_t>(c, tiles);
-      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(PlainCodes{codeA}, nc, 0ull, pass_counters(c) + 1, heads);
+      // the leaves' scenes come with the first pass over their codes
+      const SceneOut own{levelScenes && lev == (int)L - 2 ? (*levelScenes)[L - 1] : nullptr, kSceneTagShift - 3};
+      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(PlainCodes{codeA}, nc, 0ull, pass_counters(c) + 1, heads,
+                                                            own);
       scan_exclusive(c, heads, heads, tiles, nullptr);
       k_inner_scanned<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(codeA, nc, heads, lv.rec, codeB, sc);
       check_launch("k_inner_scanned");
@@ -1580,7 +1599,7 @@ uint64_t svo_levels_from_codes(svd_ctx* c, const uint64_t* dcodes, uint64_t n, u
   uint32_t* state = pass_counters(c) + 1;    // bad codes, workgroups done
   auto finest = [&](auto src, uint64_t hi) {
     if (scanned) {
-      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, hi, state, heads);
+      k_run_count<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, hi, state, heads, SceneOut{nullptr, 0});
       scan_exclusive(c, heads, heads, tiles, leaves);
       k_leaf_scanned<<<(uint32_t)tiles, kRunT, 0, c->stream>>>(src, n, heads, leafMask, codeA);
     } else {
@@ -1597,7 +1616,9 @@ uint64_t svo_levels_from_codes(svd_ctx* c, const uint64_t* dcodes, uint64_t n, u
   } else {
     finest(PlainCodes{dcodes}, hiMask);
   }
-  const uint32_t grid = std::min<uint32_t>(kHistGrid, div_up(n, 4096));
+  // Half the workgroups below 64M codes: each counts itself done at one
+  // address (13.7M codes: 22 us with 256, 27 with 512; 463M: 282 and 241).
+  const uint32_t grid = std::min<uint32_t>(n < (64ull << 20) ? kHistGrid / 2 : kHistGrid, div_up(n, 4096));
   k_level_hist<<<grid, 1024, 0, c->stream>>>(codeA, leaves, L, state, part, hist);
   check_launch("k_leaf_build");
   uint32_t h[kMaxLevels + 1];
@@ -1621,7 +1642,9 @@ uint64_t svo_levels_from_codes(svd_ctx* c, const uint64_t* dcodes, uint64_t n, u
   leaf.rec = leafMask;
   if (levelScenes) {
     (*levelScenes)[L - 1] = dalloc<uint32_t>(c, leaf.n + 1);
-    k_code_scenes<<<div_up(leaf.n, kB), kB, 0, c->stream>>>(codeA, leaf.n, kSceneTagShift - 3, (*levelScenes)[L - 1]);
+    if (L < 2 || leaf.n < kTwoPassCodes)       // else by the level above's first pass
+      k_code_scenes<<<div_up(leaf.n, kB), kB, 0, c->stream>>>(codeA, leaf.n, kSceneTagShift - 3,
+                                                              (*levelScenes)[L - 1]);
   }
   const uint64_t nNodes = (L >= 2) ? leaf.n : 0;
   return nNodes + svo_inner_levels(c, codeA, leaf.n, L, svo, levelScenes, sizes.data());
@@ -1648,7 +1671,7 @@ void dedup_level_dev(svd_ctx* c, const uint32_t* rec, uint64_t n, uint32_t* rema
   check_launch("k_insert");
   scan_op<4>(c, n, RepFlagOp{slot, table, pos}, total);
   uint32_t* out = dalloc<uint32_t>(c, (n ? n : 1) * kRecWords);
-  k_compact<<<div_up(n, kB), kB, 0, c->stream>>>(rec, slot, table, pos, n, out, remap);
+  k_compact<<<div_up(n, kB), kB, 0, c->stream>>>(rec, slot, pos, n, out, remap);
   check_launch("k_compact");
   dfree(c, table); dfree(c, slot); dfree(c, pos);
   *outRec = out;
@@ -1686,8 +1709,8 @@ uint64_t dedup_all(svd_ctx* c, uint32_t L, const std::vector<Level>& src, std::v
     dl.rec = dalloc<uint32_t>(c, 256);
     fill_u32(c, firstocc, kNone, 256);
     if (sl.n) {
-      const uint64_t nb = div_up(sl.n, 256) < (uint64_t)kFoBlocks ? div_up(sl.n, 256) : (uint64_t)kFoBlocks;
-      k_leaf_firstocc<<<nb, 256, 0, c->stream>>>(sl.rec, sl.n, firstocc);
+      const uint64_t nb = div_up(sl.n, kFoT) < (uint64_t)kFoBlocks ? div_up(sl.n, kFoT) : (uint64_t)kFoBlocks;
+      k_leaf_firstocc<<<nb, kFoT, 0, c->stream>>>(sl.rec, sl.n, firstocc);
     }
     k_leaf_rank<<<1, 256, 0, c->stream>>>(firstocc, idOfMask, dl.rec, counts + (L - 1));
     if (sl.n) k_leaf_remap<<<div_up(sl.n, kB), kB, 0, c->stream>>>(sl.rec, sl.n, idOfMask, remap);
