@@ -631,11 +631,13 @@ constexpr uint64_t kStRep = (uint64_t)kRep << 32, kStMerged = (uint64_t)kMerged 
 
 __global__ void __launch_bounds__(256) k_resolve_init(uint64_t n, const uint64_t* __restrict__ refs, uint64_t maxRefs,
                                                       unsigned long long* __restrict__ st,
+                                                      uint32_t* __restrict__ tdist,
                                                       unsigned long long* __restrict__ stats) {
   unsigned long long cands = 0;
   for (uint64_t j = (uint64_t)blockIdx.x * 256 + threadIdx.x; j < n; j += (uint64_t)gridDim.x * 256) {
     const bool cand = refs[j] <= maxRefs;
     st[j] = cand ? (unsigned long long)kUnres << 32 : (unsigned long long)(kStRep | j);
+    tdist[j] = 0;              // the walk's place in the list while j is unresolved
     cands += cand ? 1 : 0;
   }
   add_block(cands, 0, &stats[2], &stats[2]);
@@ -646,7 +648,10 @@ __global__ void __launch_bounds__(256) k_resolve_init(uint64_t n, const uint64_t
 // target (a representative), taken when the exact difference to j is within
 // the bound; an unresolved entry makes j wait.  States only move away from
 // "unresolved", so a stale read delays a node by one round and never changes
-// its outcome.  *unresolved is set while a node waits.
+// its outcome, and an entry that was passed over stays passed over: j resumes
+// where it waited (tdist[j] holds that place until j has its target).  The
+// longest walk of dependent reads bounds a round, so four entries are read at a
+// time, with (D == 0) the targets' occupancies.  *unresolved is set while a node waits.
 template <int D>
 __global__ void k_resolve(LevelView v, uint32_t lev, const uint32_t* __restrict__ lists,
                           const uint32_t* __restrict__ dv, const uint32_t* __restrict__ counts, uint64_t n,
@@ -655,30 +660,56 @@ __global__ void k_resolve(LevelView v, uint32_t lev, const uint32_t* __restrict_
   uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   if ((__atomic_load_n(&st[j], __ATOMIC_RELAXED) >> 32) != kUnres) return;
+  constexpr uint32_t kAhead = 4;
   const uint32_t cnt = counts[j];
-  for (uint32_t t = 0; t < cnt; ++t) {
-    const uint64_t e = j * cap + t;
-    if (dv[e] > bound) continue;
-    const uint32_t i = lists[e];
-    const unsigned long long w = __atomic_load_n(&st[i], __ATOMIC_RELAXED);
-    const uint32_t s = (uint32_t)(w >> 32);
-    if (s == kRep) {
-      tdist[j] = dv[e];
-      __atomic_store_n(&st[j], (unsigned long long)(kStMerged | i), __ATOMIC_RELAXED);
-      return;
+  uint32_t own[16];
+  if constexpr (D == 0) {
+    const uint4* o = reinterpret_cast<const uint4*>(v.occ + j * 16);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) { const uint4 x = o[q]; own[4 * q] = x.x; own[4 * q + 1] = x.y; own[4 * q + 2] = x.z; own[4 * q + 3] = x.w; }
+  }
+  for (uint32_t t = tdist[j]; t < cnt; t += kAhead) {
+    uint32_t dd[kAhead], ii[kAhead];
+    unsigned long long ww[kAhead];
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; ++k) {
+      const uint64_t e = j * cap + min(t + k, cnt - 1);
+      dd[k] = dv[e];
+      ii[k] = lists[e];
     }
-    if (s == kMerged) {
-      const uint32_t r = (uint32_t)w;
-      const uint32_t d = subtree_diff<D>(v, lev, r, (uint32_t)j, bound);
-      if (d <= bound) {
-        tdist[j] = d;
-        __atomic_store_n(&st[j], (unsigned long long)(kStMerged | r), __ATOMIC_RELAXED);
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; ++k) ww[k] = __atomic_load_n(&st[ii[k]], __ATOMIC_RELAXED);
+    uint32_t td[kAhead];               // D == 0: differences to the targets of entries that merged
+    if constexpr (D == 0) {
+#pragma unroll
+      for (uint32_t k = 0; k < kAhead; ++k) {
+        const bool m = t + k < cnt && dd[k] <= bound && (uint32_t)(ww[k] >> 32) == kMerged;
+        td[k] = hamming512(reinterpret_cast<const uint4*>(v.occ + (m ? (uint64_t)(uint32_t)ww[k] : j) * 16), own);
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kAhead; ++k) {
+      if (t + k >= cnt || dd[k] > bound) continue;
+      const uint32_t s = (uint32_t)(ww[k] >> 32);
+      if (s == kUnres) {
+        tdist[j] = t + k;
+        // one address: a store from every wavefront with a waiting node took
+        // most of a round (466K nodes: 256 us, looked at first 49)
+        if (!__hip_atomic_load(unresolved, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+          __hip_atomic_store(unresolved, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
       }
-      continue;
+      uint32_t r = ii[k], d = dd[k];
+      if (s == kMerged) {
+        r = (uint32_t)ww[k];
+        if constexpr (D == 0) d = td[k];
+        else d = subtree_diff<D>(v, lev, r, (uint32_t)j, bound);
+        if (d > bound) continue;
+      }
+      tdist[j] = d;
+      __atomic_store_n(&st[j], (unsigned long long)(kStMerged | r), __ATOMIC_RELAXED);
+      return;
     }
-    __atomic_store_n(unresolved, 1u, __ATOMIC_RELAXED);
-    return;
   }
   __atomic_store_n(&st[j], (unsigned long long)(kStRep | j), __ATOMIC_RELAXED);
 }
@@ -963,7 +994,7 @@ void lossy_merge(svd_octree* o, const svd_lossy_params* p, std::vector<svd_lossy
                                                                  dstats + 5);
       check_launch("k_verify");
       clk.mark(5);
-      if (n) k_resolve_init<<<grid(n), 256, 0, c->stream>>>(n, refs[lev], maxRefs, state, dstats + 5);
+      if (n) k_resolve_init<<<grid(n), 256, 0, c->stream>>>(n, refs[lev], maxRefs, state, tdist, dstats + 5);
       check_launch("k_resolve_init");
       // kRounds rounds between looks: a round over settled nodes costs less
       // than a read-back (2 to 6 rounds settle the levels measured)
