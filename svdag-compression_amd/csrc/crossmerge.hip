@@ -112,7 +112,8 @@ __device__ __forceinline__ uint32_t class_of(const LevelPtrs& P, uint32_t lev, u
   return cls ? cls[i] : node_mask(P, lev, i);
 }
 
-// bestOf[class] = min over the nodes of levels 1..top of (level << 32 | index)
+// bestOf[class] = min over the nodes of levels 1..top of (level << 32 | index),
+// at a depth with class numbers (from 1)
 __global__ void k_class_best(LevelPtrs P, uint32_t top, const uint32_t* __restrict__ cls,
                              unsigned long long* __restrict__ bestOf) {
   const uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -120,8 +121,31 @@ __global__ void k_class_best(LevelPtrs P, uint32_t top, const uint32_t* __restri
   uint32_t j;
   const uint32_t levB = level_of(P, e + P.base[1], 1, top, j);
   const unsigned long long key = ((unsigned long long)levB << 32) | j;
-  unsigned long long* b = &bestOf[cls ? cls[e] : node_mask(P, levB, j)];
+  unsigned long long* b = &bestOf[cls[e]];
   if (key < __atomic_load_n(b, __ATOMIC_RELAXED)) atomicMin(b, key);
+}
+
+// The same at depth 0, where the class is the node's mask: folded in LDS
+// first, as tens of thousands of nodes share a mask and the atomics of one
+// address serialise (395K nodes: 142 us one by one, 8 so).
+constexpr int kMaskBestT = 1024, kMaskBestGrid = 256;
+__global__ void __launch_bounds__(kMaskBestT) k_mask_best(LevelPtrs P, uint32_t top,
+                                                          unsigned long long* __restrict__ bestOf) {
+  __shared__ unsigned long long fo[256];
+  if (threadIdx.x < 256) fo[threadIdx.x] = ~0ull;
+  __syncthreads();
+  const uint64_t n = P.base[top + 1] - P.base[1], chunk = (n + gridDim.x - 1) / gridDim.x;
+  const uint64_t lo = blockIdx.x * chunk, hi = lo + chunk < n ? lo + chunk : n;
+  for (uint64_t e = lo + threadIdx.x; e < hi; e += kMaskBestT) {
+    uint32_t j;
+    const uint32_t levB = level_of(P, e + P.base[1], 1, top, j);
+    const unsigned long long key = ((unsigned long long)levB << 32) | j;
+    unsigned long long* b = &fo[node_mask(P, levB, j)];
+    if (key < *b) atomicMin(b, key);
+  }
+  __syncthreads();
+  const unsigned long long v = threadIdx.x < 256 ? fo[threadIdx.x] : ~0ull;
+  if (v != ~0ull) atomicMin(&bestOf[threadIdx.x], v);
 }
 
 // Frontier nodes of levA take their class's first match; matched ones start
@@ -138,7 +162,10 @@ __global__ void k_frontier_best(LevelPtrs P, uint32_t levA, const uint8_t* __res
   sa[a] = b != ~0ull ? a : kNone;
   sp[a] = 0;
   sb[a] = b;
-  if (b != ~0ull) __atomic_store_n(nMatched, 1u, __ATOMIC_RELAXED);   // any match: the levels below are recorded
+  // any match: the levels below are recorded (looked at first: stores of every
+  // matched wavefront to the one address took up to half of the pass)
+  if (b != ~0ull && !__hip_atomic_load(nMatched, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    __hip_atomic_store(nMatched, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // One level of the recording pass: children (level lev+1) of recorded nodes.
@@ -342,7 +369,10 @@ void cross_level_merge(svd_octree* o) {
     k_fill64<<<div_up(capOf[D], kB), kB, 0, c->stream>>>((uint64_t*)bestOf, ~0ull, capOf[D]);
     const uint32_t* cl = D ? cls[D] : nullptr;
     const uint64_t nb = nodes(levA - 1);
-    if (nb) k_class_best<<<div_up(nb, kB), kB, 0, c->stream>>>(P, levA - 1, cl, bestOf);
+    if (nb && cl) k_class_best<<<div_up(nb, kB), kB, 0, c->stream>>>(P, levA - 1, cl, bestOf);
+    else if (nb)
+      k_mask_best<<<(uint32_t)std::min<uint64_t>(kMaskBestGrid, div_up(nb, kMaskBestT)), kMaskBestT, 0, c->stream>>>(
+          P, levA - 1, bestOf);
     k_frontier_best<<<div_up(nA, kB), kB, 0, c->stream>>>(P, levA, front + bA, cl ? cl + (bA - P.base[1]) : nullptr,
                                                             bestOf, best, sa + bA, sp + bA, cand + bA, matched + levA);
     check_launch("k_frontier_best");
