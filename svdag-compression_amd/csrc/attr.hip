@@ -126,11 +126,11 @@ __device__ __forceinline__ void walk_chunk(uint64_t mask, uint32_t hc, Put& put)
   }
 }
 
-// The bits walk_chunk puts, without the walk (which took a count 61 us over 5.8M
-// attributes, with this 21; emission 142 and 92).  A node is emitted under a mixed parent, so
-// height h emits twice the mixed nodes of height h + 1; a mixed node takes one
-// bit, a uniform one two, an element one.  A group of 2^h elements is mixed when
-// two neighbours in it differ.
+// The bits walk_chunk puts, without the walk (which took a count 61 us over
+// 5.8M attributes, with this 21; emission 142 and 92).  A node is emitted
+// under a mixed parent, so height h emits twice the mixed nodes of height
+// h + 1; a mixed node takes one bit, a uniform one two, an element one.  A
+// group of 2^h elements is mixed when two neighbours in it differ.
 __device__ __forceinline__ uint32_t chunk_bits(uint64_t mask, uint32_t hc) {
   if (hc == 0) return 1u;
   if (mask == 0 || mask == chunk_full(hc)) return 2u;
