@@ -47,12 +47,39 @@ __global__ void k_put_batch(PutBatch p) {
 }
 
 // ---------------------------------------------------------------- SVDAG / USSVDAG
-__global__ void k_word_counts(LevelSet a, uint64_t n, uint32_t* __restrict__ out) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t l = level_of(a, i);
-  const uint64_t j = i - a.start[l];
-  out[i] = ((a.leafBits >> l) & 1u) ? 1u : 1u + (uint32_t)__popc(a.rec[l][j * kRecWords] & 0xFFu);
+// One or two formats side by side: their sizes, scanned, in one launch and
+// their words in another.  A launch costs more than its work on small scenes:
+// with three per format a 64^3 build took 390 us, so 361 (2048^3 terrain 1621 and
+// 1555, of which 15 us are the pointers read before a node's first store).
+struct WordJobs {
+  LevelSet a[2];
+  uint64_t n[2];                     // nodes
+  uint32_t* ptrs[2];                 // first word of every node
+  uint32_t* words[2];                // the image's words
+  uint32_t* cnt[2];                  // the header's two count words
+  uint32_t* dev;                     // per format: word count, error flags
+  int ussv[2];
+  uint32_t T0;                       // scan tiles / workgroups of the first format
+};
+struct WordCountOp {
+  const LevelSet& a;
+  uint32_t* __restrict__ ptrs;
+  __device__ uint32_t value(uint64_t i, uint32_t&) const {
+    const uint32_t l = level_of(a, i);
+    const uint64_t j = i - a.start[l];
+    return ((a.leafBits >> l) & 1u) ? 1u : 1u + (uint32_t)__popc(a.rec[l][j * kRecWords] & 0xFFu);
+  }
+  __device__ void report(uint32_t) const {}
+  __device__ void apply(uint64_t i, uint32_t ex) const { ptrs[i] = ex; }
+};
+constexpr int kWordPer = 4;
+__global__ void __launch_bounds__(kScanOpT) k_word_scan(WordJobs jb, LbPass p) {
+  __shared__ uint32_t lds[kScanOpT / 64 + 2];
+  __shared__ uint32_t word;
+  const uint32_t tile = __builtin_amdgcn_readfirstlane(lb_take_tile(p, &word));
+  const uint32_t s = tile >= jb.T0 ? 1u : 0u;      // uniform: the job is read from the kernel arguments
+  scan_tile<kWordPer>(jb.n[s], p, tile, s ? jb.T0 : 0u, s ? p.tiles - 1 : jb.T0 - 1, WordCountOp{jb.a[s], jb.ptrs[s]},
+                      jb.dev + 2 * s, lds);
 }
 
 // ussv = 0: header word = mask; child pointers follow childLevels
@@ -61,12 +88,17 @@ __global__ void k_word_counts(LevelSet a, uint64_t n, uint32_t* __restrict__ out
 //           next level (childLevels ignored, encoded_ussvdag.cpp:137).
 // The header's two count words (_firstLeafPtr and the array length, both =
 // the word count *total, see encode_words) go to cnt from thread 0.
-__global__ void k_write_words(LevelSet a, int ussv, const uint32_t* __restrict__ truePtrs, uint64_t totalNodes,
-                              uint32_t* __restrict__ words, uint32_t* __restrict__ err,
-                              const uint32_t* __restrict__ total, uint32_t* __restrict__ cnt) {
-  uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) cnt[0] = cnt[1] = *total;
+__global__ void k_write_words(WordJobs jb) {
+  const uint32_t s = blockIdx.x >= jb.T0 ? 1u : 0u;
+  const LevelSet& a = jb.a[s];
+  const int ussv = jb.ussv[s];
+  const uint32_t* __restrict__ truePtrs = jb.ptrs[s];
+  const uint64_t totalNodes = jb.n[s];
+  uint32_t* __restrict__ words = jb.words[s];
+  uint32_t* __restrict__ err = jb.dev + 2 * s + 1;
+  const uint64_t i = (uint64_t)(blockIdx.x - (s ? jb.T0 : 0u)) * blockDim.x + threadIdx.x;
   if (i >= totalNodes) return;
+  if (i == 0) jb.cnt[s][0] = jb.cnt[s][1] = jb.dev[2 * s];
   const uint32_t lev = level_of(a, i);
   const uint64_t j = i - a.start[lev];
   const uint32_t at = truePtrs[i];
@@ -77,15 +109,22 @@ __global__ void k_write_words(LevelSet a, int ussv, const uint32_t* __restrict__
   words[at] = ussv ? w0 : (w0 & 0xFFu);
   uint32_t k = at + 1;
   const uint32_t kEnd = k + (uint32_t)__popc(w0 & 0xFFu);   // the words the size pass reserved
+  // all pointers before the first store, which the loads could not pass
+  uint32_t ch[8], to[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) ch[c] = r[1 + c];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const uint32_t cl = (!ussv && childLv && ch[c] != kNull) ? childLv[j * 8 + c] : lev + 1;
+    const uint64_t g = (ch[c] != kNull && cl < a.L) ? (uint64_t)ch[c] + a.start[cl] : totalNodes;
+    to[c] = g < totalNodes ? truePtrs[g] : kNone;
+  }
 #pragma unroll
   for (int c = 7; c >= 0; --c) {
-    const uint32_t ch = r[1 + c];
-    if (ch == kNull) continue;
+    if (ch[c] == kNull) continue;
     if (k >= kEnd) { atomicAdd(err, 1u); break; }
-    const uint32_t cl = (!ussv && childLv) ? childLv[j * 8 + c] : lev + 1;
-    const uint64_t g = cl < a.L ? (uint64_t)ch + a.start[cl] : totalNodes;
-    if (g >= totalNodes) { atomicAdd(err, 1u); words[k++] = 0u; continue; }
-    words[k++] = truePtrs[g];
+    if (to[c] == kNone) { atomicAdd(err, 1u); words[k++] = 0u; continue; }
+    words[k++] = to[c];
   }
 }
 
@@ -473,19 +512,17 @@ void encode_words_enqueue(svd_octree* o, const int* fmts, int K, WordsPending& w
   wp.dev = dev;
   uint32_t** ptrsOf = wp.ptrs;
   uint64_t* hdrBytesOf = wp.hdrBytes;
+  WordJobs jb = {};
+  jb.dev = dev;
   for (int s = 0; s < K; ++s) {
     wp.fmts[s] = fmts[s];
     const int fmt = fmts[s];
     const bool ussv = fmt == SVD_FMT_USSVDAG;
     const std::vector<Level>& lv = ussv ? o->sdag : (o->hasX ? o->xdag : o->dag);
-    const LevelSet a = level_set(lv, L, !ussv);
-    const uint64_t N = a.start[L];
-    uint32_t* ptrs = dalloc<uint32_t>(c, N + 1);
-    ptrsOf[s] = ptrs;
-    uint32_t* d = dev + 2 * s;
-    if (N) k_word_counts<<<div_up(N, kB), kB, 0, c->stream>>>(a, N, ptrs);
-    check_launch("k_word_counts");
-    scan_exclusive(c, ptrs, ptrs, N, d);
+    jb.a[s] = level_set(lv, L, !ussv);
+    const uint64_t N = jb.n[s] = jb.a[s].start[L];
+    ptrsOf[s] = jb.ptrs[s] = dalloc<uint32_t>(c, N + 1);
+    jb.ussv[s] = ussv ? 1 : 0;
     // The reference assigns _firstLeafPtr after the loop over ALL levels
     // (encoded_svdag.cpp:129-137), so the stored value is the total word
     // count.  Every node takes at most 9 words: the image is allocated for
@@ -503,12 +540,23 @@ void encode_words_enqueue(svd_octree* o, const int* fmts, int K, WordsPending& w
     e.valid = false;
     if (!N) hdr.resize(hdr.size() + 8, 0);   // no words: both count words are 0
     wp.puts.add(c, e.d, hdr);
-    uint32_t* words = (uint32_t*)(e.d + hdrBytes);
-    if (N)
-      k_write_words<<<div_up(N, kB), kB, 0, c->stream>>>(a, ussv ? 1 : 0, ptrs, N, words, d + 1, d,
-                                                         (uint32_t*)(e.d + hdrBytes - 8));
-    check_launch("k_write_words");
+    jb.words[s] = (uint32_t*)(e.d + hdrBytes);
+    jb.cnt[s] = (uint32_t*)(e.d + hdrBytes - 8);
   }
+  // the second format's tiles (workgroups) come after the first one's; a format
+  // without nodes has none, and its word count stays the zero it was filled with
+  uint64_t T[2], W[2];
+  for (int s = 0; s < 2; ++s) {
+    T[s] = div_up(jb.n[s], (uint64_t)kScanOpT * kWordPer);
+    W[s] = div_up(jb.n[s], kB);
+  }
+  if (!(T[0] + T[1])) return;
+  jb.T0 = (uint32_t)T[0];
+  k_word_scan<<<(uint32_t)(T[0] + T[1]), kScanOpT, 0, c->stream>>>(jb, lb_pass(c, T[0] + T[1]));
+  check_launch("k_word_scan");
+  jb.T0 = (uint32_t)W[0];
+  k_write_words<<<(uint32_t)(W[0] + W[1]), kB, 0, c->stream>>>(jb);
+  check_launch("k_write_words");
 }
 
 // h: the 2K words of wp.dev, read back.

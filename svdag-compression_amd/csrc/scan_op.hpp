@@ -73,17 +73,9 @@ __global__ void __launch_bounds__(kScanOpT) k_scan_op(uint64_t n, LbPass p, Op o
 // n1) in one launch: the first T0 tiles are op0's, the rest op1's, each with
 // its own look-back chain in the shared pass.
 template <int PER, typename Op>
-__global__ void __launch_bounds__(kScanOpT) k_scan_op2(uint64_t n0, uint64_t n1, uint32_t T0, LbPass p, Op op0,
-                                                       Op op1, uint32_t* __restrict__ total0,
-                                                       uint32_t* __restrict__ total1) {
+__device__ __forceinline__ void scan_tile(uint64_t n, const LbPass& p, uint32_t tile, uint32_t first, uint32_t last,
+                                          const Op& op, uint32_t* __restrict__ total, uint32_t* lds) {
   constexpr uint32_t kTile = kScanOpT * PER;
-  __shared__ uint32_t lds[kScanOpT / 64 + 2];
-  __shared__ uint32_t word;
-  const uint32_t tile = lb_take_tile(p, &word);
-  const bool second = tile >= T0;
-  const Op& op = second ? op1 : op0;
-  const uint64_t n = second ? n1 : n0;
-  const uint32_t first = second ? T0 : 0u;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t base = (uint64_t)(tile - first) * kTile + (uint64_t)wave * (64 * PER) + lane;
   uint32_t ex[PER];
@@ -117,9 +109,20 @@ __global__ void __launch_bounds__(kScanOpT) k_scan_op2(uint64_t n0, uint64_t n1,
     const uint64_t i = base + 64 * k;
     if (i < n) op.apply(i, off + ex[k]);
   }
-  uint32_t* total = second ? total1 : total0;
-  const uint32_t last = second ? p.tiles - 1 : T0 - 1;
   if (total && tile == last && threadIdx.x == 0) *total = off + agg;
+}
+
+template <int PER, typename Op>
+__global__ void __launch_bounds__(kScanOpT) k_scan_op2(uint64_t n0, uint64_t n1, uint32_t T0, LbPass p, Op op0,
+                                                       Op op1, uint32_t* __restrict__ total0,
+                                                       uint32_t* __restrict__ total1) {
+  __shared__ uint32_t lds[kScanOpT / 64 + 2];
+  __shared__ uint32_t word;
+  const uint32_t tile = lb_take_tile(p, &word);
+  const bool second = tile >= T0;
+  const Op& op = second ? op1 : op0;
+  scan_tile<PER>(second ? n1 : n0, p, tile, second ? T0 : 0u, second ? p.tiles - 1 : T0 - 1, op,
+                 second ? total1 : total0, lds);
 }
 
 template <int PER, typename Op>
