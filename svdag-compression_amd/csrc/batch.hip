@@ -168,11 +168,14 @@ __global__ void k_batch_write_words(const uint32_t* __restrict__ rec, uint64_t n
   uint64_t k = at + 1;
   const uint64_t nb = base[(uint64_t)(lev + 1) * S + s];
   const uint32_t ns = scanStart[(uint64_t)(lev + 1) * S + s];
+  uint32_t ch[8], to[8];                 // all loads before the stores
 #pragma unroll
-  for (int c = 7; c >= 0; --c) {
-    if (!((m >> c) & 1u)) continue;
-    words[k++] = (uint32_t)(nb + scanNext[r[1 + c]] - ns);
-  }
+  for (int c = 0; c < 8; ++c) ch[c] = r[1 + c];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) to[c] = ((m >> c) & 1u) ? scanNext[ch[c]] : 0u;
+#pragma unroll
+  for (int c = 7; c >= 0; --c)
+    if ((m >> c) & 1u) words[k++] = (uint32_t)(nb + to[c] - ns);
 }
 
 __global__ void k_gather_starts(const uint32_t* __restrict__ remap, const uint32_t* __restrict__ svoStart, uint32_t S,
