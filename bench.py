@@ -220,6 +220,7 @@ def level_signatures(S, g, lev):
     import torch
     n = g.level_size(S.VIEW_DAG, lev)
     sig = torch.zeros(max(n, 1) * 16, dtype=torch.int32, device="cuda:0")
+    torch.cuda.synchronize()
     g.lossy_signatures(lev, sig.data_ptr())
     torch.cuda.synchronize()
     return sig.view(torch.int64).view(-1, 8)[:n]
@@ -307,6 +308,7 @@ def batch_bench(S, W, ctx, n_scenes, log):
     nr = n_cam * cw * ch
     prim = torch.zeros(nr * 6, dtype=torch.int32, device="cuda:0")
     shad = torch.zeros(nr * 6, dtype=torch.int32, device="cuda:0")
+    torch.cuda.synchronize()
     b.trace(cams, cam_scene, prim.data_ptr(), shad.data_ptr())          # warm-up
     tt = []
     for _ in range(3):
@@ -434,6 +436,7 @@ def attr_bench(S, W, ctx, levels, log, cpu=True):
     out["csvdag_bytes"] = int(g.encoded_device(S.FMT_SVDAG)[1])
     g.free()
     mat = torch.zeros(max(u.n, 1), dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
     ctx.materials(u, levels, mat.data_ptr(), seed=4, n_values=16)
     for tag, gray in (("gray", True), ("binary", False)):
         blob = ctx.attr_bittree((mat.data_ptr(), u.n), gray)        # warm-up
@@ -454,6 +457,7 @@ def attr_bench(S, W, ctx, levels, log, cpu=True):
     p = W.trace_params(w, h, seed=5, levels=levels, shadows=True)
     prim = torch.zeros(w * h * 6, dtype=torch.int32, device="cuda:0")
     shad = torch.zeros(w * h * 6, dtype=torch.int32, device="cuda:0")
+    torch.cuda.synchronize()
     tile = ctx.autotune_trace(sc, p, prim.data_ptr(), shad.data_ptr(), reps=2)
     tk = []
     for _ in range(3):

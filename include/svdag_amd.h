@@ -72,7 +72,11 @@ int svd_ctx_synchronize(svd_ctx* ctx);
  * it (they have read back every size they need; the codes have been read).
  * Every call that returns data (counts, levels, sizes, copies, device
  * pointers) is ordered after them; work of the caller's own on other streams
- * is not: svd_ctx_synchronize first.                                        */
+ * is not: svd_ctx_synchronize first.  The other way round, no call waits for
+ * work on other streams, the default stream included: what fills or still
+ * uses a device array has to be over before the array is passed in, be it as
+ * input or output (hipStreamSynchronize, or an event that this stream waits
+ * for).                                                                     */
 void* svd_ctx_stream(svd_ctx* ctx);
 
 /* ---- construction --------------------------------------------------------

@@ -925,11 +925,6 @@ int svd_lossy_merge(svd_octree* o, const svd_lossy_params* p, svd_lossy_level_st
 int svd_lossy_signatures(svd_octree* o, uint32_t lev, uint32_t* sig) {
   if (!o || !sig) return SVD_ERR_ARG;
   return guarded(o->ctx, [&] {
-    // The call is over in microseconds: a caller's fill of the buffer on the
-    // default stream may still be under way when its kernel would start.
-    svd_ctx* c = o->ctx;
-    SVD_HIP(hipEventRecord(c->ev[0], nullptr));
-    SVD_HIP(hipStreamWaitEvent(c->stream, c->ev[0], 0));
     lossy_signatures(o, lev, sig);
     SVD_HIP(hipStreamSynchronize(o->ctx->stream));
   });

@@ -114,11 +114,13 @@ def test_batch_trace_equals_single_traces(ctx):
     n = W_ * H_
     prim = torch.zeros(len(cams) * n * 6, dtype=torch.int32, device=DEV)
     shad = torch.zeros(len(cams) * n * 6, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
     b.trace(cams, cam_scene, prim.data_ptr(), shad.data_ptr())
     pr = prim.cpu().numpy().view(S.RAY_DTYPE).reshape(len(cams), n)
     sh = shad.cpu().numpy().view(S.RAY_DTYPE).reshape(len(cams), n)
     one_p = torch.zeros(n * 6, dtype=torch.int32, device=DEV)
     one_s = torch.zeros(n * 6, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
     for k, s in enumerate(cam_scene):
         sc = S.Scene.from_bytes(ctx, S.FMT_SVDAG, b.svdag_bytes(s))
         sc.trace_device(cams[k], one_p.data_ptr(), one_s.data_ptr())
@@ -162,6 +164,7 @@ def test_trace_launch_shapes_give_identical_rays(ctx, tmp_path, fmt):
             ctx.trace_tile = w
             prim.fill_(-7)
             shad.fill_(-7)
+            torch.cuda.synchronize()
             sc.trace_device(p, prim.data_ptr(), shad.data_ptr())
             ctx.sync()
             got = (prim.cpu().numpy().copy(), shad.cpu().numpy().copy())

@@ -175,6 +175,7 @@ def test_lossy_signatures_match_oracle(ctx):
     for lev in range(1, L - 1):
         n = g.level_size(S.VIEW_DAG, lev)
         sig = torch.zeros(n * 16, dtype=torch.int32, device=DEV)
+        torch.cuda.synchronize()
         g.lossy_signatures(lev, sig.data_ptr())
         np.testing.assert_array_equal(sig.cpu().numpy().view(np.uint32).reshape(n, 16), o.lossy_signatures(lev))
 
@@ -192,6 +193,22 @@ def test_lossy_signatures_every_level(ctx, L):
         g.lossy_signatures(lev, sig.data_ptr())
         ctx.sync()
         np.testing.assert_array_equal(sig.cpu().numpy().view(np.uint32).reshape(n, 16), o.lossy_signatures(lev))
+
+
+def test_signatures_do_not_wait_for_other_streams(ctx):
+    """The caller orders its own work: a call runs beside what is pending on
+    the default stream (a spinning kernel of some milliseconds)."""
+    codes, L = W.terrain_codes(7, seed=1), 7
+    g = gpu_dag(ctx, codes, L)
+    sig = torch.zeros(g.level_size(S.VIEW_DAG, 4) * 16, dtype=torch.int32, device=DEV)
+    g.lossy_signatures(4, sig.data_ptr())
+    torch.cuda.synchronize()
+    done = torch.cuda.Event()
+    torch.cuda._sleep(20_000_000)
+    done.record()
+    g.lossy_signatures(4, sig.data_ptr())
+    assert not done.query()
+    torch.cuda.synchronize()
 
 
 def test_lossy_argument_errors(ctx):
@@ -232,6 +249,7 @@ def test_mlp_forward_matches_oracle(ctx):
     sig = _rand_sigs(n, 1)
     emb = torch.zeros(n * 32, dtype=torch.float32, device=DEV)
     dsig = _dev_u32(sig)                 # keep the tensor alive while the library reads it
+    torch.cuda.synchronize()
     m.embed(dsig.data_ptr(), n, emb.data_ptr())
     e_g = emb.cpu().numpy().reshape(n, 32)
     e_o, _ = M.forward(p, M.unpack_bits(sig))
@@ -252,6 +270,7 @@ def test_mlp_gradients_match_oracle(ctx, P):
     H = M.hamming(sig[0::2], sig[1::2])
     # both tensors stay referenced: a freed temporary's block is reused by the next allocation
     dsig, dlab = _dev_u32(sig), _dev_u32(H.astype(np.uint32))
+    torch.cuda.synchronize()
     loss_g, grad_g = m.loss_grad(dsig.data_ptr(), dlab.data_ptr(), P)
     loss_o, grad_o = M.loss_and_grads(p, M.unpack_bits(sig), H)
     errs = {"loss": abs(loss_g - loss_o) / abs(loss_o)}
@@ -286,6 +305,7 @@ def test_knn_matches_oracle(ctx):
     e[100] = e[7]                       # an exact duplicate (distance 0, tie by index)
     de = torch.from_numpy(e).to(DEV)
     out = torch.zeros(n * 16, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
     ctx.knn(de.data_ptr(), n, 16, 4, 16, 32, 7, out.data_ptr())
     got = out.cpu().numpy().view(np.uint32).reshape(n, 16)
     np.testing.assert_array_equal(got, O.knn_lsh(e, 16, 4, 16, 32, 7))
@@ -293,6 +313,7 @@ def test_knn_matches_oracle(ctx):
     # signature re-ranking
     sig = _rand_sigs(n, 6, density=0.1)
     dsig = _dev_u32(sig)
+    torch.cuda.synchronize()
     ctx.knn(de.data_ptr(), n, 16, 4, 12, 48, 9, out.data_ptr(), sig_ptr=dsig.data_ptr())
     np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32).reshape(n, 16),
                                   O.knn_lsh(e, 16, 4, 12, 48, 9, sig=sig))
@@ -325,6 +346,7 @@ def test_knn_full_window_is_brute_force(ctx):
     e = rng.standard_normal((n, 32)).astype(np.float32)
     de = torch.from_numpy(e).to(DEV)
     out = torch.zeros(n * 8, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
     ctx.knn(de.data_ptr(), n, 8, 1, 4, 96, 3, out.data_ptr())
     got = out.cpu().numpy().view(np.uint32).reshape(n, 8)
     d = np.zeros((n, n), np.float32)           # the same sequential fp32 sum as the kernel
@@ -365,8 +387,9 @@ def test_lossy_learned_matches_oracle_given_knn(ctx):
     # checked against the oracle's search on the same signatures / embeddings
     n0 = g.level_size(S.VIEW_DAG, L - 2)
     dsig = torch.zeros(n0 * 16, dtype=torch.int32, device=DEV)
-    g.lossy_signatures(L - 2, dsig.data_ptr())
     demb = torch.zeros(n0 * 32, dtype=torch.float32, device=DEV)
+    torch.cuda.synchronize()
+    g.lossy_signatures(L - 2, dsig.data_ptr())
     m.embed(dsig.data_ptr(), n0, demb.data_ptr())
     sig0 = dsig.cpu().numpy().view(np.uint32).reshape(n0, 16)
     emb0 = demb.cpu().numpy().reshape(n0, 32)

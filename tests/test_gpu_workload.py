@@ -22,6 +22,7 @@ def test_materials_match_numpy(ctx, levels):
     import torch
     d = ctx.caves(levels, seed=3)
     out = torch.zeros(d.n, dtype=torch.uint8, device="cuda:0")
+    torch.cuda.synchronize()
     ctx.materials(d, levels, out.data_ptr(), seed=4, n_values=16)
     codes = d.numpy()
     d.free()
