@@ -11,6 +11,7 @@ import svdag_amd.workloads as W
 pytestmark = pytest.mark.gpu
 
 FORMATS = [S.FMT_SVDAG, S.FMT_USSVDAG, S.FMT_SSVDAG, S.FMT_ESVDAG]
+O_FMT = {S.FMT_SVDAG: 0, S.FMT_USSVDAG: 1, S.FMT_SSVDAG: 2, S.FMT_ESVDAG: 2}   # the oracle's encoders
 
 
 @pytest.fixture(scope="module")
@@ -161,6 +162,45 @@ def test_shared_out_rays_match_oracle(ctx, scene_files, size, samples, nrays):
         S.Scene.from_bytes(ctx, fmt, files[fmt]).ao_device(p, nrays, vis.data_ptr())
         ctx.sync()
         np.testing.assert_array_equal(vis.cpu().numpy().reshape(p.height, p.width), want)
+
+
+def deep_file(fmt, L):
+    """A sphere of points in a 2^L grid, in the given format."""
+    rng = np.random.default_rng(L)
+    d = rng.standard_normal((30000, 3))
+    xyz = ((0.5 + 0.4 * d / np.linalg.norm(d, axis=1)[:, None]) * (1 << L)).astype(np.int64)
+    o = O.OracleOctree.from_morton(W.sorted_codes(xyz[:, 0], xyz[:, 1], xyz[:, 2]), L)
+    o.to_dag()
+    o.init_child_levels()
+    if fmt in (S.FMT_USSVDAG, S.FMT_SSVDAG):
+        o.to_sdag()
+    return o.encode(O_FMT[fmt])
+
+
+@pytest.mark.parametrize("L", [19, 20, 21])
+@pytest.mark.parametrize("fmt", [S.FMT_USSVDAG, S.FMT_SSVDAG])
+def test_deepest_scenes_match_oracle(ctx, fmt, L):
+    """The descent stacks of the deepest scenes take the most LDS a workgroup
+    asks for (three words per level and lane in the USSVDAG format): the shaded
+    frame, with and without the primary records, and the AO pass."""
+    import torch
+    buf = deep_file(fmt, L)
+    p = W.trace_params(70, 45, seed=4, levels=L, shadows=True, light=(1.0, 0.6, 1.0))
+    v = S.ViewParams.defaults(render_mode=3, norm_samples=3)
+    want, wprim = O.render_frame(buf, fmt, p, v)
+    assert (wprim["t"] >= 0).mean() > 0.1
+    got, gprim = gpu_render(ctx, fmt, buf, p, v, 0.0)
+    np.testing.assert_array_equal(gprim, wprim)
+    np.testing.assert_array_equal(got, want)
+    sc = S.Scene.from_bytes(ctx, fmt, buf)
+    rgb = torch.full((p.width * p.height * 3,), float("nan"), dtype=torch.float32, device="cuda")
+    vis = torch.full((p.width * p.height,), float("nan"), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    sc.render_device(p, v, rgb.data_ptr())
+    sc.ao_device(p, 5, vis.data_ptr())
+    ctx.sync()
+    np.testing.assert_array_equal(rgb.cpu().numpy().reshape(want.shape), want)
+    np.testing.assert_array_equal(vis.cpu().numpy().reshape(p.height, p.width), O.trace_ao(buf, fmt, p, 5)[0])
 
 
 def test_render_and_ao_reject_bad_arguments(ctx, scene_files):
