@@ -100,6 +100,74 @@ def test_batch_device_scenes_equal_single_builds(ctx):
         d.free()
 
 
+def test_batch_of_two_pass_levels_equals_single_builds(ctx):
+    """More than 4M codes and 4M leaf nodes: the leaf level and the level above
+    it come from two passes over 4096-code tiles, and the leaves' scenes from
+    the first of them.  Scenes of 70-80K sparse codes that begin on, one before
+    and one after a tile's first code, and runs of tiny scenes that share a tile
+    (their codes bisect the scene offsets).  A bad code in any of the tiles is
+    refused, and the next build is right again."""
+    rng = np.random.default_rng(5)
+    codes, levels = [], []
+    at = 0
+
+    def add(c, L):
+        nonlocal at
+        codes.append(c)
+        levels.append(L)
+        at += c.size
+
+    def sparse(L, n):
+        c = np.unique(rng.integers(0, 1 << (3 * L), n + n // 8, dtype=np.uint64))
+        return np.sort(rng.permutation(c)[:n])
+
+    for k in range(58):
+        L = int(rng.integers(9, 11))
+        n = 70000 + int(rng.integers(0, 10000))
+        n += (-(at + n)) % 4096 + (0, 1, 4095)[k % 3]      # the next scene begins there
+        add(sparse(L, n), L)
+        for _ in range(25 if k % 2 else 0):
+            L = int(rng.integers(2, 6))
+            add(sparse(L, int(rng.integers(1, 41))), L)
+    allc, off = _pack(codes)
+    leaves = sum(np.unique(c >> np.uint64(3)).size for c in codes)
+    print(f"[case] batch of {len(codes)} scenes, {allc.size} voxels, {leaves} leaf nodes", flush=True)
+    assert leaves >= 4 << 20
+    d = torch.from_numpy(allc.view(np.int64)).to(DEV)
+    torch.cuda.synchronize()
+
+    def check():
+        b = S.Batch(ctx, d.data_ptr(), off, levels, on_device=True)
+        for s, (c, L) in enumerate(zip(codes, levels)):
+            if c.size > 1000:
+                g = S.Octree.from_morton(ctx, (d.data_ptr() + 8 * int(off[s]), c.size), L)
+                g.to_dag()
+                g.encode(S.FMT_SVDAG)
+                want, nodes = g.encoded_bytes(S.FMT_SVDAG), g.counts()[0]
+                g.free()
+            else:
+                o = O.OracleOctree.from_morton(c, L)
+                o.to_dag()
+                o.init_child_levels()
+                want, nodes = o.encode(0), o.n_nodes
+            assert b.info(s)["nodes"] == nodes and b.svdag_bytes(s) == want, f"scene {s} ({L} levels, {c.size} voxels)"
+        b.free()
+
+    check()
+    tiny = next(s for s, c in enumerate(codes) if 2 <= c.size < 1000)
+    for i, v in ((4096 * 517, int(allc[4096 * 517 - 1])),            # a duplicate across a tile's end inside a scene
+                 (int(off[tiny]), 1 << (3 * levels[tiny])),           # beyond the scene's depth
+                 (allc.size - 1, int(allc[-2]))):                     # the last code, a duplicate
+        good = int(d[i])
+        d[i] = v
+        torch.cuda.synchronize()
+        with pytest.raises(S.SvdError):
+            S.Batch(ctx, d.data_ptr(), off, levels, on_device=True)
+        d[i] = good
+    torch.cuda.synchronize()
+    check()
+
+
 def test_batch_trace_equals_single_traces(ctx):
     specs, codes = _scenes(6, 3, (5, 7))
     levels = [s["levels"] for s in specs]
