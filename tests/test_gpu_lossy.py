@@ -159,6 +159,23 @@ def test_lossy_exhaustive_lists_of_a_large_level(ctx):
         np.testing.assert_array_equal(st[0][f], st[1][f], err_msg=f)
 
 
+@pytest.mark.parametrize("bound,cap", [(4, 1), (4, 16), (6, 2), (8, 64), (24, 16)])
+def test_lossy_exhaustive_full_lists_of_a_large_level(ctx, bound, cap):
+    """The two-tile workgroups with lists that overflow twice their capacity,
+    and nodes that stop between chunks (bounds that fill a list within a few
+    thousand nodes, and bounds that leave some open to the end): the merged
+    level equals the oracle's, which walks the earlier nodes in order."""
+    codes, L = random_codes(9, 380000, 5), 9
+    g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
+    n = g.level_size(S.VIEW_DAG, 6)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert n >= 256 * cus, "the level is too small for two tiles per wavefront"
+    kw = dict(max_diff=bound, list_cap=cap)
+    st_g, st_o = g.lossy_merge(6, 6, **kw), o.lossy_merge(6, 6, **kw)
+    assert_same_stats(st_g, st_o)
+    assert_same_dag(g, o, L)
+
+
 def test_lossy_error_within_accounted_bound(ctx):
     codes, L = W.cave_codes(7, seed=3), 7
     g = gpu_dag(ctx, codes, L)
