@@ -375,7 +375,52 @@ def test_knn_full_window_is_brute_force(ctx):
     np.testing.assert_array_equal(got, want)
 
 
+def test_knn_of_more_points_than_22_bits(ctx):
+    """Beyond 2^22 points a (distance, node) key no longer fits 32 bits: the
+    window kernel that keeps them apart, at its list size of 16, over two
+    tables and many equal signatures."""
+    n = (1 << 22) + 777
+    rng = np.random.default_rng(3)
+    e = rng.standard_normal((n, 32), dtype=np.float32)
+    sig = (rng.integers(0, 1 << 32, (n // 4, 16), dtype=np.uint32) &
+           rng.integers(0, 1 << 32, (n // 4, 16), dtype=np.uint32))[rng.integers(0, n // 4, n)]
+    de, dsig = torch.from_numpy(e).to(DEV), _dev_u32(sig)
+    out = torch.zeros(n * 16, dtype=torch.int32, device=DEV)
+    torch.cuda.synchronize()
+    ctx.knn(de.data_ptr(), n, 16, 2, 12, 3, 9, out.data_ptr(), sig_ptr=dsig.data_ptr())
+    ctx.sync()
+    print(f"[case] {n} points searched", flush=True)
+    np.testing.assert_array_equal(out.cpu().numpy().view(np.uint32).reshape(n, 16),
+                                  O.knn_lsh(e, 16, 2, 12, 3, 9, sig=sig))
+
+
 # ---------------------------------------------------------------- learned lossy
+def test_knn_refine_of_more_nodes_than_22_bits(ctx):
+    """A level of more than 2^22 nodes takes the refinement with 64-bit keys."""
+    L, lev, k = 11, 8, 2
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    codes = torch.unique(torch.randint(0, 1 << (3 * L), (36_000_000,), dtype=torch.int64, device=DEV, generator=gen))
+    torch.cuda.synchronize()
+    g, m = S.Octree.from_morton(ctx, (codes.data_ptr(), codes.numel()), L), S.MLP(ctx, seed=1)
+    g.to_dag()
+    n = g.level_size(S.VIEW_DAG, lev)
+    print(f"[case] {codes.numel()} voxels, {n} nodes in level {lev}", flush=True)
+    assert n > 1 << 22
+    dsig = torch.zeros(n * 16, dtype=torch.int32, device=DEV)
+    demb = torch.zeros(n * 32, dtype=torch.float32, device=DEV)
+    torch.cuda.synchronize()
+    g.lossy_signatures(lev, dsig.data_ptr())
+    m.embed(dsig.data_ptr(), n, demb.data_ptr())
+    ctx.sync()
+    sig, emb = dsig.cpu().numpy().view(np.uint32).reshape(n, 16), demb.cpu().numpy().reshape(n, 32)
+    kw = dict(k=k, tables=1, bits=12, window=2)
+    _, rec = g.lossy_merge(lev, lev, max_diff=1, model=m, refine=1, record_knn=True, **kw)
+    g.free()
+    print("[case] merged", flush=True)
+    want = O.knn_refine(sig, O.knn_lsh(emb, k, 1, 12, 2, 7, sig=sig), 1)
+    np.testing.assert_array_equal(rec[:n * k].reshape(n, k), want)
+
+
 @pytest.mark.parametrize("k,rounds", [(1, 1), (15, 2), (16, 1), (16, 3), (17, 2), (32, 1)])
 def test_knn_refine_list_sizes(ctx, k, rounds):
     """Refinement with 32-bit keys (k <= 16) and 64-bit ones, after an odd and
