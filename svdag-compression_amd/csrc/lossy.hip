@@ -781,8 +781,11 @@ void exhaustive_lists(svd_ctx* c, const uint32_t* sig, uint64_t n, const uint64_
   SVD_HIP(rocprim::radix_sort_pairs(tmp, bytes, keys, keys2, ids, ids2, (size_t)n, 0, bits, c->stream));
   c->arena->put(tmp);
   k_list_gather<<<div_up(n * 4, kB), kB, 0, c->stream>>>(sig, ids2, keys2, n, nKeys, ssig, off);
-  // two j tiles per wavefront where that still gives every CU a workgroup
-  if (n >= 256 * (uint64_t)std::max(c->numCU, 1))
+  // two j tiles per wavefront (256 nodes per workgroup) where that still gives
+  // every CU the three workgroups it holds: one and two tiles took 7.1 and 5.7
+  // ms on 372K nodes (2048^3 caves), 1.65 and 1.67 on 204K, 1.94 and 2.65 on
+  // 126K, 1.20 and 1.77 on 68K
+  if (n >= 768 * (uint64_t)std::max(c->numCU, 1))
     k_exhaustive_lists<2><<<div_up(n, 256), 256, 0, c->stream>>>(ssig, ids2, keys2, off, (uint32_t)n, C, refs, maxRefs,
                                                                  bound, cap, lists, spill, counts);
   else

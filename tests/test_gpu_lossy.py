@@ -159,17 +159,19 @@ def test_lossy_exhaustive_lists_of_a_large_level(ctx):
         np.testing.assert_array_equal(st[0][f], st[1][f], err_msg=f)
 
 
-@pytest.mark.parametrize("bound,cap", [(4, 1), (4, 16), (6, 2), (8, 64), (24, 16)])
-def test_lossy_exhaustive_full_lists_of_a_large_level(ctx, bound, cap):
-    """The two-tile workgroups with lists that overflow twice their capacity,
-    and nodes that stop between chunks (bounds that fill a list within a few
-    thousand nodes, and bounds that leave some open to the end): the merged
-    level equals the oracle's, which walks the earlier nodes in order."""
-    codes, L = random_codes(9, 380000, 5), 9
+@pytest.mark.parametrize("two_tiles,voxels,bound,cap", [(False, 380000, 4, 16), (True, 800000, 6, 1),
+                                                         (True, 800000, 8, 2), (True, 800000, 8, 64),
+                                                         (True, 800000, 24, 16)])
+def test_lossy_exhaustive_full_lists_of_a_large_level(ctx, two_tiles, voxels, bound, cap):
+    """Lists of a large level that overflow twice their capacity, and nodes
+    that stop between chunks (bounds that fill a list within a few thousand
+    nodes, and bounds that leave some open to the end), by both workgroup
+    shapes: the merged level equals the oracle's, which walks the earlier nodes
+    in order."""
+    codes, L = random_codes(9, voxels, 5), 9
     g, o = gpu_dag(ctx, codes, L), oracle_dag(codes, L)
-    n = g.level_size(S.VIEW_DAG, 6)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert n >= 256 * cus, "the level is too small for two tiles per wavefront"
+    assert (g.level_size(S.VIEW_DAG, 6) >= 768 * cus) == two_tiles
     kw = dict(max_diff=bound, list_cap=cap)
     st_g, st_o = g.lossy_merge(6, 6, **kw), o.lossy_merge(6, 6, **kw)
     assert_same_stats(st_g, st_o)
