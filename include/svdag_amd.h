@@ -455,7 +455,8 @@ int svd_mlp_embed(svd_mlp* m, const uint32_t* sig_dev, uint64_t n, float* emb_de
 int svd_mlp_loss_grad(svd_mlp* m, const uint32_t* sig_dev, const uint32_t* labels_dev, uint64_t npairs,
                       float* loss, float* grads);
 /* Train on node pairs of oct's DAG levels with exact Hamming labels (Adam);
- * the step is captured once in a HIP graph and replayed.                     */
+ * a step is three launches, enqueued one after another; the call waits for
+ * the last.                                                                 */
 int svd_mlp_train(svd_mlp* m, svd_octree* oct, const svd_mlp_train_params* p, svd_mlp_train_stats* st);
 /* k nearest neighbours of n points of dim 32 (DEVICE), searched in `tables`
  * LSH orderings of `bits` sign bits within +-window positions; distance =

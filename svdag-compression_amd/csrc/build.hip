@@ -219,7 +219,11 @@ __device__ __forceinline__ void leaf_write(const Src& code, uint64_t n, uint64_t
 // the codes once, but holds every tile until its predecessors are known: the
 // leaves of 463M codes (a batch) took 1.84 ms in one pass and 1.03 + 0.60 ms in
 // two, of 13.7M codes 63 and 58 us; of 12K codes the two launches more cost
-// 40 us of a build's 400.
+// 40 us of a build's 400.  Whole SVO builds with the leaves in one and in two
+// passes: 137 and 138 us at 2M codes of the 2048^3 terrain (139 and 145 of the
+// 4096^3 caves), 145 and 144 at 3M, 154 and 150 at 4M, 178 and 174 at 8M, 210
+// and 199 at 13.7M; with the level above so too: the same up to 4M child codes,
+// 363 and 354 at 10.8M, 768 and 743 at 30M.
 constexpr uint64_t kTwoPassCodes = 4ull << 20;
 
 // The leaves in one pass; bad codes are added to bad[0] (zero between builds;
@@ -1617,7 +1621,8 @@ uint64_t svo_levels_from_codes(svd_ctx* c, const uint64_t* dcodes, uint64_t n, u
     finest(PlainCodes{dcodes}, hiMask);
   }
   // Half the workgroups below 64M codes: each counts itself done at one
-  // address (13.7M codes: 22 us with 256, 27 with 512; 463M: 282 and 241).
+  // address (13.7M codes: 21 us with 256, 27 with 512; 27M: 29 and 35; 55M: 46
+  // and 49; 93M: 81 and 81; 187M: 147 and 138; 463M: 282 and 241).
   const uint32_t grid = std::min<uint32_t>(n < (64ull << 20) ? kHistGrid / 2 : kHistGrid, div_up(n, 4096));
   k_level_hist<<<grid, 1024, 0, c->stream>>>(codeA, leaves, L, state, part, hist);
   check_launch("k_leaf_build");

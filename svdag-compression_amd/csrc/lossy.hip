@@ -7,12 +7,14 @@
 //      (bit c1*64 + c2*8 + c3 for the child-slot path; voxels at level L-3);
 //   2. lists: for each candidate j (effective reference count <= max_refs,
 //      :945) the first list_cap earlier nodes i < j with
-//      popcount(sig_i ^ sig_j) <= bound -- exhaustively (an LDS-tiled
-//      all-pairs XOR-popcount scan), or the list_cap nearest of them by
-//      (popcount, i) (ranked, the same scan to the end), or among the learned
-//      proposals (kNN of the MLP embeddings, sorted and de-duplicated);
+//      popcount(sig_i ^ sig_j) <= bound -- exhaustively (all pairs inside the
+//      bound's popcount window, their distances as a GEMM on the matrix
+//      cores), or the list_cap nearest of them by (popcount, i) (ranked, an
+//      LDS-tiled XOR-popcount scan), or among the learned proposals (kNN of
+//      the MLP embeddings, sorted and de-duplicated);
 //   3. verify: exact voxel difference of the two subtrees by a joint descent
-//      with early abort (the Hamming distance above is a lower bound of it);
+//      with early abort that ends at 512-bit occupancies (the Hamming distance
+//      above is a lower bound of it);
 //   4. resolve: j walks its verified entries in order; a representative
 //      becomes its target, an entry that merged earlier offers its own target
 //      (taken when the exact difference to j is within the bound); resolved
@@ -227,7 +229,7 @@ __device__ __forceinline__ uint32_t order_list(uint32_t* lists, uint64_t at, uin
 //    most before the smallest cap are kept; k_list_order sorts at the end.
 //  - Later j have more to scan, so the last workgroups start first.
 // Bound by the matrix cores: on 466K nodes of the 2048^3 caves (bound 10, 36%
-// of the pairs inside the popcount window) 9.0 ms at 66% of the MFMA cycles,
+// of the pairs inside the popcount window) 8.6 - 9.0 ms at 66% of the MFMA cycles,
 // against 19.3 ms without the window and 172 ms for an XOR/popcount scan.
 template <int JT>
 __global__ void __launch_bounds__(256, 3)
@@ -397,8 +399,10 @@ __global__ void __launch_bounds__(256) k_list_order(uint64_t n, uint32_t cap, ui
 
 // Ranked pre-filter lists: every earlier node i < j within the bound, the K
 // nearest kept by (hamming << 32 | i) in a sorted register list (an insertion
-// bubbles the new key in and drops the largest); the same LDS tiles as
-// k_exhaustive_lists, scanned to the end (no early stop).
+// bubbles the new key in and drops the largest).  Block = 256 consecutive j;
+// the earlier nodes are streamed through LDS in tiles of 256 signatures (16
+// KB) that every lane reads in the same order (LDS broadcast), to the end (no
+// early stop).
 template <int K>
 __global__ void __launch_bounds__(256) k_ranked_lists(const uint32_t* __restrict__ sig, uint64_t n,
                                                       const uint64_t* __restrict__ refs, uint64_t maxRefs,

@@ -69,8 +69,10 @@ __device__ __forceinline__ Stack make_stack(uint32_t* mem, int depth, int lane) 
 }
 
 // An SSVDAG's level offsets in LDS behind the stacks: every fetch adds its
-// level's, and a read from memory would stand in front of each of them.  All
-// threads of the workgroup call it before any leaves.
+// level's, and a read from memory would stand in front of each of them.  (A
+// third fewer vector memory reads; with the shared settle() a 1080p frame with
+// shadows 631 -> 610 us, as instruction issue under divergence bounds it.)
+// All threads of the workgroup call it before any leaves.
 template <int FMT>
 __device__ __forceinline__ const uint32_t* stage_offsets(const Dev& s, uint32_t* mem) {
   uint32_t* l = mem + kStackWords<FMT> * (s.innerLevels + 1) * kBT;
@@ -1145,7 +1147,7 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_gbuffer(Dev s, svd_tra
 // the next pair once kRayRefill lanes wait (or all): the rays over a hemisphere
 // differ so much in length that wavefronts which ran until their longest ray
 // kept 18% of their lanes busy (16 rays a pixel of a 1080p frame: 3.29 ms, with
-// refills 1.80).  The entry count is read once and a wavefront's runs
+// refills 1.72).  The entry count is read once and a wavefront's runs
 // ascend, so every wavefront leaves when its runs are beyond it and its rays,
 // of at most max_iters iterations each, have ended.
 constexpr uint32_t kAOEntries = 8;   // 4: the same, 16: 2% of the frame more, 64: 7%
