@@ -69,10 +69,10 @@ __device__ __forceinline__ Stack make_stack(uint32_t* mem, int depth, int lane) 
 }
 
 // An SSVDAG's level offsets in LDS behind the stacks: every fetch adds its
-// level's, and a read from memory would stand in front of each of them.  (A
-// third fewer vector memory reads; with the shared settle() a 1080p frame with
-// shadows 631 -> 610 us, as instruction issue under divergence bounds it.)
-// All threads of the workgroup call it before any leaves.
+// level's, and a read from memory would stand in front of each of them (a
+// third fewer vector memory reads: frames of 6 to 11 levels take 0 to 14% less,
+// the 1080p one of the 2048^3 terrain 7%).  All threads of the workgroup call it
+// before any leaves.
 template <int FMT>
 __device__ __forceinline__ const uint32_t* stage_offsets(const Dev& s, uint32_t* mem) {
   uint32_t* l = mem + kStackWords<FMT> * (s.innerLevels + 1) * kBT;
@@ -227,8 +227,7 @@ struct Tracer {
   __device__ __forceinline__ static bool in_bounds(const int li[3], int sz) {
     return (uint32_t)li[0] < (uint32_t)sz && (uint32_t)li[1] < (uint32_t)sz && (uint32_t)li[2] < (uint32_t)sz;
   }
-  // Up to the pushed node; settle() follows, as after down_in.
-  __device__ __forceinline__ void up_in(TS& ts) {
+  __device__ __forceinline__ void up_in(const float o[3], TS& ts) {
     uint32_t dl = ts.level;
     pop(ts);
     dl -= ts.level;
@@ -236,6 +235,9 @@ struct Tracer {
     for (int a = 0; a < 3; ++a) ts.idx[a] >>= dl;
     ts.cell *= (float)(1 << dl);
     ts.cns = (int)ts.level < s.innerLevels ? 2 : s.leafSize;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & 1;
+    next_crossing(ts, o);
   }
   // The position step of go_down_one_level (octree_dda.frag.glsl:434-451).
   // Its next-crossing and local-index updates read nothing this step reads,
@@ -262,18 +264,13 @@ struct Tracer {
       int vc = s.leafSize / 2;
       while (vc > 1) { step_down(o, d, ts); vc >>= 1; }
     }
+    next_crossing(ts, o);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & (ts.cns - 1);
     if (INSTR) {
       path = (path ^ (uint32_t)ts.node_index) * 16777619u;
       path = (path ^ ts.level) * 16777619u;
     }
-  }
-  // The next crossings and the local index in a node just entered: the same
-  // for a step up (into a node of side 2) and a step down, so a wavefront whose
-  // lanes do both runs it once.
-  __device__ __forceinline__ static void settle(TS& ts, const float o[3]) {
-    next_crossing(ts, o);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) ts.li[a] = ts.idx[a] & (ts.cns - 1);
   }
 
   // Per-ray state between iterations of the traversal loop.
@@ -356,6 +353,9 @@ struct Tracer {
   }
 
   // One iteration of traceRay's loop; returns true when the ray is finished.
+  // A step up and a step down each end with their own next crossings: shared
+  // after the branch, for wavefronts whose lanes do both, they took 4 - 8% more
+  // in every format (SVDAG and USSVDAG frames of 6 to 11 levels).
   __device__ __forceinline__ bool step(Ray& r, float out[4]) {
     TS& ts = r.ts;
     const bool full = fetch_voxel_bit(ts);
@@ -364,14 +364,12 @@ struct Tracer {
 #pragma unroll
     for (int a = 0; a < 3; ++a) { delta[a] = m[a] ? ts.di[a] : 0; nl[a] = ts.li[a] + delta[a]; }
     const bool next_in_node = in_bounds(nl, ts.cns);
-    bool entered = full;
     if (!full) {
       r.stepm = (uint32_t)(m[0] | (m[1] << 1) | (m[2] << 2));
       dda_next(ts, m, delta);
       if (!next_in_node) {
         if (st.size == 0) { out[0] = -1.f; out[1] = 0.f; out[2] = (float)r.it; out[3] = -1.f; return true; }
-        up_in(ts);
-        entered = true;
+        up_in(r.o, ts);
       }
     } else {
       const bool hit = (ts.level >= r.maxLevel) || ((ts.cell * r.projf) < ts.t_current);
@@ -383,7 +381,6 @@ struct Tracer {
       down_in(r.o, r.d, ts, next_in_node);
       fetch_data(ts);
     }
-    if (entered) settle(ts, r.o);
     ts.cli = lin_idx(ts, ts.cns);
     ++r.it;
     if ((ts.t_current < r.tmax) && ((uint32_t)r.it < r.maxIters)) return false;
@@ -1265,7 +1262,7 @@ namespace {
 // LDS of one workgroup: the descent stacks of its kBT lanes, the level offsets
 size_t stack_bytes(const svd_scene* sc, const Dev& d) {
   return ((size_t)(sc->fmt == SVD_FMT_USSVDAG ? kStackWords<SVD_FMT_USSVDAG> : 2) * (d.innerLevels + 1) * kBT +
-          kMaxLevels) * sizeof(uint32_t);
+          (sc->fmt == SVD_FMT_SSVDAG || sc->fmt == SVD_FMT_ESVDAG ? kMaxLevels : 0)) * sizeof(uint32_t);
 }
 
 // The DEPTH_MODE pre-pass into `depth` ((width/8) x (height/8) floats).  The
