@@ -1138,16 +1138,20 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_gbuffer(Dev s, svd_tra
   if (has) entries[wgBase + waveN[wave] + (uint32_t)__popcll(b & ((1ull << (tid & 63)) - 1ull))] = e;
 }
 
-// A wavefront takes its (entry, ray) pairs in runs of perRun entries, one run
-// of all wavefronts after the other (consecutive lanes take the rays of one
-// entry; a run has at least 64 pairs), and a lane that finished its ray takes
-// the next pair once kRayRefill lanes wait (or all): the rays over a hemisphere
-// differ so much in length that wavefronts which ran until their longest ray
-// kept 18% of their lanes busy (16 rays a pixel of a 1080p frame: 3.29 ms, with
-// refills 1.72).  The entry count is read once and a wavefront's runs
-// ascend, so every wavefront leaves when its runs are beyond it and its rays,
-// of at most max_iters iterations each, have ended.
-constexpr uint32_t kAOEntries = 8;   // 4: the same, 16: 2% of the frame more, 64: 7%
+// A wavefront takes its (entry, ray) pairs in runs of runLen pairs, one run of
+// all wavefronts after the other (consecutive lanes take the rays of one entry),
+// and a lane that finished its ray takes the next pair once kRayRefill lanes
+// wait (or all): the rays over a hemisphere differ so much in length that
+// wavefronts which ran until their longest ray kept 18% of their lanes busy (16
+// rays a pixel of a 1080p frame: 3.29 ms, with refills 1.72; runs of 64 to 256
+// pairs measure the same, 512 took 2% more, 1024 7%).  A frame with little work
+// needs its pairs on as many wavefronts as can be, so runs of a wavefront's
+// width where each would get fewer than four of them: runs of eight entries, as
+// 1080p frames would have them too, took 1.27 ms for 97x61 pixels with 256 rays
+// each (0.20 so; 0.22 without refills) and 1.59 ms for 200x120 (0.45; 0.55).
+// The entry count is read once and a wavefront's runs ascend, so every
+// wavefront leaves when its runs are beyond it and its rays, of at most
+// max_iters iterations each, have ended.
 template <int FMT>
 __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_rays(Dev s, svd_trace_params p, const float* __restrict__ hs,
                                                                  uint32_t nrays, const AOEntry* __restrict__ entries,
@@ -1156,26 +1160,32 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_rays(Dev s, svd_trace_
   extern __shared__ uint32_t stackMem[];
   Tracer<FMT, false> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, threadIdx.x), stage_offsets<FMT>(s, stackMem));
   typename Tracer<FMT, false>::Ray ray;
-  const uint32_t nE = *nEntries;
-  const uint32_t perRun = max(kAOEntries, (63u + nrays) / nrays), runLen = perRun * nrays;
-  const uint64_t stride = (uint64_t)gridDim.x * (kBT / 64) * perRun;
-  uint64_t first = (uint64_t)(blockIdx.x * (kBT / 64) + (threadIdx.x >> 6)) * perRun;   // the run's first entry
-  uint32_t at = 0;                                                                       // pairs taken of it
+  const uint64_t total = (uint64_t)*nEntries * nrays;
+  const uint32_t waves = gridDim.x * (kBT / 64), wave = blockIdx.x * (kBT / 64) + (threadIdx.x >> 6);
+  const uint32_t runLen = total >= (uint64_t)waves * 256u ? 128u : 64u;
+  const uint32_t stride = waves * runLen, strideE = stride / nrays, strideR = stride - strideE * nrays;
+  uint32_t runE = wave * runLen / nrays, runR = wave * runLen - runE * nrays;   // the run's first entry and ray
+  int64_t left = (int64_t)total - (int64_t)(wave * runLen);                      // pairs from the run's first on
+  uint32_t at = 0;                                                               // pairs taken of the run
   const uint64_t below = (1ull << (threadIdx.x & 63)) - 1ull;
   bool busy = false;
   uint32_t pixel = 0;
-  auto pairs_left = [&] { return first < nE && at < (uint32_t)min((uint64_t)perRun, nE - first) * nrays; };
-  bool more = pairs_left();
+  bool more = left > 0;
   while (true) {
     const uint64_t idle = __ballot(!busy);
     if (more && !busy) {
-      uint32_t v = at + (uint32_t)__popcll(idle & below);
-      const bool wrap = v >= runLen;
-      v -= wrap ? runLen : 0u;
-      const uint32_t q = v / nrays, i = v - q * nrays;
-      const uint64_t k = first + (wrap ? stride : 0ull) + q;
-      if (k < nE) {
-        const AOEntry e = entries[k];
+      uint32_t v = at + (uint32_t)__popcll(idle & below), e0 = runE, r0 = runR;
+      int64_t l = left;
+      if (v >= runLen) {                 // of the wavefront's next run
+        v -= runLen;
+        l -= stride;
+        e0 += strideE;
+        r0 += strideR;
+        if (r0 >= nrays) { r0 -= nrays; ++e0; }
+      }
+      if ((int64_t)v < l) {
+        const uint32_t q = (r0 + v) / nrays, i = r0 + v - q * nrays;
+        const AOEntry e = entries[e0 + q];
         const float hn[3] = {-(float)e.step[0], -(float)e.step[1], -(float)e.step[2]};
         const float rv[3] = {0.f, 1.f, 0.f};
         const float dn = dot3(rv, hn);
@@ -1199,9 +1209,12 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_ao_rays(Dev s, svd_trace_
       at += (uint32_t)__popcll(idle);
       if (at >= runLen) {
         at -= runLen;
-        first += stride;
+        left -= stride;
+        runE += strideE;
+        runR += strideR;
+        if (runR >= nrays) { runR -= nrays; ++runE; }
       }
-      more = pairs_left();
+      more = (int64_t)at < left;
     }
     while (true) {
       if (busy) {

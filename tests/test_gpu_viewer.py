@@ -141,11 +141,12 @@ def test_ao_matches_oracle(ctx, scene_files, fmt, nrays):
 
 
 @pytest.mark.parametrize("size,samples,nrays", [((1, 1), 1, 1), ((17, 9), 64, 256), ((33, 47), 1, 3),
-                                                ((16, 16), 5, 64), ((70, 45), 3, 7)])
+                                                ((16, 16), 5, 64), ((70, 45), 3, 7), ((400, 300), 1, 60)])
 def test_shared_out_rays_match_oracle(ctx, scene_files, size, samples, nrays):
     """The rays that a workgroup or wavefront shares out over its lanes: fewer
     than a wavefront, partial tiles and runs, the most rays a pixel takes, and
-    lanes that take a second ray (also with rays that end by max_iters)."""
+    lanes that take a second ray (also with rays that end by max_iters); the
+    last frame's AO pairs take the longer runs, which end inside entries."""
     import torch
     L, files = scene_files
     fmt = S.FMT_SSVDAG
