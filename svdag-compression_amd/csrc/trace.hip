@@ -615,12 +615,13 @@ struct ViewArgs {
 // colouring and the shadow ray.  rgb gets the colour the fragment writes; a
 // fragment the shader discards gets 0.
 //
-// One workgroup per pixel tile, in three phases over its pixels with a hit:
+// Two forms, bit for bit alike: k_render_lane with a lane per pixel, and k_render
+// with one workgroup per pixel tile, in three phases over its pixels with a hit:
 // the primary rays of all pixels, the (hit, normal sample) rays shared out over
 // the lanes, and shading with the shadow ray, a lane per hit.  A lane per pixel
-// throughout left the lanes of pixels without a hit idle, and the others
-// waiting for the longest ray of each sample in turn (1080p, 4 samples and a
-// shadow ray: 1.28 ms, shared out 1.13).
+// leaves the lanes of pixels without a hit idle, and the others waiting for the
+// longest ray of each sample in turn; sharing out costs barriers and the set-up
+// of a refill.
 struct RenderHit {
   float res[4];
   uint32_t where;   // pixel in the tile (x | y << 8), primary step (axis a: bits 16 + 2a, step + 1)
@@ -979,6 +980,64 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_trace_batch(const Dev* __
 constexpr uint32_t kRayRefill = 16;
 
 // prim (primary records with path and bytes) only with INSTR, here and below.
+// A lane per pixel throughout (render_shares says when).
+template <int FMT, bool INSTR>
+__global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_render_lane(Dev s, svd_trace_params p, ViewArgs va,
+                                                                     float* __restrict__ rgb,
+                                                                     svd_ray_result* __restrict__ prim, MinDepth md) {
+  extern __shared__ uint32_t stackMem[];
+  const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t py = blockIdx.y * blockDim.y + threadIdx.y;
+  const int tid = threadIdx.y * blockDim.x + threadIdx.x;
+  const uint32_t* lofs = stage_offsets<FMT>(s, stackMem);
+  if (px >= p.width || py >= p.height) return;
+  Tracer<FMT, INSTR> tr(s, make_stack<FMT>(stackMem, s.innerLevels + 1, tid), lofs);
+  float scx, scy, o[3], d[3];
+  render_camera(p, px, py, scx, scy, o, d);
+  const float tmin = md.t ? min_t(md, px, py) - 1e-3f : 0.0f;
+  RenderHit e;
+  int step[3];
+  tr.trace(o, d, tmin, 1e30f, p.projection_factor, p.max_iters, p.draw_level, e.res, step);
+  if (tr.bad) { e.res[0] = -6.f; e.res[1] = 0.f; e.res[3] = -1.f; }
+  const size_t k = (size_t)py * p.width + px;
+  if (INSTR) prim[k] = svd_ray_result{e.res[0], e.res[1], e.res[2], e.res[3], tr.path, tr.bytes};
+  float col[3];
+  if (e.res[0] >= 0.f) {
+    const float hit[3] = {o[0] + e.res[0] * d[0], o[1] + e.res[0] * d[1], o[2] + e.res[0] * d[2]};
+    float hn[3] = {-(float)step[0], -(float)step[1], -(float)step[2]};
+    if (va.mode == 3) {
+      for (int i = 0; i < va.normSamples; ++i) {
+        float so[3], sd[3], t0, t1, sres[4];
+        int sstep[3];
+        sample_ray(s, p, va, e, px, py, i, so, sd, t0, t1);
+        tr.trace(so, sd, t0, t1, p.projection_factor, p.max_iters, p.draw_level, sres, sstep);
+        if (sres[0] >= 0.f && fabsf(sres[0] - e.res[0]) <= 64.0f * cell_size(s, e.res)) {
+          hn[0] = hn[0] + -(float)sstep[0];
+          hn[1] = hn[1] + -(float)sstep[1];
+          hn[2] = hn[2] + -(float)sstep[2];
+        }
+      }
+    }
+    shade_hit<FMT>(s, p, va, e.res, hit, hn, col);
+    if (p.shadows) {
+      const ShadowRay sh = shadow_from(p, hit, hn, cell_size(s, e.res));
+      float sres[4];
+      int sstep[3];
+      tr.trace(sh.o, sh.d, sh.tmin, sh.tmax, sh.projf, p.max_iters, p.draw_level, sres, sstep);
+      const float f = sres[0] > 0.f ? 0.8f : 1.0f;
+      col[0] = col[0] * f;
+      col[1] = col[1] * f;
+      col[2] = col[2] * f;
+    }
+  } else {
+    miss_colour(e.res, col);
+  }
+  rgb[3 * k + 0] = col[0];
+  rgb[3 * k + 1] = col[1];
+  rgb[3 * k + 2] = col[2];
+}
+
+// A workgroup per pixel tile in three phases (render_shares says when).
 template <int FMT, bool INSTR>
 __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_render(Dev s, svd_trace_params p, ViewArgs va,
                                                                 float* __restrict__ rgb,
@@ -1035,7 +1094,7 @@ __global__ void __launch_bounds__(kBT) SVD_TRACE_OCC k_render(Dev s, svd_trace_p
   for (int w = 0; w < kBT / 64; ++w) nHits += waveN[w];
   // 2. the normal samples, a quarter of the (hit, sample) rays per wavefront;
   // refills as in k_ao_rays
-  if (va.mode == 3 && va.normSamples > 0) {
+  {
     const uint32_t ns = (uint32_t)va.normSamples, total = nHits * ns;
     const uint32_t share = (total + kBT / 64 - 1) / (kBT / 64);
     uint32_t at = min(total, (uint32_t)wave * share);
@@ -1278,6 +1337,25 @@ size_t stack_bytes(const svd_scene* sc, const Dev& d) {
           (sc->fmt == SVD_FMT_SSVDAG || sc->fmt == SVD_FMT_ESVDAG ? kMaxLevels : 0)) * sizeof(uint32_t);
 }
 
+// Whether a frame's normal samples are shared out (k_render).  Where a voxel
+// covers many pixels, neighbours' samples are alike and a lane per pixel wastes
+// little, so the line lies at a number of samples per pixel of a voxel's
+// height: 1.5 for SSVDAG scenes and 6 for the others, whose fetches are cheaper
+// (12 in large frames).  Shared out / lane per pixel, us: SSVDAG with 4 samples
+// at 480x270 of 8 levels (3.8 samples per such pixel) 547 / 609, of 7 (1.9) 484 /
+// 471, 960x540 of 6 (0.5) 387 / 338, 1920x1080 of 11 (7.6) 1098 / 1184 and of 8
+// (0.9) 948 / 899; SVDAG with 7 samples at 480x270 of 8 (6.6) 505 / 567 and of 7
+// (3.3) 454 / 468, with 4 at 1920x1080 of 11 (7.6) 826 / 787 and of 6 (0.2) 491 /
+// 385.  With fewer than four samples a lane per pixel is as fast or faster
+// throughout (1 sample, 960x540 of 11 levels: 423 / 389; none: 400 / 378).
+bool render_shares(const svd_scene* sc, const svd_trace_params& p, const ViewArgs& va) {
+  if (va.mode != 3 || va.normSamples < 4) return false;
+  const bool sym = sc->fmt == SVD_FMT_SSVDAG || sc->fmt == SVD_FMT_ESVDAG;
+  const uint64_t detail = (uint64_t)va.normSamples << sc->levels, h = p.height;
+  const bool large = (uint64_t)p.width * p.height > (1u << 20);
+  return detail >= (sym ? h + h / 2 : large ? 12 * h : 6 * h);
+}
+
 // The DEPTH_MODE pre-pass into `depth` ((width/8) x (height/8) floats).  The
 // texture is (int)width / 8 x (int)height / 8; its screenRes uniform is the
 // float width / 8, height / 8.
@@ -1458,9 +1536,12 @@ void render_frame(svd_scene* sc, const svd_trace_params* p, const svd_view_param
     depth = depthBuf ? depthBuf : dalloc<float>(c, (uint64_t)(p->width / 8) * (p->height / 8) + 1);
     md = depth_prepass(sc, d, p, beamProjf, depth);
   }
+  const bool share = render_shares(sc, *p, va);
   auto render = [&](auto fmt) {
-    if (prim) k_render<fmt(), true><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md);
-    else k_render<fmt(), false><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, nullptr, md);
+    if (share && prim) k_render<fmt(), true><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md);
+    else if (share) k_render<fmt(), false><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, nullptr, md);
+    else if (prim) k_render_lane<fmt(), true><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, prim, md);
+    else k_render_lane<fmt(), false><<<grid, block, shmem, c->stream>>>(d, *p, va, rgb, nullptr, md);
   };
   switch (sc->fmt) {
     case SVD_FMT_SVDAG: render(std::integral_constant<int, SVD_FMT_SVDAG>()); break;

@@ -165,6 +165,31 @@ def test_shared_out_rays_match_oracle(ctx, scene_files, size, samples, nrays):
         np.testing.assert_array_equal(vis.cpu().numpy().reshape(p.height, p.width), want)
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("L,size,samples", [(5, (480, 270), 4), (8, (161, 113), 5), (8, (161, 113), 3)])
+def test_render_forms_match_oracle(ctx, fmt, L, size, samples):
+    """Both forms of the shading kernel, with and without the primary records:
+    a lane per pixel (large voxels, or few samples) and samples shared out."""
+    import torch
+    o = O.OracleOctree.from_morton(W.terrain_codes(L, seed=1), L)
+    o.to_dag()
+    o.init_child_levels()
+    if fmt in (S.FMT_USSVDAG, S.FMT_SSVDAG):
+        o.to_sdag()
+    buf = o.encode(O_FMT[fmt])
+    p = W.trace_params(size[0], size[1], seed=4, levels=L, shadows=True, light=(1.0, 0.6, 1.0))
+    v = S.ViewParams.defaults(render_mode=3, norm_samples=samples)
+    want, wprim = O.render_frame(buf, fmt, p, v)
+    got, gprim = gpu_render(ctx, fmt, buf, p, v, 0.0)
+    np.testing.assert_array_equal(gprim, wprim)
+    np.testing.assert_array_equal(got, want)
+    rgb = torch.full((p.width * p.height * 3,), float("nan"), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    S.Scene.from_bytes(ctx, fmt, buf).render_device(p, v, rgb.data_ptr())
+    ctx.sync()
+    np.testing.assert_array_equal(rgb.cpu().numpy().reshape(want.shape), want)
+
+
 def deep_file(fmt, L):
     """A sphere of points in a 2^L grid, in the given format."""
     rng = np.random.default_rng(L)
